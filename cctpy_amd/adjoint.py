@@ -122,8 +122,9 @@ class AdjointTracker:
         """In-place tracking of device state (6, P), keeping checkpoints every K steps (or, with
         K = 0, the tape of every step)."""
         if self.ckpt_every > 0:
-            self.model.track_tensors(self.plan, self.precision, state, self.kq, self.dt, self.ns, self.max_steps,
-                                     self.scratch, self.partial, record=self.ckpt, record_every=self.ckpt_every)
+            # every segment summed, as the reverse pass recomputes the steps
+            self.model._track(self.plan, self.precision, state, self.kq, self.dt, self.ns, self.max_steps,
+                              self.scratch, self.partial, self.ckpt, self.ckpt_every, far_field=False)
             return
         m, plan = self.model, self.plan
         seg, org, near = m._seg(self.precision)

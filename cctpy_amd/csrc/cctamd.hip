@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "far.hpp"
 
 namespace cctamd_detail {
 namespace {
@@ -255,7 +256,11 @@ constexpr double kFp64Tile = 1.5;
 // update at the end alone would otherwise set their register count (~120-160
 // VGPRs against 44 for k_bs_partial_f32k<1, 8>).  1 = no hint.
 constexpr int kKindF32 = 0, kKindF32k = 1, kKindF64 = 2;
-constexpr int fused_waves(int kind, int ppl, int s) {
+constexpr int fused_waves(int kind, int ppl, int s, bool far = false) {
+    // Far-field kernels: enough for two workgroups per CU (ppl 1, 2).  Their series hold 98 and
+    // 143 VGPRs by themselves; held to 96 and 128 they spill 1 and 13 outside its loop, and the
+    // 512-proton AG-CCT section's stage takes 58 instead of 67 us (FP32), one item per CU more.
+    if (far) return ppl == 1 ? 5 : ppl == 2 ? 4 : 2;
     if (s < 0) return 1;
     if (kind == kKindF32) return ppl == 1 ? 6 : 4;
     if (kind == kKindF32k) return ppl == 1 ? 8 : ppl == 2 ? 6 : 4;
@@ -567,13 +572,46 @@ __device__ inline void tile_direct_term(const float4& a, const float4& b, const 
     bz += (a.x * ry - a.y * rx) * w3;
 }
 
-template <int PPL, int NW, int S = -1>
-__global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fused_waves(kKindF32k, PPL, S)))) void k_bs_partial_f32k(const float* __restrict__ seg32k,
+// A work item's share of its block's lists (far.hpp), for the scalar-load kernels: near tiles and
+// series are dealt out to all waves of the block's items, numbered so that neighbours in a
+// list go to different items.  A series is cut into NW shares (pairs of its rows m) as long
+// as the block has few series per wave: their lengths differ by a factor of ten, and one wave
+// alone takes 45,000 cycles for order 31 at two points per lane.  With many series each wave
+// takes whole ones, which saves the powers of X + iY that every sharer computes.
+constexpr int kFarShared = 4;  // series per wave of the block below which they are shared
+
+template <bool F64, int PPL, int NW, typename Tile>
+__device__ __forceinline__ void far_scalar_walk(const FarSet& fs, const Work& w, int wave, int lane,
+                                                const double (&px)[PPL], const double (&py)[PPL],
+                                                const double (&pz)[PPL], double (&ax)[PPL], double (&ay)[PPL],
+                                                double (&az)[PPL], Tile&& tile) {
+    __shared__ FarLists<NW> L;
+    const Ball ball = block_ball<PPL>(px, py, pz);
+    const int me = wave * w.nchunk + w.chunk, all = w.nchunk * NW;
+    for (int base = 0; base * kParts < w.tile_count; base += FarLists<NW>::kRound) {
+        far_lists<F64, NW>(L, fs, w, ball, base, wave, lane);
+        const int ntile = __builtin_amdgcn_readfirstlane(L.nnear) * kSmallTiles;
+        for (int t = me; t < ntile; t += all)
+            tile(__builtin_amdgcn_readfirstlane(L.near[t / kSmallTiles]) * kSmallTiles + t % kSmallTiles);
+        // from the other end: the waves with one more near tile have one share less
+        const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
+        const int shares = nfar < kFarShared * all ? NW : 1;
+        for (int e = all - 1 - me; e < nfar * shares; e += all) {
+            const int s = e % shares;
+            far_entry<F64 ? kFarQ64 : kFarQ32, NW, PPL>(L, fs, e / shares, s, 2 * shares - 1 - s, 2 * shares, px, py, pz,
+                                                         ax, ay, az);
+        }
+        __syncthreads();  // before the next round's lists
+    }
+}
+
+template <int PPL, int NW, bool FAR = false, int S = -1>
+__global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fused_waves(kKindF32k, PPL, S, FAR)))) void k_bs_partial_f32k(const float* __restrict__ seg32k,
                                                           const double* __restrict__ tile_org,
                                                           const double* __restrict__ seg64,
                                                           const Work* __restrict__ work,
                                                           const double* __restrict__ pts, int64_t ptot,
-                                                          double* __restrict__ partial, StageArgs sa) {
+                                                          double* __restrict__ partial, StageArgs sa, FarSet fs) {
     constexpr int PB = kWave * PPL;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
@@ -584,8 +622,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
 #pragma unroll
     for (int j = 0; j < PPL; ++j) ax[j] = ay[j] = az[j] = 0.0;
 
-    const int tend = w.tile_start + w.tile_count;
-    for (int t = w.tile_start + wave; t < tend; t += NW) {
+    const auto tile = [&](int t) {
         const double ox = tile_org[4 * t], oy = tile_org[4 * t + 1], oz = tile_org[4 * t + 2];
         const double e2 = tile_org[4 * t + 3];
         float qx[PPL], qy[PPL], qz[PPL], qq[PPL], kx[PPL], ky[PPL], kz[PPL], cx[PPL], cy[PPL], cz[PPL];
@@ -605,7 +642,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
         const float4* s = reinterpret_cast<const float4*>(seg32k) + (int64_t)t * kTile * 3;
         if (__any(f64)) {  // wave-uniform: FP64 terms for the whole wave on this tile
             tile_terms_f64<PPL>(seg64, t, px, py, pz, ax, ay, az);
-            continue;
+            return;
         }
         if (__any(near)) {  // wave-uniform: FP32 direct form
 #pragma unroll 1
@@ -620,7 +657,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
                 ay[j] += (double)ky[j];
                 az[j] += (double)kz[j];
             }
-            continue;
+            return;
         }
 #pragma unroll CCTAMD_KC_UNROLL
         for (int k = 0; k < kTile; ++k) kc_terms<PPL>(kc_seg(s, k), qx, qy, qz, qq, kx, ky, kz, cx, cy, cz);
@@ -630,6 +667,15 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
             ay[j] += (double)((kz[j] * qx[j] - kx[j] * qz[j]) - cy[j]);
             az[j] += (double)((kx[j] * qy[j] - ky[j] * qx[j]) - cz[j]);
         }
+    };
+    if constexpr (FAR) {
+        far_scalar_walk<false, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az, [&](int place) {
+            const int t = __builtin_amdgcn_readfirstlane(fs.tiles[place]);
+            if (t >= 0) tile(t);
+        });
+    } else {
+        const int tend = w.tile_start + w.tile_count;
+        for (int t = w.tile_start + wave; t < tend; t += NW) tile(t);
     }
     write_partial<PPL, NW>(ax, ay, az, wave, lane, partial + partial_base(w, PB), w.nchunk);
     if constexpr (S >= 0) stage_after_last_chunk<S, NW>(w, sa);
@@ -707,12 +753,13 @@ __device__ __forceinline__ void direct_row_steps(const KCRow& g, const float (&q
 
 // 6 waves per SIMD (80 VGPRs): hints of 7 (72 VGPRs, 10 spilled) and 8 (64, 23
 // spilled) measured 8 % and 11 % slower on the 64-design population.
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(6))) void k_bs_partial_f32k_row(const float* __restrict__ seg32k,
+template <bool FAR>
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 6))) void k_bs_partial_f32k_row(const float* __restrict__ seg32k,
                                                              const double* __restrict__ tile_org,
                                                              const double* __restrict__ seg64,
                                                              const Work* __restrict__ work,
                                                              const double* __restrict__ pts, int64_t ptot,
-                                                             double* __restrict__ partial) {
+                                                             double* __restrict__ partial, FarSet fs) {
     constexpr int LG = 16;                  // lanes per row
     constexpr int PB = 2 * LG;              // 32 points per block
     constexpr int NS = kWavesPerWG * 4;     // tile streams (rows) per workgroup
@@ -738,7 +785,6 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(6))) void k
     }
 #pragma unroll
     for (int c = 0; c < 6; ++c) acc[c][tid] = 0.0;
-    const int tend = w.tile_start + w.tile_count;
     const float4* src = reinterpret_cast<const float4*>(seg32k);
     auto load = [&](int t, KCRow& g0, KCRow& g1) {  // segments gl and gl + 16 of tile t
         const float4* r0 = src + ((int64_t)t * kTile + gl) * 3;
@@ -746,9 +792,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(6))) void k
         g0 = KCRow{r0[0], r0[1], r0[2]};
         g1 = KCRow{r1[0], r1[1], r1[2]};
     };
-    int t = w.tile_start + stream;
-    while (t < tend) {  // uniform within a row
-        const int tn = t + NS;
+    const auto tile = [&](int t) {  // uniform within a row
         KCRow g0, g1;
         load(t, g0, g1);
         const double ox = tile_org[4 * t], oy = tile_org[4 * t + 1], oz = tile_org[4 * t + 2];
@@ -796,7 +840,34 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(6))) void k
                 acc[4 + j][tid] += (double)((kx[j] * qy[j] - ky[j] * qx[j]) - cz[j]);
             }
         }
-        t = tn;
+    };
+    if constexpr (FAR) {
+        __shared__ FarLists<kWavesPerWG> L;
+        const Ball ball = block_ball<2>(px, py, pz);
+        for (int base = 0; base * kParts < w.tile_count; base += FarLists<kWavesPerWG>::kRound) {
+            far_lists<false, kWavesPerWG>(L, fs, w, ball, base, wave, lane);
+            const int ntile = L.nnear * kSmallTiles;
+            for (int t = w.chunk * NS + stream; t < ntile; t += w.nchunk * NS) {  // uniform within a row
+                const int id = fs.tiles[L.near[t / kSmallTiles] * kSmallTiles + t % kSmallTiles];
+                if (id >= 0) tile(id);
+            }
+            // a series per wave, its rows m shared by the four rows of lanes
+            const int me = __builtin_amdgcn_readfirstlane(wave) * w.nchunk + w.chunk, all = w.nchunk * kWavesPerWG;
+            const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
+            double ax[2] = {0.0, 0.0}, ay[2] = {0.0, 0.0}, az[2] = {0.0, 0.0};
+            for (int e = all - 1 - me; e < nfar; e += all)
+                far_entry<kFarQ32, kWavesPerWG, 2>(L, fs, e, lane / LG, 7 - lane / LG, 8, px, py, pz, ax, ay, az);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[j][tid] += ax[j];
+                acc[2 + j][tid] += ay[j];
+                acc[4 + j][tid] += az[j];
+            }
+            __syncthreads();  // before the next round's lists
+        }
+    } else {
+        const int tend = w.tile_start + w.tile_count;
+        for (int t = w.tile_start + stream; t < tend; t += NS) tile(t);
     }
     double ax[2] = {acc[0][tid], acc[1][tid]}, ay[2] = {acc[2][tid], acc[3][tid]}, az[2] = {acc[4][tid], acc[5][tid]};
 #pragma unroll
@@ -963,12 +1034,25 @@ __global__ __launch_bounds__(kWG) void k_bs_partial_f32k_grp(const float* __rest
     }
 }
 
+// Two packed rows {kl, m} of the FP64 path's clusters.
+struct SegPair {
+    double v[12];
+};
+
+__device__ __forceinline__ SegPair seg_pair(ConstDoubles s) {
+    s = apart(s);
+    SegPair p;
+#pragma unroll
+    for (int i = 0; i < 12; ++i) p.v[i] = s[i];
+    return p;
+}
+
 // Plain FP64 terms on global-frame segments.
-template <int PPL, int NW, int S = -1>
-__global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fused_waves(kKindF64, PPL, S)))) void k_bs_partial_f64(const double* __restrict__ seg64,
+template <int PPL, int NW, bool FAR = false, int S = -1>
+__global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fused_waves(kKindF64, PPL, S, FAR)))) void k_bs_partial_f64(const double* __restrict__ seg64,
                                                          const Work* __restrict__ work,
                                                          const double* __restrict__ pts, int64_t ptot,
-                                                         double* __restrict__ partial, StageArgs sa) {
+                                                         double* __restrict__ partial, StageArgs sa, FarSet fs) {
     constexpr int PB = kWave * PPL;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
@@ -979,8 +1063,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
 #pragma unroll
     for (int j = 0; j < PPL; ++j) ax[j] = ay[j] = az[j] = 0.0;
 
-    const int tend = w.tile_start + w.tile_count;
-    for (int t = w.tile_start + wave; t < tend; t += NW) {
+    const auto tile = [&](int t) {
         const double2* s = reinterpret_cast<const double2*>(seg64) + (int64_t)t * kTile * 4;
 #pragma unroll CCTAMD_F64_UNROLL
         for (int k = 0; k < kTile; ++k) {
@@ -996,6 +1079,42 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
                 az[j] += (k01.x * ry - k01.y * rx) * inv3;
             }
         }
+    };
+    if constexpr (FAR) {
+        far_scalar_walk<true, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az, [&](int t) {
+            // packed rows {kl, m}, two pairs in turn (as the records of far_series)
+            ConstDoubles s = const_doubles(seg64 + (int64_t)t * kTile * 6);
+            const auto terms = [&](const SegPair& p) {
+#pragma unroll
+                for (int i = 0; i < 12; i += 6) {
+#pragma unroll
+                    for (int j = 0; j < PPL; ++j) {
+                        const double rx = px[j] - p.v[i + 3], ry = py[j] - p.v[i + 4], rz = pz[j] - p.v[i + 5];
+                        const double r2 = rx * rx + ry * ry + rz * rz;
+                        const double inv = rsqrt_f64(r2);
+                        const double inv3 = inv * inv * inv;
+                        ax[j] += (p.v[i + 1] * rz - p.v[i + 2] * ry) * inv3;
+                        ay[j] += (p.v[i + 2] * rx - p.v[i] * rz) * inv3;
+                        az[j] += (p.v[i] * ry - p.v[i + 1] * rx) * inv3;
+                    }
+                }
+            };
+            SegPair p = seg_pair(s), q;
+#pragma unroll 1
+            for (int k = 0; k < kTile; k += 4, s += 24) {
+                loads_done();
+                q = seg_pair(s + 12);
+                __builtin_amdgcn_sched_barrier(0);
+                terms(p);
+                loads_done();
+                p = seg_pair(s + 24);  // past the last tile: kFarPad rows follow the array
+                __builtin_amdgcn_sched_barrier(0);
+                terms(q);
+            }
+        });
+    } else {
+        const int tend = w.tile_start + w.tile_count;
+        for (int t = w.tile_start + wave; t < tend; t += NW) tile(t);
     }
     write_partial<PPL, NW>(ax, ay, az, wave, lane, partial + partial_base(w, PB), w.nchunk);
     if constexpr (S >= 0) stage_after_last_chunk<S, NW>(w, sa);
@@ -1010,11 +1129,11 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
 // LDS per workgroup small enough for several workgroups per CU (<4, 2, 2>:
 // 7 waves per SIMD, 2.5 % faster than whole tiles at 4; 8 groups of 4 points
 // per lane were slower).
-template <int G, int PL, int PARTS>
-__global__ __launch_bounds__(kWG) void k_bs_partial_f64_grp(const double* __restrict__ seg64,
+template <int G, int PL, int PARTS, bool FAR>
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1))) void k_bs_partial_f64_grp(const double* __restrict__ seg64,
                                                              const Work* __restrict__ work,
                                                              const double* __restrict__ pts, int64_t ptot,
-                                                             double* __restrict__ partial) {
+                                                             double* __restrict__ partial, FarSet fs) {
     constexpr int LG = kWave / G;         // lanes per group
     constexpr int PB = LG * PL;           // points per block
     constexpr int NS = kWavesPerWG * G;   // tile streams per workgroup
@@ -1039,26 +1158,34 @@ __global__ __launch_bounds__(kWG) void k_bs_partial_f64_grp(const double* __rest
         pz[j] = pts[2 * ptot + gp];
         ax[j] = ay[j] = az[j] = 0.0;
     }
-    const int tend = w.tile_start + w.tile_count;
     const float4* src = reinterpret_cast<const float4*>(seg64);
     static_assert(NS * SEGS == kWG, "one segment per thread and staging round");
     const int st = (int)threadIdx.x / SEGS, sk = (int)threadIdx.x % SEGS;
-    for (int t0 = w.tile_start; t0 < tend; t0 += NS) {
+    // one round: every stream sums its own tile; tload: the tile this thread stages, tsum: the one
+    // of its stream (-1: none)
+    const auto tiles = [&](int tload, int tsum) {
 #pragma unroll 1
         for (int h = 0; h < PARTS; ++h) {
             float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0, v2 = v0, v3 = v0;  // absent tiles: not read
-            if (t0 + st < tend) {
-                const float4* g = src + (int64_t)(t0 + st) * ROW + (h * SEGS + sk) * 4;
-                v0 = g[0];  // kl.x, kl.y
-                v1 = g[1];  // kl.z, pad
-                v2 = g[2];  // m.x, m.y
-                v3 = g[3];  // m.z, pad
+            if (tload >= 0) {
+                if constexpr (FAR) {  // packed rows
+                    const float4* g = src + ((int64_t)tload * kTile + h * SEGS + sk) * 3;
+                    v0 = g[0];
+                    v1 = g[1];
+                    v2 = g[2];
+                } else {
+                    const float4* g = src + (int64_t)tload * ROW + (h * SEGS + sk) * 4;
+                    v0 = g[0];  // kl.x, kl.y
+                    v1 = g[1];  // kl.z, pad
+                    v2 = g[2];  // m.x, m.y
+                    v3 = g[3];  // m.z, pad
+                }
             }
             lds[st][3 * sk] = v0;
-            lds[st][3 * sk + 1] = make_float4(v1.x, v1.y, v2.x, v2.y);
-            lds[st][3 * sk + 2] = make_float4(v2.z, v2.w, v3.x, v3.y);
+            lds[st][3 * sk + 1] = FAR ? v1 : make_float4(v1.x, v1.y, v2.x, v2.y);
+            lds[st][3 * sk + 2] = FAR ? v2 : make_float4(v2.z, v2.w, v3.x, v3.y);
             __syncthreads();
-            if (t0 + stream < tend) {  // uniform within a lane group
+            if (tsum >= 0) {  // uniform within a lane group
                 const double2* r = reinterpret_cast<const double2*>(lds[stream]);
 #pragma unroll CCTAMD_F64G_UNROLL
                 for (int k = 0; k < SEGS; ++k) {
@@ -1077,6 +1204,43 @@ __global__ __launch_bounds__(kWG) void k_bs_partial_f64_grp(const double* __rest
             }
             __syncthreads();
         }
+    };
+    if constexpr (FAR) {
+        __shared__ FarLists<kWavesPerWG> L;
+        const Ball ball = block_ball<PL>(px, py, pz);
+        for (int base = 0; base * kParts < w.tile_count; base += FarLists<kWavesPerWG>::kRound) {
+            far_lists<true, kWavesPerWG>(L, fs, w, ball, base, wave, lane);
+            const int ntile = __builtin_amdgcn_readfirstlane(L.nnear) * kSmallTiles;
+            const auto near = [&](int t) {
+                return t < ntile ? L.near[t / kSmallTiles] * kSmallTiles + t % kSmallTiles : -1;
+            };
+            for (int t = w.chunk * NS; t < ntile; t += w.nchunk * NS) tiles(near(t + st), near(t + stream));
+            // the 16-lane rows of the workgroup share a series (groups of 8 lanes: the first of a row
+            // takes its sum), or those of a wave where there are many; a share per wave as in
+            // far_scalar_walk measured up to 8 % slower here
+            const int me = w.chunk * kWavesPerWG + __builtin_amdgcn_readfirstlane(wave), all = w.nchunk * kWavesPerWG;
+            const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
+            const bool shared = nfar < kFarShared * all;
+            const int from = shared ? w.nchunk - 1 - w.chunk : all - 1 - me, by = shared ? w.nchunk : all;
+            const int row = shared ? (int)threadIdx.x / 16 : lane / 16, rows = shared ? kWG / 16 : kWave / 16;
+            double fx[PL], fy[PL], fz[PL];
+#pragma unroll
+            for (int j = 0; j < PL; ++j) fx[j] = fy[j] = fz[j] = 0.0;
+            for (int e = from; e < nfar; e += by)
+                far_entry<kFarQ64, kWavesPerWG, PL>(L, fs, e, row, 2 * rows - 1 - row, 2 * rows, px, py, pz, fx, fy, fz);
+            const bool mine = LG >= 16 || (lane & 8) == 0;
+#pragma unroll
+            for (int j = 0; j < PL; ++j) {
+                ax[j] += mine ? fx[j] : 0.0;
+                ay[j] += mine ? fy[j] : 0.0;
+                az[j] += mine ? fz[j] : 0.0;
+            }
+            __syncthreads();  // before the next round's lists
+        }
+    } else {
+        const int tend = w.tile_start + w.tile_count;
+        for (int t0 = w.tile_start; t0 < tend; t0 += NS)
+            tiles(t0 + st < tend ? t0 + st : -1, t0 + stream < tend ? t0 + stream : -1);
     }
 #pragma unroll
     for (int j = 0; j < PL; ++j) {
@@ -1151,20 +1315,23 @@ __global__ __launch_bounds__(kWG) void k_rk4_stage(StageArgs sa) {
     rk4_stage_point<S>(sa, g);
 }
 
-template <int PPL, int S = -1>
+template <int PPL, bool FAR = false, int S = -1>
 hipError_t launch_bs(int precision, const void* seg, const double* tile_org, const double* seg_near, const Work* work,
                      int64_t nwork, const double* pts, int64_t ptot, double* partial, hipStream_t st,
-                     const StageArgs& sa = StageArgs{}) {
+                     const FarSet& fs = FarSet{}, const StageArgs& sa = StageArgs{}) {
     if (nwork == 0) return hipSuccess;
-    if (precision == 32)
-        hipLaunchKernelGGL((k_bs_partial_f32<PPL, S>), dim3((unsigned)nwork), dim3(kWG), 0, st,
-                           (const float*)seg, tile_org, seg_near, work, pts, ptot, partial, sa);
-    else if (precision == 33)
-        hipLaunchKernelGGL((k_bs_partial_f32k<PPL, kBsWaves, S>), dim3((unsigned)nwork), dim3(kWave * kBsWaves), 0,
-                           st, (const float*)seg, tile_org, seg_near, work, pts, ptot, partial, sa);
+    if (precision == 32) {
+        if constexpr (FAR)
+            return hipErrorInvalidValue;  // the direct FP32 form has no far-field kernel
+        else
+            hipLaunchKernelGGL((k_bs_partial_f32<PPL, S>), dim3((unsigned)nwork), dim3(kWG), 0, st,
+                               (const float*)seg, tile_org, seg_near, work, pts, ptot, partial, sa);
+    } else if (precision == 33)
+        hipLaunchKernelGGL((k_bs_partial_f32k<PPL, kBsWaves, FAR, S>), dim3((unsigned)nwork), dim3(kWave * kBsWaves), 0,
+                           st, (const float*)seg, tile_org, seg_near, work, pts, ptot, partial, sa, fs);
     else
-        hipLaunchKernelGGL((k_bs_partial_f64<PPL, kBsWaves, S>), dim3((unsigned)nwork), dim3(kWave * kBsWaves), 0,
-                           st, (const double*)seg, work, pts, ptot, partial, sa);
+        hipLaunchKernelGGL((k_bs_partial_f64<PPL, kBsWaves, FAR, S>), dim3((unsigned)nwork), dim3(kWave * kBsWaves), 0,
+                           st, (const double*)seg, work, pts, ptot, partial, sa, fs);
     return hipGetLastError();
 }
 
@@ -1175,14 +1342,14 @@ hipError_t launch_bs_stage(const DeviceSet& ds, int64_t ptot, double* partial, c
     const double* pts = sa.scratch;  // rows 0-2: the stage points
     switch (ds.ppl) {
         case 1:
-            return launch_bs<1, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts, ptot,
-                                   partial, st, sa);
+            return launch_bs<1, false, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
+                                          ptot, partial, st, FarSet{}, sa);
         case 2:
-            return launch_bs<2, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts, ptot,
-                                   partial, st, sa);
+            return launch_bs<2, false, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
+                                          ptot, partial, st, FarSet{}, sa);
         default:
-            return launch_bs<4, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts, ptot,
-                                   partial, st, sa);
+            return launch_bs<4, false, S>(ds.precision, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
+                                          ptot, partial, st, FarSet{}, sa);
     }
 }
 
@@ -1199,34 +1366,45 @@ bool valid_common(int precision, int ppl, const void* seg, const double* tile_or
     return true;
 }
 
-hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
-                         const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
-                         hipStream_t st) {
+// The kernels of a points-per-lane code, with or without the far field.
+template <bool FAR>
+hipError_t launch_bs_shape(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
+                           const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
+                           hipStream_t st, const FarSet& fs) {
+    if (nwork == 0) return hipSuccess;
     if (ppl < 0) {
-        if (nwork == 0) return hipSuccess;
         if (precision == 64) {
             if (ppl == -2)
-                hipLaunchKernelGGL((k_bs_partial_f64_grp<4, 2, 2>), dim3((unsigned)nwork), dim3(kWG), 0, st,
-                                   (const double*)seg, work, pts, ptot, partial);
+                hipLaunchKernelGGL((k_bs_partial_f64_grp<4, 2, 2, FAR>), dim3((unsigned)nwork), dim3(kWG), 0, st,
+                                   (const double*)seg, work, pts, ptot, partial, fs);
             else
-                hipLaunchKernelGGL((k_bs_partial_f64_grp<8, 2, 4>), dim3((unsigned)nwork), dim3(kWG), 0, st,
-                                   (const double*)seg, work, pts, ptot, partial);
+                hipLaunchKernelGGL((k_bs_partial_f64_grp<8, 2, 4, FAR>), dim3((unsigned)nwork), dim3(kWG), 0, st,
+                                   (const double*)seg, work, pts, ptot, partial, fs);
             return hipGetLastError();
         }
         if (precision != 33) return hipErrorInvalidValue;
         if (ppl == -2)
-            hipLaunchKernelGGL(k_bs_partial_f32k_row, dim3((unsigned)nwork), dim3(kWG), 0, st,
-                               (const float*)seg, tile_org, seg_near, work, pts, ptot, partial);
+            hipLaunchKernelGGL(k_bs_partial_f32k_row<FAR>, dim3((unsigned)nwork), dim3(kWG), 0, st,
+                               (const float*)seg, tile_org, seg_near, work, pts, ptot, partial, fs);
+        else if (FAR)
+            return hipErrorInvalidValue;  // 16-point blocks of the FP32 path have no far-field kernel
         else
             hipLaunchKernelGGL((k_bs_partial_f32k_grp<8, 2>), dim3((unsigned)nwork), dim3(kWG), 0, st,
                                (const float*)seg, tile_org, seg_near, work, pts, ptot, partial);
         return hipGetLastError();
     }
     switch (ppl) {
-        case 1: return launch_bs<1>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st);
-        case 2: return launch_bs<2>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st);
-        default: return launch_bs<4>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st);
+        case 1: return launch_bs<1, FAR>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st, fs);
+        case 2: return launch_bs<2, FAR>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st, fs);
+        default: return launch_bs<4, FAR>(precision, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st, fs);
     }
+}
+
+hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
+                         const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
+                         hipStream_t st) {
+    return launch_bs_shape<false>(precision, ppl, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st,
+                                  FarSet{});
 }
 
 int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, double* partial, double* B,
@@ -1260,7 +1438,7 @@ int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, do
 // single CCT whatever the item count (6x slower there; 2.9x on the
 // 368,640-segment AG-CCT section), against ~5 us for the stage kernel.
 bool fused_stages(const DeviceSet& ds) {
-    if (ds.ppl <= 0 || ds.nwork == 0) return false;
+    if (ds.ppl <= 0 || ds.nwork == 0 || ds.far.geo) return false;
     const char* env = getenv("CCTAMD_FUSED_STAGES");
     return env && env[0] == '1';
 }
@@ -1285,8 +1463,10 @@ hipError_t launch_rk4_steps(const DeviceSet& ds, double* state, int64_t ptot, co
     if (fused) {                                                                                                  \
         e = launch_bs_stage<S>(ds, ptot, partial, sa, st);                                                        \
     } else {                                                                                                      \
-        e = launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, scratch,    \
-                          ptot, partial, st);                                                                     \
+        e = ds.far.geo ? launch_bs_shape<true>(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work,   \
+                                               ds.nwork, scratch, ptot, partial, st, ds.far)                      \
+                       : launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, \
+                                       scratch, ptot, partial, st);                                               \
         if (e != hipSuccess) return e;                                                                            \
         hipLaunchKernelGGL(k_rk4_stage<S>, dim3((unsigned)rblocks), dim3(kWG), 0, st, sa);                        \
         e = hipGetLastError();                                                                                    \
@@ -1438,24 +1618,50 @@ int cctamd_bs_field(int precision, int ppl, const void* seg, const double* tile_
     return field_checked(ds, points, npoints, partial, B, (hipStream_t)stream);
 }
 
+namespace {
+int track_checked(const DeviceSet& ds, double* state, int64_t nparticles, const double* kq, const double* dt,
+                  const int64_t* nsteps, int64_t max_steps, double* scratch, double* partial, double* record,
+                  int64_t record_every, void* stream) {
+    if (!valid_common(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.nwork, ds.ndesign))
+        return CCTAMD_EINVAL;
+    if (nparticles < 0 || max_steps < 0 || record_every <= 0) return CCTAMD_EINVAL;
+    if (nparticles == 0) return CCTAMD_OK;
+    if (!state || !kq || !dt || !nsteps || !scratch || !ds.design_wbase || !ds.design_nchunk || !ds.design_pt_off ||
+        !ds.design_qs_off || !ds.bconst)
+        return CCTAMD_EINVAL;
+    if (ds.nwork > 0 && (!ds.work || !partial)) return CCTAMD_EINVAL;
+    if (ceil_div(nparticles, kWavesPerWG) > 0x7fffffff) return CCTAMD_ERANGE;
+    return hip_status(launch_rk4_steps(ds, state, nparticles, kq, dt, nsteps, 0, max_steps, scratch, partial, record,
+                                       record_every, nullptr, (hipStream_t)stream));
+}
+}  // namespace
+
 int cctamd_track_rk4(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                      const int32_t* work, int64_t nwork, const int64_t* design_wbase, const int32_t* design_nchunk,
                      const int64_t* design_pt_off, int64_t ndesign, const double* qs, const int64_t* design_qs_off,
                      const double* bconst, double* state, int64_t nparticles, const double* kq, const double* dt,
                      const int64_t* nsteps, int64_t max_steps, double* scratch, double* partial, double* record,
                      int64_t record_every, void* stream) {
-    if (!valid_common(precision, ppl, seg, tile_org, seg_near, nwork, ndesign)) return CCTAMD_EINVAL;
-    if (nparticles < 0 || max_steps < 0 || record_every <= 0) return CCTAMD_EINVAL;
-    if (nparticles == 0) return CCTAMD_OK;
-    if (!state || !kq || !dt || !nsteps || !scratch || !design_wbase || !design_nchunk || !design_pt_off ||
-        !design_qs_off || !bconst)
-        return CCTAMD_EINVAL;
-    if (nwork > 0 && (!work || !partial)) return CCTAMD_EINVAL;
-    if (ceil_div(nparticles, kWavesPerWG) > 0x7fffffff) return CCTAMD_ERANGE;
     const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
                        design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst};
-    return hip_status(launch_rk4_steps(ds, state, nparticles, kq, dt, nsteps, 0, max_steps, scratch, partial, record,
-                                       record_every, nullptr, (hipStream_t)stream));
+    return track_checked(ds, state, nparticles, kq, dt, nsteps, max_steps, scratch, partial, record, record_every,
+                         stream);
+}
+
+int cctamd_track_rk4_far(const double* geo, const double* geo_large, const double* coef, const double* coef_large,
+                         const int32_t* tiles, int precision, int ppl, const void* seg, const double* tile_org,
+                         const double* seg_near, const int32_t* work, int64_t nwork, const int64_t* design_wbase,
+                         const int32_t* design_nchunk, const int64_t* design_pt_off, int64_t ndesign, const double* qs,
+                         const int64_t* design_qs_off, const double* bconst, double* state, int64_t nparticles,
+                         const double* kq, const double* dt, const int64_t* nsteps, int64_t max_steps, double* scratch,
+                         double* partial, double* record, int64_t record_every, void* stream) {
+    if (!geo || !geo_large || !coef || !coef_large) return CCTAMD_EINVAL;
+    if (precision == 33 ? (!tiles || ppl == -4) : precision != 64) return CCTAMD_EINVAL;
+    const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
+                       design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst,
+                       FarSet{geo, geo_large, coef, coef_large, tiles}};
+    return track_checked(ds, state, nparticles, kq, dt, nsteps, max_steps, scratch, partial, record, record_every,
+                         stream);
 }
 
 }  // extern "C"

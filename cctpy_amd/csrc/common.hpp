@@ -312,6 +312,14 @@ __device__ inline void analytic_fields(int64_t d, const double* __restrict__ qs,
     analytic_fields(analytic_set(d, design_qs_off, bconst), qs, p, b);
 }
 
+// What a kernel reads of a set of segment clusters (far.hpp).
+struct FarSet {
+    const double *geo, *geo_large;    // [C][kFarGeo] small clusters, [C / 4][kFarGeo] large ones
+    const double *coef, *coef_large;  // [C][far_records(Q)][kFarRec], [C / 4][far_records(Q)][kFarRec]
+    const int32_t* tiles;             // [C][kSmall * kNodeTiles] tile of each place, -1 for none (FP32 path); NULL:
+                                      // places are tiles of the packed rows passed beside this set (FP64 path)
+};
+
 // ---------------------------------------------------- shared host helpers
 struct DeviceSet {  // one segment set + analytic magnets of D designs
     int precision, ppl;
@@ -327,6 +335,7 @@ struct DeviceSet {  // one segment set + analytic magnets of D designs
     const double* qs;
     const int64_t* design_qs_off;
     const double* bconst;
+    FarSet far = {nullptr, nullptr, nullptr, nullptr, nullptr};  // geo NULL: every segment summed one by one
 };
 
 bool valid_common(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,

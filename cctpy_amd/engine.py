@@ -21,6 +21,7 @@ import collections
 import ctypes
 import hashlib
 import math
+import threading
 from dataclasses import dataclass, field as dc_field
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -31,6 +32,16 @@ from . import _native as N
 
 _TARGET_WG_PER_CU = 4
 _MIN_TILES_PER_ITEM = 4
+_LARGE_TILES = 64   # tiles of a large segment cluster (kParts * kSmallTiles in csrc/far.hpp)
+_FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
+# Where tracking takes the far field (per launch: lanes x segments, large clusters per design).  Measured
+# per RK4 stage, all segments summed against the far field: FP64, 64 protons in one CCT of 360 tiles
+# (2.9e6, 12 clusters) 13 / 20 us, 300 in one of 1,440 (1.8e7, 23) 34 / 22-28, 24 in two gantries at 120 segments
+# per winding (1.0e7, 79) 21 / 15, 64 protons in the AG-CCT section at 360 (1.2e7, 90) 24 / 16-21, 512 at
+# 720 (1.9e8, 180) 158 / 45-60.
+_FAR_MIN_PAIRS = {64: 1.0e7}
+_FAR_MIN_LARGE = {64: 60}
+_FAR_ANY_PAIRS = {64: 4.0e7}  # from here on whatever the number of clusters
 
 
 def device() -> torch.device:
@@ -97,6 +108,15 @@ class DesignSpec:
 
 
 @dataclass
+class FarPlan:
+    """Work items of the far-field kernels for a plan's point blocks."""
+    nwork: int
+    work: torch.Tensor
+    wbase: torch.Tensor
+    nchunk: torch.Tensor
+
+
+@dataclass
 class Plan:
     ppl: int
     nwork: int
@@ -105,6 +125,46 @@ class Plan:
     nchunk: torch.Tensor
     design_pt_off: torch.Tensor
     npt: int
+    design_npt: tuple = ()
+    far: Dict[int, FarPlan] = dc_field(default_factory=dict)  # by precision
+
+
+class FarField:
+    """Segment clusters of a model and their multipole coefficients (csrc/far.hip)."""
+
+    def __init__(self, model: "DeviceModel", precision: int):
+        dev = model.seg64.device
+        large = -(-model.design_ntile // _LARGE_TILES)
+        self.cluster_off = numpy.concatenate([[0], numpy.cumsum(4 * large)]).astype(numpy.int64)
+        C = int(self.cluster_off[-1])
+        unit = N.TILE
+        if precision == 64:  # fine units where the design is small or coarse, so that its splits are too
+            unit = 1
+            while unit < 8 and int(model.design_ntile.max()) * N.TILE > unit * 2 * _FAR_CHUNK:
+                unit *= 2
+        unit_off = model.design_tile_off * (N.TILE // unit)
+        chunk_off = numpy.concatenate([[0], numpy.cumsum(-(-numpy.diff(unit_off) // _FAR_CHUNK))]).astype(numpy.int64)
+        U = int(unit_off[-1])
+        uo, co, so = (torch.from_numpy(a).to(dev) for a in (unit_off, self.cluster_off, chunk_off))
+        key = torch.empty(U, dtype=torch.int64, device=dev)
+        centre = torch.empty((U, 4), dtype=torch.float32, device=dev)
+        N.check(N.lib.cctamd_far_keys(_p(model.seg64), unit, _p(uo), model.ndesign, U, _p(key), _p(centre),
+                                      _stream()), "cctamd_far_keys")
+        perm = torch.sort(key, stable=True).indices
+        per = int(N.lib.cctamd_far_coef_doubles(precision))
+
+        def empty(n, dtype=torch.float64):
+            return torch.empty(n, dtype=dtype, device=dev)
+
+        self.rows = empty(6 * (C * 512 + 4)) if precision == 64 else None
+        self.tiles = empty(C * 16, torch.int32) if precision != 64 else None
+        self.geo, self.geo_large = empty(8 * C), empty(2 * C)
+        self.coef, self.coef_large = empty(C * per + 128), empty(C // 4 * per + 128)
+        mom = empty(C * per // 4 * 3)
+        N.check(N.lib.cctamd_far_build(precision, _p(model.seg64), unit, _p(centre), _p(uo), _p(so), int(chunk_off[-1]),
+                                       _p(co), model.ndesign, C, _p(perm), _p(self.rows), _p(self.tiles),
+                                       _p(self.geo), _p(self.geo_large), _p(mom), _p(self.coef),
+                                       _p(self.coef_large), _stream()), "cctamd_far_build")
 
 
 class DeviceModel:
@@ -187,6 +247,8 @@ class DeviceModel:
             b[d, :3] = s.bconst
         self.bconst = torch.from_numpy(b).to(dev)
         self._plans: Dict[tuple, Plan] = {}
+        self._far: Dict[int, FarField] = {}
+        self._far_lock = threading.Lock()
 
     # --------------------------------------------------------- adjoint data
     def adjoint_data(self):
@@ -239,9 +301,94 @@ class DeviceModel:
         dev = device()
         p = Plan(ppl=ppl, nwork=int(n), work=torch.from_numpy(work).to(dev), wbase=torch.from_numpy(wbase).to(dev),
                  nchunk=torch.from_numpy(nchunk).to(dev), design_pt_off=torch.from_numpy(pt_off).to(dev),
-                 npt=int(pt_off[-1]))
+                 npt=int(pt_off[-1]), design_npt=tuple(npt.tolist()))
         self._plans[key] = p
         return p
+
+    # --------------------------------------------------------- far field
+    def far_field(self, plan: Plan, precision: int, max_steps: int) -> Optional[FarField]:
+        """The segment clusters that tracking ``plan`` for ``max_steps`` steps uses, built on first
+        need, with their work items in ``plan.far``; None where every segment is summed."""
+        if not self._far_pays(plan, precision, max_steps):
+            return None
+        with self._far_lock:
+            far = self._far.get(precision)
+            if far is not None and precision in plan.far:
+                return far
+            if torch.cuda.is_current_stream_capturing():
+                return None  # a capture cannot build them
+            try:
+                if far is None:
+                    far = FarField(self, precision)
+            except torch.OutOfMemoryError:
+                return None  # the clusters need as much again as the segments
+            plan.far[precision] = self._far_plan(far, plan, precision)
+            torch.cuda.current_stream().synchronize()  # ready for every stream that tracks this model
+            self._far[precision] = far
+            return far
+
+    def _far_pays(self, plan: Plan, precision: int, max_steps: int) -> bool:
+        """Whether tracking ``plan`` for ``max_steps`` steps is faster with the far field, its set-up
+        (once per model) included: a function of the sizes alone, so that equal calls give equal bits."""
+        if precision not in _FAR_MIN_PAIRS or plan.npt == 0 or self.nseg_padded == 0 or self.ndesign > 0x7fff:
+            return False
+        pb = points_per_block(plan.ppl)
+        blocks = -(-numpy.asarray(plan.design_npt, numpy.int64) // pb)
+        pairs = float((blocks * pb * self.design_ntile).sum()) * N.TILE
+        large = float((blocks * self.design_ntile).sum()) / max(float(blocks.sum()), 1.0) / _LARGE_TILES
+        if pairs < _FAR_MIN_PAIRS[precision] or (large < _FAR_MIN_LARGE[precision]
+                                                 and pairs < _FAR_ANY_PAIRS[precision]):
+            return False
+        # the set-up takes 1.5 ms + 2 ns per segment; a stage saves a third of its pair terms' time at
+        # the least (1.2e12 terms per second summed one by one)
+        return 4 * max_steps * pairs / 3 / 1.2e12 > 1.5e-3 + 2.0e-9 * self.nseg_padded
+
+    def _far_plan(self, far: FarField, plan: Plan, precision: int) -> FarPlan:
+        nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
+        npt = numpy.asarray(plan.design_npt, numpy.int64)
+        pt_off = numpy.concatenate([[0], numpy.cumsum(npt)]).astype(numpy.int64)
+        # Work items: one per CU for a small beam in one design (its lists cost each item 5 us), more where
+        # there is more to deal out, up to two resident per CU; several designs differ in what their
+        # blocks need and balance over smaller items.  512 protons in the AG-CCT section: 256 items 60 us,
+        # 1,024 69 us; 24 designs x 32: 256 items 153 us, 1,440 84 us.
+        clusters = int((-(-npt // points_per_block(plan.ppl)) * -(-nt // 16)).sum())
+        cus = cu_count()
+        target = min(max(clusters // 5, cus), 6 * cus) if self.ndesign > 1 else min(max(clusters // 11, cus), 2 * cus)
+        target = min(plan.nwork, target)
+        while True:  # the caller's partial sums hold plan.nwork items (every point block has one)
+            args = (self.ndesign, _np(nt), _np(npt), _np(far.cluster_off), _np(pt_off), plan.ppl)
+            n = int(N.lib.cctamd_far_plan(*args, target, None, None, None))
+            if n < 0:
+                N.check(n, "cctamd_far_plan")
+            if n <= plan.nwork or target == 1:
+                break
+            target = max(1, target - (n - plan.nwork))
+        work = numpy.zeros((max(n, 1), N.WORK_INTS), numpy.int32)
+        wbase = numpy.zeros(self.ndesign, numpy.int64)
+        nchunk = numpy.zeros(self.ndesign, numpy.int32)
+        n2 = N.lib.cctamd_far_plan(*args, target, _np(work), _np(wbase), _np(nchunk))
+        if n2 != n or n > plan.nwork:
+            raise N.CctamdError(f"cctamd_far_plan: {n2} work items, {n} expected, {plan.nwork} at most")
+        dev = self.seg64.device
+        return FarPlan(n, torch.from_numpy(work).to(dev), torch.from_numpy(wbase).to(dev),
+                       torch.from_numpy(nchunk).to(dev))
+
+    def _track(self, plan: Plan, precision: int, state, kq, dt, nsteps, max_steps: int, scratch, partial, record,
+               record_every: int, far_field: bool = True) -> None:
+        seg, org, near = self._seg(precision)
+        far = self.far_field(plan, precision, max_steps) if far_field else None
+        w = plan if far is None else plan.far[precision]
+        args = (_p(org), _p(near), _p(w.work), w.nwork, _p(w.wbase), _p(w.nchunk), _p(plan.design_pt_off),
+                self.ndesign, _p(self.qs), _p(self.design_qs_off), _p(self.bconst), _p(state), plan.npt, _p(kq),
+                _p(dt), _p(nsteps), int(max_steps), _p(scratch), _p(partial), _p(record), int(record_every),
+                _stream())
+        if far is None:
+            N.check(N.lib.cctamd_track_rk4(precision, plan.ppl, _p(seg), *args), "cctamd_track_rk4")
+        else:
+            rows = seg if far.rows is None else far.rows
+            N.check(N.lib.cctamd_track_rk4_far(_p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large),
+                                               _p(far.tiles), precision, plan.ppl, _p(rows), *args),
+                    "cctamd_track_rk4_far")
 
     def _seg(self, precision: int):
         """(segment rows, tile origins, FP64 rows for near tiles) of a precision."""
@@ -306,12 +453,7 @@ class DeviceModel:
         scratch = torch.empty((15, plan.npt), dtype=torch.float64, device=dev)
         partial = torch.empty(max(plan.nwork * 3 * points_per_block(ppl), 1), dtype=torch.float64, device=dev)
         rec = torch.empty((max_steps + 1, 6, plan.npt), dtype=torch.float64, device=dev) if record else None
-        seg, org, near = self._seg(precision)
-        N.check(N.lib.cctamd_track_rk4(precision, ppl, _p(seg), _p(org), _p(near), _p(plan.work), plan.nwork, _p(plan.wbase),
-                                       _p(plan.nchunk), _p(plan.design_pt_off), self.ndesign, _p(self.qs),
-                                       _p(self.design_qs_off), _p(self.bconst), _p(soa), plan.npt, _p(kq_t),
-                                       _p(dt_t), _p(ns_t), max_steps, _p(scratch), _p(partial), _p(rec), 1,
-                                       _stream()), "cctamd_track_rk4")
+        self._track(plan, precision, soa, kq_t, dt_t, ns_t, max_steps, scratch, partial, rec, 1)
         out = soa.cpu().numpy().T.copy()
         return out, (rec.cpu().numpy().transpose(0, 2, 1).copy() if rec is not None else None)
 
@@ -326,12 +468,7 @@ class DeviceModel:
                       nsteps: torch.Tensor, max_steps: int, scratch: torch.Tensor, partial: torch.Tensor,
                       record: Optional[torch.Tensor] = None, record_every: int = 1) -> None:
         """In-place RK4 tracking of device-resident SoA state (6, P); nothing crosses PCIe."""
-        seg, org, near = self._seg(precision)
-        N.check(N.lib.cctamd_track_rk4(precision, plan.ppl, _p(seg), _p(org), _p(near), _p(plan.work), plan.nwork,
-                                       _p(plan.wbase), _p(plan.nchunk), _p(plan.design_pt_off), self.ndesign,
-                                       _p(self.qs), _p(self.design_qs_off), _p(self.bconst), _p(state), plan.npt,
-                                       _p(kq), _p(dt), _p(nsteps), int(max_steps), _p(scratch), _p(partial),
-                                       _p(record), int(record_every), _stream()), "cctamd_track_rk4")
+        self._track(plan, precision, state, kq, dt, nsteps, max_steps, scratch, partial, record, record_every)
 
     def field_tensors(self, plan: "Plan", precision: int, points: torch.Tensor, partial: torch.Tensor,
                       out: torch.Tensor) -> None:
@@ -366,6 +503,7 @@ class TrackGraph:
                  dt: torch.Tensor, nsteps: torch.Tensor, max_steps: int, scratch: torch.Tensor,
                  partial: torch.Tensor):
         self.buffers = (state, kq, dt, nsteps, scratch, partial)  # kept alive with the graph
+        model.far_field(plan, precision, max_steps)  # built before the capture, which cannot
         self.graph = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream()  # default priority
         side.wait_stream(torch.cuda.current_stream())

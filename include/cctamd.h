@@ -180,6 +180,52 @@ int cctamd_track_rk4(int precision, int ppl, const void *seg, const double *tile
                      double *record, int64_t record_every, void *stream);
 
 /*
+ * Far field of segment clusters, for tracking many particles or steps through one segment
+ * set (no counterpart in the reference, which sums every segment).  The segments of each
+ * design are ordered in space and cut into small clusters of 16 tiles of 32 rows and large
+ * ones of four small ones; a cluster that lies several of its radii away from a whole point
+ * block acts through a multipole series cut below the rounding of the sum it replaces, the
+ * others are summed segment by segment.  Precisions 33 and 64.  Set-up, once per segment set:
+ *   cctamd_far_coef_doubles   doubles of a cluster's coefficients (3/4 of them for `mom`)
+ *   cctamd_far_keys           int64 sort key of every unit of `unit` consecutive rows of seg64
+ *                             (design, place along a Hilbert curve) and its centre
+ *                             (float[U][4]); unit 32 (a tile) at precision 33, 1, 2, 4 or 8 at
+ *                             64.  unit_off int64[D+1]: units of each design.
+ *   cctamd_far_build          perm int64[U] holds the unit numbers in ascending order of their
+ *                             keys and is rearranged; cluster_off int64[D+1] counts the small
+ *                             clusters (a multiple of 4 per design, C in all), chunk_off
+ *                             int64[D+1] stretches of 16,384 units (the last one of a design
+ *                             may be shorter).  Writes geo double[C][8], geo_large
+ *                             double[C/4][8], coef and coef_large (allocated with 128 doubles more
+ *                             than their clusters), and rows double[C*512 + 4][6] (precision 64:
+ *                             {kl, m} in cluster order, passed as `seg` when tracking) or
+ *                             tiles int32[C*16] (precision 33); mom is scratch for C clusters.
+ *   cctamd_far_plan           work items as in cctamd_plan (host arrays), the tile range replaced
+ *                             by the design's first small cluster and their number: an
+ *                             item takes its share of what its block needs of them.
+ * cctamd_track_rk4_far is cctamd_track_rk4 with these clusters (precision 33: ppl 1, 2, 4, -2;
+ * precision 64: any ppl).
+ */
+int64_t cctamd_far_coef_doubles(int precision);
+int cctamd_far_keys(const double *seg64, int unit, const int64_t *unit_off, int64_t ndesign, int64_t nunit,
+                    int64_t *key, float *centre, void *stream);
+int cctamd_far_build(int precision, const double *seg64, int unit, const float *centre, const int64_t *unit_off,
+                     const int64_t *chunk_off, int64_t nchunk, const int64_t *cluster_off, int64_t ndesign,
+                     int64_t ncluster, int64_t *perm, double *rows, int32_t *tiles, double *geo, double *geo_large,
+                     double *mom, double *coef, double *coef_large, void *stream);
+int64_t cctamd_far_plan(int64_t ndesign, const int64_t *design_ntile, const int64_t *design_npt,
+                        const int64_t *design_cluster_off, const int64_t *design_pt_off, int ppl,
+                        int64_t target_items, int32_t *work, int64_t *design_wbase, int32_t *design_nchunk);
+int cctamd_track_rk4_far(const double *geo, const double *geo_large, const double *coef, const double *coef_large,
+                         const int32_t *tiles, int precision, int ppl, const void *seg, const double *tile_org,
+                         const double *seg_near, const int32_t *work, int64_t nwork, const int64_t *design_wbase,
+                         const int32_t *design_nchunk, const int64_t *design_pt_off, int64_t ndesign,
+                         const double *qs, const int64_t *design_qs_off, const double *bconst, double *state,
+                         int64_t nparticles, const double *kq, const double *dt, const int64_t *nsteps,
+                         int64_t max_steps, double *scratch, double *partial, double *record,
+                         int64_t record_every, void *stream);
+
+/*
  * Winding tangents for the adjoint, per tile of a segment set whose CCTs each start
  * on a tile boundary: float[ntile][33][8]; entry k < 32 is the winding point at the
  * start of the tile's segment k, entry 32 the end point of segment 31:
