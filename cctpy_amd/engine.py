@@ -34,14 +34,18 @@ _TARGET_WG_PER_CU = 4
 _MIN_TILES_PER_ITEM = 4
 _LARGE_TILES = 64   # tiles of a large segment cluster (kParts * kSmallTiles in csrc/far.hpp)
 _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
-# Where tracking takes the far field (per launch: lanes x segments, large clusters per design).  Measured
-# per RK4 stage, all segments summed against the far field: FP64, 64 protons in one CCT of 360 tiles
-# (2.9e6, 12 clusters) 13 / 20 us, 300 in one of 1,440 (1.8e7, 23) 34 / 22-28, 24 in two gantries at 120 segments
-# per winding (1.0e7, 79) 21 / 15, 64 protons in the AG-CCT section at 360 (1.2e7, 90) 24 / 16-21, 512 at
-# 720 (1.9e8, 180) 158 / 45-60.
-_FAR_MIN_PAIRS = {64: 1.0e7}
-_FAR_MIN_LARGE = {64: 60}
-_FAR_ANY_PAIRS = {64: 4.0e7}  # from here on whatever the number of clusters
+# Where tracking takes the far field: lanes x segments of a launch and large clusters per design from
+# which it does, or the lanes x segments from which it does whatever the clusters; the pair terms per
+# second of the full sum (64-point blocks and larger, smaller blocks), the share of their time that it
+# saves at the least, and the work items per cluster and block of a single design.
+# Measured per RK4 stage, full sum / far field.  FP64: 64 protons in one CCT of 360 tiles (2.9e6, 12
+# clusters) 13 / 20 us, 300 in one of 1,440 (1.8e7, 23) 34 / 22-28, 24 in two gantries at 120 segments per
+# winding (1.0e7, 79) 21 / 15, 64 in the AG-CCT section at 360 (1.2e7, 90) 24 / 16-21, 512 at 720 (1.9e8, 180)
+# 158 / 45-60.  FP32: 2,048 protons in the CCT of 1,440 tiles (9.4e7, 23) 53 / 45-55, 400 in the gantry at
+# 60 (4.1e7, 31) 37 / 29, 64 in the section at 360 (1.2e7, 90) 18 / 18-23, 128 at 720 (4.7e7, 180) 37-40 /
+# 24-34, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 300.
+_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.5, share=11),
+        33: dict(pairs=4.0e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
 
 
 def device() -> torch.device:
@@ -330,18 +334,20 @@ class DeviceModel:
     def _far_pays(self, plan: Plan, precision: int, max_steps: int) -> bool:
         """Whether tracking ``plan`` for ``max_steps`` steps is faster with the far field, its set-up
         (once per model) included: a function of the sizes alone, so that equal calls give equal bits."""
-        if precision not in _FAR_MIN_PAIRS or plan.npt == 0 or self.nseg_padded == 0 or self.ndesign > 0x7fff:
+        if precision not in _FAR or plan.npt == 0 or self.nseg_padded == 0 or self.ndesign > 0x7fff:
             return False
+        if precision == 33 and plan.ppl == -4:
+            return False  # no far-field kernel for 16-point blocks of the FP32 path
+        rule = _FAR[precision]
         pb = points_per_block(plan.ppl)
         blocks = -(-numpy.asarray(plan.design_npt, numpy.int64) // pb)
         pairs = float((blocks * pb * self.design_ntile).sum()) * N.TILE
         large = float((blocks * self.design_ntile).sum()) / max(float(blocks.sum()), 1.0) / _LARGE_TILES
-        if pairs < _FAR_MIN_PAIRS[precision] or (large < _FAR_MIN_LARGE[precision]
-                                                 and pairs < _FAR_ANY_PAIRS[precision]):
+        if pairs < rule["pairs"] or (large < rule["large"] and pairs < rule["any_pairs"]):
             return False
-        # the set-up takes 1.5 ms + 2 ns per segment; a stage saves a third of its pair terms' time at
-        # the least (1.2e12 terms per second summed one by one)
-        return 4 * max_steps * pairs / 3 / 1.2e12 > 1.5e-3 + 2.0e-9 * self.nseg_padded
+        # the set-up, 1.5 ms + 2 (FP32 1) ns per segment, against what the stages save
+        rate = rule["rate"][0 if plan.ppl > 0 else 1]
+        return 4 * max_steps * rule["saved"] * pairs / rate > 1.5e-3 + precision / 32 * 1e-9 * self.nseg_padded
 
     def _far_plan(self, far: FarField, plan: Plan, precision: int) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
@@ -353,7 +359,8 @@ class DeviceModel:
         # 1,024 69 us; 24 designs x 32: 256 items 153 us, 1,440 84 us.
         clusters = int((-(-npt // points_per_block(plan.ppl)) * -(-nt // 16)).sum())
         cus = cu_count()
-        target = min(max(clusters // 5, cus), 6 * cus) if self.ndesign > 1 else min(max(clusters // 11, cus), 2 * cus)
+        target = min(max(clusters // 5, cus), 6 * cus) if self.ndesign > 1 else \
+            min(max(clusters // _FAR[precision]["share"], cus), 2 * cus)
         target = min(plan.nwork, target)
         while True:  # the caller's partial sums hold plan.nwork items (every point block has one)
             args = (self.ndesign, _np(nt), _np(npt), _np(far.cluster_off), _np(pt_off), plan.ppl)

@@ -3,7 +3,8 @@
 Single steps of 0.2 m, so that a relative field error e turns into a velocity error of about
 0.2 m / 0.95 m x e: with the cut of the series below 1e-15 and sums of up to 10^5 terms in another
 order (1e-14 at the worst of the forms below, which come to within centimetres of the windings) the
-states agree to 1e-13 of the velocity and 1e-13 m."""
+states agree to 1e-13 of the velocity and 1e-13 m.  FP32 path: both sums within 1e-6 of the
+field, so 2 x 0.21 x 1e-6 of each other."""
 import numpy as np
 import pytest
 import torch
@@ -20,7 +21,7 @@ from cctpy_amd.magnets import device_parts  # noqa: E402
 if not gpu_available():
     pytest.skip("no GPU visible", allow_module_level=True)
 
-TOLERANCE = {64: 1e-13}
+TOLERANCE = {64: 1e-13, 33: 4.2e-7}
 
 
 def _specs():
@@ -61,7 +62,8 @@ def _track(model, plan, precision, state, steps, far):
     return st.cpu().numpy()
 
 
-@pytest.mark.parametrize("precision,ppl", [(64, 1), (64, 2), (64, 4), (64, -2), (64, -4)])
+@pytest.mark.parametrize("precision,ppl", [(64, 1), (64, 2), (64, 4), (64, -2), (64, -4), (33, 1), (33, 2), (33, 4),
+                                           (33, -2)])
 @pytest.mark.parametrize("steps", [1, 3])
 def test_far_field_matches_the_full_sum(precision, ppl, steps, monkeypatch):
     monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
