@@ -80,13 +80,17 @@ __global__ void k_far_keys(const double* __restrict__ seg64, int unit, const int
 }
 
 // Splits a stretch of kChunk units of one design into halves across the longest side of their
-// bounding box, then each half, down to groups of `group` units (a power of two): every level
-// finds the median of each group bit by bit on 16-bit places along the side (all groups at
-// once) and moves the units to their half, in LDS.  Places past the design's units come last in
-// every group.  One workgroup per stretch; sorting the groups instead took eight times as long.
+// bounding box, then each half, down to groups of `group` units (a power of two).  Every level
+// finds the median of each group bit by bit and moves the units to their half, in LDS, all
+// groups at once; a thread holds kPer places of one group, so that a level of groups of up to
+// 1,024 units needs no barrier for its counts.  Places past the design's units come last in
+// every group.  One workgroup per stretch (0.23 ms; stretches of half the size take half of it but
+// cost the design search 8 % of its tracking, their clusters being rounder only within them).
 constexpr int kChunk = 16384;
 constexpr int kSplitWG = 1024;
 constexpr int kPer = kChunk / kSplitWG;
+constexpr int kSplitBits = 11;  // resolution of a split along its side
+constexpr unsigned kNoCurrent = 65534, kNoUnit = 65535;
 
 __device__ inline unsigned ordered_bits(float v) {
     const unsigned b = __float_as_uint(v);
@@ -96,141 +100,206 @@ __device__ inline float from_ordered_bits(unsigned b) {
     return __uint_as_float(b & 0x80000000u ? b & 0x7fffffffu : ~b);
 }
 
+// Smallest and largest of three values over the `width` neighbouring lanes (a power of two).
+__device__ inline void box_lanes(unsigned (&lo)[3], unsigned (&hi)[3], int width) {
+    for (int off = 1; off < width; off <<= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const unsigned a = __shfl_xor(lo[k], off), b = __shfl_xor(hi[k], off);
+            lo[k] = a < lo[k] ? a : lo[k];
+            hi[k] = b > hi[k] ? b : hi[k];
+        }
+}
+
 __global__ __launch_bounds__(kSplitWG) void k_far_split(int64_t* __restrict__ perm, const float4* __restrict__ centre,
                                                         const int64_t* __restrict__ unit_off,
                                                         const int64_t* __restrict__ chunk_off, int64_t nd, int group) {
-    constexpr int kMaxGroups = kChunk / 32;  // groups of a level: of 32 units at least
-    __shared__ uint16_t id[2][kChunk];
-    __shared__ unsigned box[6][kMaxGroups];
-    __shared__ int count[kMaxGroups], less[kMaxGroups], same[kMaxGroups];  // less, same: by run of `width` places
+    constexpr int kGroups = kChunk / (kWave * kPer);  // groups of more than a wave's places, at most
+    __shared__ uint16_t xyz[3][kChunk];               // places in the stretch's box, by unit
+    __shared__ uint16_t id[kChunk];
+    __shared__ unsigned box[6][kGroups];
+    __shared__ int count[2][kGroups], tot[2][kSplitWG / kWave];
     const int64_t d = find_design(chunk_off, nd, blockIdx.x);
     const int64_t first = unit_off[d] + ((int64_t)blockIdx.x - chunk_off[d]) * kChunk;
     const int64_t left = unit_off[d + 1] - first;
     const int n = left < kChunk ? (int)left : kChunk;
-    const int lane = threadIdx.x & (kWave - 1);
-    int from = 0;
-    for (int e = threadIdx.x; e < kChunk; e += kSplitWG) id[0][e] = (uint16_t)e;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, e0 = tid * kPer;
+    // the stretch's box (units with current), then every unit's place in it
+    if (tid < 6) box[tid][0] = tid < 3 ? 0xffffffffu : 0u;
+    __syncthreads();
+    {
+        unsigned lo[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, hi[3] = {0u, 0u, 0u};
+        for (int i = 0; i < kPer; ++i) {
+            if (e0 + i >= n) break;
+            const float4 c = centre[perm[first + e0 + i]];
+            if (!(c.x < 3.0e38f && c.y < 3.0e38f && c.z < 3.0e38f)) continue;
+            const unsigned v[3] = {ordered_bits(c.x), ordered_bits(c.y), ordered_bits(c.z)};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = v[k] < lo[k] ? v[k] : lo[k];
+                hi[k] = v[k] > hi[k] ? v[k] : hi[k];
+            }
+        }
+        box_lanes(lo, hi, kWave);
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                atomicMin(&box[k][0], lo[k]);
+                atomicMax(&box[3 + k][0], hi[k]);
+            }
+    }
+    __syncthreads();
+    {
+        float base[3], side = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            base[k] = from_ordered_bits(box[k][0]);
+            const float w = box[3 + k][0] >= box[k][0] ? from_ordered_bits(box[3 + k][0]) - base[k] : 0.0f;
+            side = w > side ? w : side;
+        }
+        const float scale = side > 0.0f ? 65533.0f / side : 0.0f;
+        for (int i = 0; i < kPer; ++i) {
+            const int e = e0 + i;
+            unsigned q[3] = {kNoUnit, kNoUnit, kNoUnit};
+            if (e < n) {
+                const float4 c = centre[perm[first + e]];
+                const bool with = c.x < 3.0e38f && c.y < 3.0e38f && c.z < 3.0e38f;
+                const float v[3] = {c.x, c.y, c.z};
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float f = (v[k] - base[k]) * scale;
+                    q[k] = !with ? kNoCurrent : f > 0.0f ? (f < 65533.0f ? (unsigned)f : 65533u) : 0u;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) xyz[k][e] = (uint16_t)q[k];
+            id[e] = (uint16_t)e;
+        }
+    }
     __syncthreads();
     for (int size = kChunk; size > group; size >>= 1) {
         if (size / 2 >= n) continue;  // uniform: nothing in the second half
-        const int ng = kChunk / size;
-        // place e = threadIdx.x + i kSplitWG: a wave's 64 places are `kWave / width` runs of one group each
-        const int width = size < kWave ? size : kWave;
-        const uint64_t run = (width == kWave ? ~0ull : ((1ull << width) - 1)) << (lane / width * width);
-        for (int i = threadIdx.x; i < 6 * ng; i += kSplitWG) box[i / ng][i % ng] = i / ng < 3 ? 0xffffffffu : 0u;
-        __syncthreads();
-        float4 c[kPer];
-        int what[kPer];  // 0: with current, 1: without, 2: no unit
+        const int threads = size / kPer, width = threads < kWave ? threads : kWave, g = e0 / size;
+        const bool wide = threads > kWave;  // uniform
+        unsigned what[kPer], lo[3] = {kNoUnit, kNoUnit, kNoUnit}, hi[3] = {0u, 0u, 0u};
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const int e = threadIdx.x + i * kSplitWG, u = id[from][e];
-            what[i] = 2;
-            unsigned lo[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, hi[3] = {0u, 0u, 0u};
-            if (u < n) {
-                c[i] = centre[perm[first + u]];
-                what[i] = c[i].x < 3.0e38f && c[i].y < 3.0e38f && c[i].z < 3.0e38f ? 0 : 1;
-                if (what[i] == 0) {
-                    lo[0] = hi[0] = ordered_bits(c[i].x);
-                    lo[1] = hi[1] = ordered_bits(c[i].y);
-                    lo[2] = hi[2] = ordered_bits(c[i].z);
-                }
-            }
-            for (int off = 1; off < width; off <<= 1)
-                for (int k = 0; k < 3; ++k) {
-                    const unsigned a = __shfl_xor(lo[k], off), b = __shfl_xor(hi[k], off);
-                    lo[k] = a < lo[k] ? a : lo[k];
-                    hi[k] = b > hi[k] ? b : hi[k];
-                }
-            if (lane % width == 0)
-                for (int k = 0; k < 3; ++k) {
-                    atomicMin(&box[k][e / size], lo[k]);
-                    atomicMax(&box[3 + k][e / size], hi[k]);
-                }
-        }
-        __syncthreads();
-        unsigned key[kPer], cut[kPer];
-        int want[kPer];
+            what[i] = id[e0 + i];
+            if (xyz[0][what[i]] >= kNoCurrent) continue;
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int g = (threadIdx.x + i * kSplitWG) / size;
-            float base = 0.0f, side = 0.0f, v = 0.0f;
             for (int k = 0; k < 3; ++k) {
-                const unsigned lo = box[k][g], hi = box[3 + k][g];
-                const float l = from_ordered_bits(lo), w = hi >= lo ? from_ordered_bits(hi) - l : 0.0f;
-                if (w > side) {
-                    side = w;
-                    base = l;
-                    v = k == 0 ? c[i].x : k == 1 ? c[i].y : c[i].z;
-                }
+                const unsigned v = xyz[k][what[i]];
+                lo[k] = v < lo[k] ? v : lo[k];
+                hi[k] = v > hi[k] ? v : hi[k];
             }
-            key[i] = what[i] == 2 ? 65535u : what[i] == 1 ? 65534u : side > 0.0f ? (unsigned)((v - base) / side * 65533.0f) : 0u;
-            cut[i] = 0;
-            want[i] = size / 2;  // the want-th smallest of those that agree with `cut` so far
         }
-        for (int bit = 15; bit >= 0; --bit) {
-            for (int g = threadIdx.x; g < ng; g += kSplitWG) count[g] = 0;
+        box_lanes(lo, hi, width);
+        if (wide) {
+            if (tid < 6 * kGroups) box[tid / kGroups][tid % kGroups] = tid / kGroups < 3 ? kNoUnit : 0u;
+            __syncthreads();
+            if (lane == 0)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    atomicMin(&box[k][g], lo[k]);
+                    atomicMax(&box[3 + k][g], hi[k]);
+                }
             __syncthreads();
 #pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const uint64_t m = __ballot((key[i] ^ cut[i]) >> bit == 0) & run;
-                if (lane % width == 0) atomicAdd(&count[(threadIdx.x + i * kSplitWG) / size], __popcll(m));
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = box[k][g];
+                hi[k] = box[3 + k][g];
             }
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < kPer; ++i) {
-                const int below = count[(threadIdx.x + i * kSplitWG) / size];
-                if (below < want[i]) {
-                    want[i] -= below;
-                    cut[i] |= 1u << bit;
-                }
-            }
-            __syncthreads();
         }
+        int axis = 0;
+        unsigned side = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const unsigned w = hi[k] >= lo[k] ? hi[k] - lo[k] : 0u;
+            if (w > side) {
+                side = w;
+                axis = k;
+            }
+        }
+        const unsigned base = axis == 0 ? lo[0] : axis == 1 ? lo[1] : lo[2];
+        const int bits = side ? 32 - __builtin_clz(side) : 0, shift = bits > kSplitBits ? bits - kSplitBits : 0;
+        unsigned key[kPer];
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const uint64_t ml = __ballot(key[i] < cut[i]) & run, ms = __ballot(key[i] == cut[i]) & run;
-            if (lane % width == 0) {
-                less[(threadIdx.x + i * kSplitWG) / width] = __popcll(ml);
-                same[(threadIdx.x + i * kSplitWG) / width] = __popcll(ms);
+            const unsigned v = xyz[axis][what[i]];
+            key[i] = v == kNoUnit ? (2u << kSplitBits) - 1 : v == kNoCurrent ? 1u << kSplitBits : (v - base) >> shift;
+        }
+        // the median: the want-th smallest key is `cut`
+        unsigned cut = 0;
+        int want = size / 2;
+        for (int bit = kSplitBits; bit >= 0; --bit) {
+            if (wide && tid < kGroups) count[bit & 1][tid] = 0;
+            int below = 0;
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) below += (key[i] ^ cut) >> bit == 0;
+            for (int off = 1; off < width; off <<= 1) below += __shfl_xor(below, off);
+            if (wide) {
+                __syncthreads();
+                if (lane == 0) atomicAdd(&count[bit & 1][g], below);
+                __syncthreads();
+                below = count[bit & 1][g];
+            }
+            if (below < want) {
+                want -= below;
+                cut |= 1u << bit;
             }
         }
-        __syncthreads();
+        // smaller and equal ones before this thread's places in its group
+        int l = 0, s = 0;
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const int e = threadIdx.x + i * kSplitWG, r0 = e / size * (size / width);
-            int l = 0, s = 0;  // smaller and equal ones before this place in its group
-            for (int r = r0; r < e / width; ++r) {
-                l += less[r];
-                s += same[r];
+            l += key[i] < cut;
+            s += key[i] == cut;
+        }
+        const int ownl = l, owns = s;
+        for (int off = 1; off < width; off <<= 1) {
+            const int a = __shfl_up(l, off), b = __shfl_up(s, off);
+            if ((lane & (width - 1)) >= off) {
+                l += a;
+                s += b;
             }
-            const uint64_t low = run & ((1ull << lane) - 1);
-            l += __popcll(__ballot(key[i] < cut[i]) & low);
-            s += __popcll(__ballot(key[i] == cut[i]) & low);
-            const int taken = s < want[i] ? s : want[i];  // equal ones that go to the first half
+        }
+        if (wide) {
+            if (lane == kWave - 1) {
+                tot[0][wave] = l;
+                tot[1][wave] = s;
+            }
+            __syncthreads();
+            for (int v = g * (threads / kWave); v < wave; ++v) {
+                l += tot[0][v];
+                s += tot[1][v];
+            }
+        }
+        l -= ownl;
+        s -= owns;
+        __syncthreads();  // every id has been read
+        int k = e0 - g * size;  // places before this one
+#pragma unroll
+        for (int i = 0; i < kPer; ++i, ++k) {
             int to;
-            if (key[i] < cut[i])
-                to = l;
-            else if (key[i] == cut[i] && s < want[i])
-                to = size / 2 - want[i] + s;
-            else
-                to = size / 2 + (e % size - l - taken);
-            id[from ^ 1][e / size * size + to] = id[from][e];
+            if (key[i] < cut)
+                to = l++;
+            else if (key[i] == cut && s < want)
+                to = size / 2 - want + s++;
+            else {
+                to = size / 2 + (k - l - (s < want ? s : want));
+                s += key[i] == cut;
+            }
+            id[g * size + to] = (uint16_t)what[i];
         }
         __syncthreads();
-        from ^= 1;
     }
     int64_t to[kPer];
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int e = threadIdx.x + i * kSplitWG;
-        to[i] = e < n ? perm[first + id[from][e]] : 0;
-    }
+    for (int i = 0; i < kPer; ++i) to[i] = e0 + i < n ? perm[first + id[e0 + i]] : 0;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const int e = threadIdx.x + i * kSplitWG;
-        if (e < n) perm[first + e] = to[i];
-    }
+    for (int i = 0; i < kPer; ++i)
+        if (e0 + i < n) perm[first + e0 + i] = to[i];
 }
 
 // The unit at each place of the clusters, -1 for none.
@@ -305,10 +374,15 @@ __device__ inline double wg_reduce(double v, double* lds, bool largest) {
 
 // Centre (middle of the bounding box) and radius of each cluster's current-carrying midpoints.
 // A cluster of one point gets a radius of 1 nm, one without current too (its series is zero).
+// Small clusters first, then the large ones (workgroups from nsmall on).
 __global__ __launch_bounds__(kFarWG) void k_far_balls(const double* __restrict__ rows, const int32_t* __restrict__ tiles,
-                                                      int ntile, double* __restrict__ geo) {
+                                                      int64_t nsmall, double* __restrict__ geo_small,
+                                                      double* __restrict__ geo_large) {
     __shared__ double lds[kFarWG];
-    const int64_t cl = blockIdx.x;
+    const bool large = blockIdx.x >= nsmall;
+    const int64_t cl = large ? blockIdx.x - nsmall : blockIdx.x;
+    const int ntile = large ? kParts * kSmallTiles : kSmallTiles;
+    double* geo = large ? geo_large : geo_small;
     const double inf = __builtin_huge_val();
     double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
     for (int i = threadIdx.x; i < ntile * kTile; i += kFarWG) {
@@ -350,11 +424,15 @@ __global__ __launch_bounds__(kFarWG) void k_far_balls(const double* __restrict__
 // Moments of the vector potential, sum over the cluster's rows of kl R_n^m((m - c) / E) with
 // the regular solid harmonics R_n^m = r^n P_n^m e^{i m phi} / (n + m)!:
 //   R_m^m = (x + iy)^m / (2^m m!),  (n + 1 - m)(n + 1 + m) R_{n+1} = (2n + 1) z R_n - r^2 R_{n-1}.
-// One wave per (cluster, m): its lanes stride the rows, kFarChunk orders at a time in
-// registers; the lanes' sums are added in a fixed order through LDS (kFarHalf orders at a
-// time), which costs 150 instructions per chunk where shuffles cost 1,400.
-constexpr int kFarChunk = 8, kFarHalf = 4;
+// One workgroup per small cluster's 512 rows, staged in LDS; a large cluster's moments are
+// the sum of its parts' about its own centre (k_far_coef adds them).  A wave takes one m at a
+// time, eight rows per lane whose recurrences stay in registers, kFarChunk orders per round;
+// the lanes' sums are added in a fixed order through LDS.  10 FP64 instructions per row and
+// order: 0.1 ms for the AG-CCT section's 368,640 rows, where one wave per m that read the rows
+// from memory for every eight orders took 0.29 ms.
+constexpr int kFarChunk = 4;
 constexpr int kMomWaves = 4;
+constexpr int kMomRows = kSmallTiles * kTile, kMomPer = kMomRows / kWave;
 
 // The recurrence's factors (2n + 1) / q and 1 / q, q = (n + 1 - m)(n + 1 + m), by n - m, for every m.
 struct RegularFactors {
@@ -373,80 +451,96 @@ constexpr RegularFactors regular_factors() {
 __constant__ RegularFactors kRegular = regular_factors();
 
 __global__ __launch_bounds__(kWave * kMomWaves) void k_far_moments(const double* __restrict__ rows,
-                                                                   const int32_t* __restrict__ tiles, int ntile, int q,
-                                                                   const double* __restrict__ geo,
+                                                                   const int32_t* __restrict__ tiles, int q, int64_t nsmall,
+                                                                   const double* __restrict__ geo_small,
+                                                                   const double* __restrict__ geo_large,
                                                                    double* __restrict__ mom) {
-    __shared__ double lds[kMomWaves][kFarHalf * 6][kWave + 1];
-    const int64_t cl = blockIdx.x;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    __shared__ double row[6][kMomRows];  // (m - c) / E and kl; zeros for a row without current
+    __shared__ double lds[kMomWaves][kFarChunk * 6][kWave + 1];
+    const bool large = blockIdx.x >= nsmall;  // about the large cluster's centre: the second half of the sets
+    const int64_t cl = large ? blockIdx.x - nsmall : blockIdx.x;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int top = 4 * q - 2;  // highest order of the potential
-    const int m = __builtin_amdgcn_readfirstlane(blockIdx.y * kMomWaves + wave);
-    if (m > top) return;  // whole waves; no barrier below
-    double(*mine)[kWave + 1] = lds[wave];
-    const double* g = geo + cl * kFarGeo;
+    const double* g = large ? geo_large + cl / kParts * kFarGeo : geo_small + cl * kFarGeo;
     const double inv = g[3];
-    double f = 1.0;
-    for (int k = 1; k <= m; ++k) f /= 2.0 * k;
-    double* out = mom + (cl * far_records(q) + far_row(q, m)) * 6;
-    const double(*fac)[2] = kRegular.f[m];  // wave-uniform: scalar loads
-#pragma unroll 1
-    for (int n0 = m; n0 <= top; n0 += kFarChunk) {
-        double acc[kFarChunk][6];
+    for (int i = threadIdx.x; i < kMomRows; i += kWave * kMomWaves) {
+        ClusterRow r;
+        const bool live = cluster_row(rows, tiles, cl, kSmallTiles, i, r);
 #pragma unroll
-        for (int k = 0; k < kFarChunk; ++k)
-#pragma unroll
-            for (int c = 0; c < 6; ++c) acc[k][c] = 0.0;
+        for (int c = 0; c < 3; ++c) {
+            row[c][i] = live ? (r.m[c] - g[c]) * inv : 0.0;
+            row[3 + c][i] = live ? r.kl[c] : 0.0;
+        }
+    }
+    __syncthreads();
+    double(*mine)[kWave + 1] = lds[wave];
 #pragma unroll 1
-        for (int i = lane; i < ntile * kTile; i += kWave) {  // the same number of rounds in every lane
-            ClusterRow r;
-            const bool live = cluster_row(rows, tiles, cl, ntile, i, r);
-            const double x = live ? (r.m[0] - g[0]) * inv : 0.0, y = live ? (r.m[1] - g[1]) * inv : 0.0;
-            const double z = live ? (r.m[2] - g[2]) * inv : 0.0;
-            const double r2 = x * x + y * y + z * z;
-            double pc = live ? f : 0.0, ps = 0.0, bc = x, bs = y;  // f (x + iy)^m by squares
+    for (int turn = 0; turn * kMomWaves <= top; ++turn) {
+        // m in turns, there and back: row m has top - m + 1 orders
+        const int m = turn * kMomWaves + (turn & 1 ? kMomWaves - 1 - wave : wave);
+        if (m > top) continue;
+        const double(*fac)[2] = kRegular.f[m];  // wave-uniform: scalar loads
+        double f = 1.0;
+        for (int k = 1; k <= m; ++k) f /= 2.0 * k;
+        double* out = mom + ((int64_t)blockIdx.x * far_records(q) + far_row(q, m)) * 6;
+        double pc[kMomPer], ps[kMomPer], cur[kMomPer], old[kMomPer];
+#pragma unroll
+        for (int j = 0; j < kMomPer; ++j) {
+            const double x = row[0][lane + j * kWave], y = row[1][lane + j * kWave];
+            pc[j] = f;  // f (x + iy)^m by squares
+            ps[j] = 0.0;
+            double bc = x, bs = y;
             for (int k = m; k != 0; k >>= 1) {
                 if (k & 1) {
-                    const double t = pc * bc - ps * bs;
-                    ps = pc * bs + ps * bc;
-                    pc = t;
+                    const double t = pc[j] * bc - ps[j] * bs;
+                    ps[j] = pc[j] * bs + ps[j] * bc;
+                    pc[j] = t;
                 }
                 const double t = bc * bc - bs * bs;
                 bs = 2.0 * bc * bs;
                 bc = t;
             }
-            double cur = 1.0, old = 0.0;  // R_n over R_m^m
-            for (int n = m; n < n0; ++n) {
-                const double nx = fac[n - m][0] * (z * cur) - fac[n - m][1] * (r2 * old);
-                old = cur;
-                cur = nx;
-            }
-            const double k0 = live ? r.kl[0] : 0.0, k1 = live ? r.kl[1] : 0.0, k2 = live ? r.kl[2] : 0.0;
-            const double kc[3] = {k0 * pc, k1 * pc, k2 * pc}, ks[3] = {k0 * ps, k1 * ps, k2 * ps};
-#pragma unroll
-            for (int k = 0; k < kFarChunk; ++k) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    acc[k][c] = __builtin_fma(kc[c], cur, acc[k][c]);
-                    acc[k][3 + c] = __builtin_fma(ks[c], cur, acc[k][3 + c]);
-                }
-                const double nx = fac[n0 + k - m][0] * (z * cur) - fac[n0 + k - m][1] * (r2 * old);
-                old = cur;
-                cur = nx;
-            }
+            cur[j] = 1.0;  // R_n over R_m^m
+            old[j] = 0.0;
         }
+#pragma unroll 1
+        for (int n0 = m; n0 <= top; n0 += kFarChunk) {
+            double acc[kFarChunk][6];
 #pragma unroll
-        for (int h = 0; h < kFarChunk; h += kFarHalf) {
+            for (int k = 0; k < kFarChunk; ++k)
 #pragma unroll
-            for (int k = 0; k < kFarHalf; ++k)
+                for (int c = 0; c < 6; ++c) acc[k][c] = 0.0;
 #pragma unroll
-                for (int c = 0; c < 6; ++c) mine[k * 6 + c][lane] = acc[h + k][c];
+            for (int j = 0; j < kMomPer; ++j) {
+                const int i = lane + j * kWave;
+                const double x = row[0][i], y = row[1][i], z = row[2][i];
+                const double r2 = x * x + y * y + z * z;
+                const double kc[3] = {row[3][i] * pc[j], row[4][i] * pc[j], row[5][i] * pc[j]};
+                const double ks[3] = {row[3][i] * ps[j], row[4][i] * ps[j], row[5][i] * ps[j]};
+#pragma unroll
+                for (int k = 0; k < kFarChunk; ++k) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) {
+                        acc[k][c] = __builtin_fma(kc[c], cur[j], acc[k][c]);
+                        acc[k][3 + c] = __builtin_fma(ks[c], cur[j], acc[k][3 + c]);
+                    }
+                    const double nx = fac[n0 + k - m][0] * (z * cur[j]) - fac[n0 + k - m][1] * (r2 * old[j]);
+                    old[j] = cur[j];
+                    cur[j] = nx;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kFarChunk; ++k)
+#pragma unroll
+                for (int c = 0; c < 6; ++c) mine[k * 6 + c][lane] = acc[k][c];
             __builtin_amdgcn_wave_barrier();
             const int v = lane >> 1;  // two lanes per value
             double s = 0.0;
-            if (v < kFarHalf * 6)
+            if (v < kFarChunk * 6)
+#pragma unroll
                 for (int i = 0; i < kWave / 2; ++i) s += mine[v][(lane & 1) * (kWave / 2) + i];
             s += __shfl_xor(s, 1);
-            if (v < kFarHalf * 6 && (lane & 1) == 0 && n0 + h + v / 6 <= top) out[(n0 - m + h) * 6 + v] = s;
+            if (v < kFarChunk * 6 && (lane & 1) == 0 && n0 + v / 6 <= top) out[(n0 - m) * 6 + v] = s;
             __builtin_amdgcn_wave_barrier();
         }
     }
@@ -455,11 +549,19 @@ __global__ __launch_bounds__(kWave * kMomWaves) void k_far_moments(const double*
 // Coefficients of the field, B = curl A, order n from the potential's order n - 1:
 //   d/dx, d/dy and d/dz of the exterior harmonic I_n^m are (I_{n+1}^{m-1} - I_{n+1}^{m+1}) / 2,
 //   i (I_{n+1}^{m-1} + I_{n+1}^{m+1}) / 2 and -I_{n+1}^m  (I^{-1} = -conj I^1).
-__global__ void k_far_coef(int q, int64_t nrec, const double* __restrict__ geo, const double* __restrict__ mom,
-                           double* __restrict__ coef) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nrec) return;
+// A large cluster's moments are the sum of its parts' (records from nsmall * far_records on).
+__global__ void k_far_coef(int q, int64_t nsmall, int64_t nrec, const double* __restrict__ geo_small,
+                           const double* __restrict__ geo_large, const double* __restrict__ mom,
+                           double* __restrict__ coef_small, double* __restrict__ coef_large) {
+    const int64_t at = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (at >= nrec) return;
     const int per = far_records(q);
+    const bool large = at >= nsmall * per;
+    const int64_t i = large ? at - nsmall * per : at;
+    const int parts = large ? kParts : 1;
+    const double* geo = large ? geo_large : geo_small;
+    double* coef = large ? coef_large : coef_small;
+    if (large) mom += nsmall * per * 6;
     const int64_t cl = i / per;
     const int rec = (int)(i % per), top = 4 * q - 1;
     int m = 0;
@@ -471,10 +573,12 @@ __global__ void k_far_coef(int q, int64_t nrec, const double* __restrict__ geo, 
     if (n > 0) o[6] = -(double)(n * n - m * m) / (double)((2 * n + 1) * (2 * n - 1));
     if (n == 0) return;
     // a(k, c): coefficient of the potential's Re I_{n-1}^k (c < 3) or Im I_{n-1}^k (c >= 3)
-    const double* base = mom + cl * per * 6;
+    const double* base = mom + cl * parts * per * 6;
     const auto a = [&](int k, int c) {
         if (k < 0 || k > n - 1 || (c >= 3 && k == 0)) return 0.0;
-        const double v = base[(far_row(q, k) + (n - 1 - k)) * 6 + c];
+        const double* at = base + (far_row(q, k) + (n - 1 - k)) * 6 + c;
+        double v = at[0];
+        for (int p = 1; p < parts; ++p) v += at[(int64_t)p * per * 6];
         return k == 0 ? v : 2.0 * v;
     };
     const double lowc = m == 1 ? 1.0 : 0.5;  // Re I^0 has only its I^1 neighbour
@@ -536,7 +640,7 @@ int cctamd_far_build(int precision, const double* seg64, int unit, const float* 
     if (precision == 64 ? !rows : !tiles) return CCTAMD_EINVAL;
     const int q = precision == 64 ? kFarQ64 : kFarQ32;
     const int ntile = kSmallTiles;
-    const int64_t places = ncluster * ntile, nrec = ncluster * far_records(q);
+    const int64_t places = ncluster * ntile, nrec = 2 * ncluster * far_records(q);
     if (places > 0x7fffffff || ceil_div(places * kTile * 2, 256) > 0x7fffffff || ceil_div(nrec, 256) > 0x7fffffff ||
         nchunk > 0x7fffffff)
         return CCTAMD_ERANGE;
@@ -551,17 +655,13 @@ int cctamd_far_build(int precision, const double* seg64, int unit, const float* 
                            cluster_off, ndesign, (int64_t)ntile, places, tiles);
     const double* src = precision == 64 ? rows : seg64;
     const int32_t* ids = precision == 64 ? nullptr : tiles;
-    for (int large = 0; large < 2; ++large) {
-        const int64_t nc = large ? ncluster / kParts : ncluster;
-        const int nt = large ? kParts * kSmallTiles : ntile;
-        double* g = large ? geo_large : geo;
-        const int64_t nr = nc * far_records(q);
-        hipLaunchKernelGGL(k_far_balls, dim3((unsigned)nc), dim3(kFarWG), 0, st, src, ids, nt, g);
-        hipLaunchKernelGGL(k_far_moments, dim3((unsigned)nc, (unsigned)((4 * q - 1 + kMomWaves - 1) / kMomWaves)),
-                           dim3(kWave * kMomWaves), 0, st, src, ids, nt, q, g, mom);
-        hipLaunchKernelGGL(k_far_coef, dim3((unsigned)ceil_div(nr, 256)), dim3(256), 0, st, q, nr, g, mom,
-                           large ? coef_large : coef);
-    }
+    const int64_t nlarge = ncluster / kParts, nr = (ncluster + nlarge) * far_records(q);
+    hipLaunchKernelGGL(k_far_balls, dim3((unsigned)(ncluster + nlarge)), dim3(kFarWG), 0, st, src, ids, ncluster, geo,
+                       geo_large);
+    hipLaunchKernelGGL(k_far_moments, dim3((unsigned)(2 * ncluster)), dim3(kWave * kMomWaves), 0, st, src, ids, q,
+                       ncluster, geo, geo_large, mom);
+    hipLaunchKernelGGL(k_far_coef, dim3((unsigned)ceil_div(nr, 256)), dim3(256), 0, st, q, ncluster, nr, geo, geo_large,
+                       mom, coef, coef_large);
     return hip_status(hipGetLastError());
 }
 

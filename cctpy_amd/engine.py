@@ -44,7 +44,7 @@ _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # 158 / 45-60.  FP32: 2,048 protons in the CCT of 1,440 tiles (9.4e7, 23) 53 / 45-55, 400 in the gantry at
 # 60 (4.1e7, 31) 37 / 29, 64 in the section at 360 (1.2e7, 90) 18 / 18-23, 128 at 720 (4.7e7, 180) 37-40 /
 # 24-34, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 300.
-_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.5, share=11),
+_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.6, share=11),
         33: dict(pairs=4.0e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
 
 
@@ -149,7 +149,7 @@ class FarField:
         unit_off = model.design_tile_off * (N.TILE // unit)
         chunk_off = numpy.concatenate([[0], numpy.cumsum(-(-numpy.diff(unit_off) // _FAR_CHUNK))]).astype(numpy.int64)
         U = int(unit_off[-1])
-        uo, co, so = (torch.from_numpy(a).to(dev) for a in (unit_off, self.cluster_off, chunk_off))
+        uo, co, so = torch.from_numpy(numpy.stack([unit_off, self.cluster_off, chunk_off])).to(dev)  # one copy
         key = torch.empty(U, dtype=torch.int64, device=dev)
         centre = torch.empty((U, 4), dtype=torch.float32, device=dev)
         N.check(N.lib.cctamd_far_keys(_p(model.seg64), unit, _p(uo), model.ndesign, U, _p(key), _p(centre),
@@ -164,7 +164,7 @@ class FarField:
         self.tiles = empty(C * 16, torch.int32) if precision != 64 else None
         self.geo, self.geo_large = empty(8 * C), empty(2 * C)
         self.coef, self.coef_large = empty(C * per + 128), empty(C // 4 * per + 128)
-        mom = empty(C * per // 4 * 3)
+        mom = empty(2 * C * per // 4 * 3)
         N.check(N.lib.cctamd_far_build(precision, _p(model.seg64), unit, _p(centre), _p(uo), _p(so), int(chunk_off[-1]),
                                        _p(co), model.ndesign, C, _p(perm), _p(self.rows), _p(self.tiles),
                                        _p(self.geo), _p(self.geo_large), _p(mom), _p(self.coef),
@@ -345,9 +345,9 @@ class DeviceModel:
         large = float((blocks * self.design_ntile).sum()) / max(float(blocks.sum()), 1.0) / _LARGE_TILES
         if pairs < rule["pairs"] or (large < rule["large"] and pairs < rule["any_pairs"]):
             return False
-        # the set-up, 1.5 ms + 2 (FP32 1) ns per segment, against what the stages save
+        # the set-up, 0.35 ms + 1.3 (FP32 0.7) ns per segment, against what the stages save
         rate = rule["rate"][0 if plan.ppl > 0 else 1]
-        return 4 * max_steps * rule["saved"] * pairs / rate > 1.5e-3 + precision / 32 * 1e-9 * self.nseg_padded
+        return 4 * max_steps * rule["saved"] * pairs / rate > 0.35e-3 + precision * 2e-11 * self.nseg_padded
 
     def _far_plan(self, far: FarField, plan: Plan, precision: int) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)

@@ -199,7 +199,7 @@ int cctamd_track_rk4(int precision, int ppl, const void *seg, const double *tile
  *                             double[C/4][8], coef and coef_large (allocated with 128 doubles more
  *                             than their clusters), and rows double[C*512 + 4][6] (precision 64:
  *                             {kl, m} in cluster order, passed as `seg` when tracking) or
- *                             tiles int32[C*16] (precision 33); mom is scratch for C clusters.
+ *                             tiles int32[C*16] (precision 33); mom is scratch for 2 C clusters.
  *   cctamd_far_plan           work items as in cctamd_plan (host arrays), the tile range replaced
  *                             by the design's first small cluster and their number: an
  *                             item takes its share of what its block needs of them.
