@@ -1407,6 +1407,14 @@ hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* 
                                   FarSet{});
 }
 
+// The Biot-Savart pass of a segment set, with its clusters if it has any.
+hipError_t launch_bs_set(const DeviceSet& ds, const double* pts, int64_t ptot, double* partial, hipStream_t st) {
+    return ds.far.geo ? launch_bs_shape<true>(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork,
+                                              pts, ptot, partial, st, ds.far)
+                      : launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
+                                      ptot, partial, st);
+}
+
 int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, double* partial, double* B,
                   hipStream_t st) {
     if (!valid_common(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.nwork, ds.ndesign))
@@ -1419,8 +1427,7 @@ int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, do
     if (ds.nwork > 0 && (!ds.work || !partial)) return CCTAMD_EINVAL;
     const int64_t blocks = ceil_div(npoints, kWavesPerWG);
     if (blocks > 0x7fffffff) return CCTAMD_ERANGE;
-    hipError_t e = launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, points,
-                                 npoints, partial, st);
+    hipError_t e = launch_bs_set(ds, points, npoints, partial, st);
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(k_field_reduce, dim3((unsigned)blocks), dim3(kWG), 0, st, ds.ppl, partial, ds.design_wbase,
                        ds.design_nchunk, ds.design_pt_off, ds.ndesign, ds.qs, ds.design_qs_off, ds.bconst, points,
@@ -1463,10 +1470,7 @@ hipError_t launch_rk4_steps(const DeviceSet& ds, double* state, int64_t ptot, co
     if (fused) {                                                                                                  \
         e = launch_bs_stage<S>(ds, ptot, partial, sa, st);                                                        \
     } else {                                                                                                      \
-        e = ds.far.geo ? launch_bs_shape<true>(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work,   \
-                                               ds.nwork, scratch, ptot, partial, st, ds.far)                      \
-                       : launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, \
-                                       scratch, ptot, partial, st);                                               \
+        e = launch_bs_set(ds, scratch, ptot, partial, st);                                                        \
         if (e != hipSuccess) return e;                                                                            \
         hipLaunchKernelGGL(k_rk4_stage<S>, dim3((unsigned)rblocks), dim3(kWG), 0, st, sa);                        \
         e = hipGetLastError();                                                                                    \
@@ -1619,6 +1623,11 @@ int cctamd_bs_field(int precision, int ppl, const void* seg, const double* tile_
 }
 
 namespace {
+bool valid_far(const FarSet& far, int precision, int ppl) {
+    if (!far.geo || !far.geo_large || !far.coef || !far.coef_large) return false;
+    return precision == 33 ? far.tiles != nullptr && ppl != -4 : precision == 64;
+}
+
 int track_checked(const DeviceSet& ds, double* state, int64_t nparticles, const double* kq, const double* dt,
                   const int64_t* nsteps, int64_t max_steps, double* scratch, double* partial, double* record,
                   int64_t record_every, void* stream) {
@@ -1648,6 +1657,19 @@ int cctamd_track_rk4(int precision, int ppl, const void* seg, const double* tile
                          stream);
 }
 
+int cctamd_bs_field_far(const double* geo, const double* geo_large, const double* coef, const double* coef_large,
+                        const int32_t* tiles, int precision, int ppl, const void* seg, const double* tile_org,
+                        const double* seg_near, const int32_t* work, int64_t nwork, const int64_t* design_wbase,
+                        const int32_t* design_nchunk, const int64_t* design_pt_off, int64_t ndesign, const double* qs,
+                        const int64_t* design_qs_off, const double* bconst, const double* points, int64_t npoints,
+                        double* partial, double* B, void* stream) {
+    const FarSet far{geo, geo_large, coef, coef_large, tiles};
+    if (!valid_far(far, precision, ppl) || (nwork > 0 && !partial)) return CCTAMD_EINVAL;
+    const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
+                       design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst, far};
+    return field_checked(ds, points, npoints, partial, B, (hipStream_t)stream);
+}
+
 int cctamd_track_rk4_far(const double* geo, const double* geo_large, const double* coef, const double* coef_large,
                          const int32_t* tiles, int precision, int ppl, const void* seg, const double* tile_org,
                          const double* seg_near, const int32_t* work, int64_t nwork, const int64_t* design_wbase,
@@ -1655,11 +1677,10 @@ int cctamd_track_rk4_far(const double* geo, const double* geo_large, const doubl
                          const int64_t* design_qs_off, const double* bconst, double* state, int64_t nparticles,
                          const double* kq, const double* dt, const int64_t* nsteps, int64_t max_steps, double* scratch,
                          double* partial, double* record, int64_t record_every, void* stream) {
-    if (!geo || !geo_large || !coef || !coef_large) return CCTAMD_EINVAL;
-    if (precision == 33 ? (!tiles || ppl == -4) : precision != 64) return CCTAMD_EINVAL;
+    const FarSet far{geo, geo_large, coef, coef_large, tiles};
+    if (!valid_far(far, precision, ppl)) return CCTAMD_EINVAL;
     const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
-                       design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst,
-                       FarSet{geo, geo_large, coef, coef_large, tiles}};
+                       design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst, far};
     return track_checked(ds, state, nparticles, kq, dt, nsteps, max_steps, scratch, partial, record, record_every,
                          stream);
 }

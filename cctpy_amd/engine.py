@@ -55,7 +55,8 @@ def device() -> torch.device:
 
 
 def _p(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() > 0 else ctypes.c_void_p(0)
+    """Device address for a void* argument (an int: a ctypes object for each argument costs a field call 1.2 us)."""
+    return t.data_ptr() if t is not None and t.numel() > 0 else None
 
 
 def _np(a: numpy.ndarray):
@@ -63,7 +64,7 @@ def _np(a: numpy.ndarray):
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch.cuda.current_stream().cuda_stream
 
 
 def points_per_block(ppl: int) -> int:
@@ -130,6 +131,8 @@ class Plan:
     design_pt_off: torch.Tensor
     npt: int
     design_npt: tuple = ()
+    pairs: float = 0.0  # lanes x segments of a launch
+    large: float = 0.0  # large segment clusters per block, in the mean
     far: Dict[int, FarPlan] = dc_field(default_factory=dict)  # by precision
 
 
@@ -306,13 +309,18 @@ class DeviceModel:
         p = Plan(ppl=ppl, nwork=int(n), work=torch.from_numpy(work).to(dev), wbase=torch.from_numpy(wbase).to(dev),
                  nchunk=torch.from_numpy(nchunk).to(dev), design_pt_off=torch.from_numpy(pt_off).to(dev),
                  npt=int(pt_off[-1]), design_npt=tuple(npt.tolist()))
+        pb = points_per_block(ppl)
+        blocks = -(-npt // pb)
+        tiles = float((blocks * nt).sum())
+        p.pairs, p.large = tiles * pb * N.TILE, tiles / max(float(blocks.sum()), 1.0) / _LARGE_TILES
         self._plans[key] = p
         return p
 
     # --------------------------------------------------------- far field
     def far_field(self, plan: Plan, precision: int, max_steps: int) -> Optional[FarField]:
-        """The segment clusters that tracking ``plan`` for ``max_steps`` steps uses, built on first
-        need, with their work items in ``plan.far``; None where every segment is summed."""
+        """The segment clusters that tracking ``plan`` for ``max_steps`` steps uses (0: one field
+        evaluation), built on first need, with their work items in ``plan.far``; None where every
+        segment is summed."""
         if not self._far_pays(plan, precision, max_steps):
             return None
         with self._far_lock:
@@ -332,22 +340,18 @@ class DeviceModel:
             return far
 
     def _far_pays(self, plan: Plan, precision: int, max_steps: int) -> bool:
-        """Whether tracking ``plan`` for ``max_steps`` steps is faster with the far field, its set-up
-        (once per model) included: a function of the sizes alone, so that equal calls give equal bits."""
-        if precision not in _FAR or plan.npt == 0 or self.nseg_padded == 0 or self.ndesign > 0x7fff:
+        """Whether tracking ``plan`` for ``max_steps`` steps (0: one evaluation) is faster with the far
+        field, its set-up (once per model) included: a function of the sizes alone, so that equal
+        calls give equal bits."""
+        rule = _FAR.get(precision)
+        if rule is None or plan.pairs < rule["pairs"] or (plan.large < rule["large"]
+                                                          and plan.pairs < rule["any_pairs"]):
             return False
-        if precision == 33 and plan.ppl == -4:
-            return False  # no far-field kernel for 16-point blocks of the FP32 path
-        rule = _FAR[precision]
-        pb = points_per_block(plan.ppl)
-        blocks = -(-numpy.asarray(plan.design_npt, numpy.int64) // pb)
-        pairs = float((blocks * pb * self.design_ntile).sum()) * N.TILE
-        large = float((blocks * self.design_ntile).sum()) / max(float(blocks.sum()), 1.0) / _LARGE_TILES
-        if pairs < rule["pairs"] or (large < rule["large"] and pairs < rule["any_pairs"]):
-            return False
-        # the set-up, 0.35 ms + 1.3 (FP32 0.7) ns per segment, against what the stages save
+        if self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
+            return False  # keys hold 15 bits of design; 16-point blocks of the FP32 path have no far-field kernel
+        # the set-up, 0.35 ms + 1.3 (FP32 0.7) ns per segment, against what the evaluations save
         rate = rule["rate"][0 if plan.ppl > 0 else 1]
-        return 4 * max_steps * rule["saved"] * pairs / rate > 0.35e-3 + precision * 2e-11 * self.nseg_padded
+        return max(4 * max_steps, 1) * rule["saved"] * plan.pairs / rate > 0.35e-3 + precision * 2e-11 * self.nseg_padded
 
     def _far_plan(self, far: FarField, plan: Plan, precision: int) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
@@ -370,32 +374,33 @@ class DeviceModel:
             if n <= plan.nwork or target == 1:
                 break
             target = max(1, target - (n - plan.nwork))
-        work = numpy.zeros((max(n, 1), N.WORK_INTS), numpy.int32)
-        wbase = numpy.zeros(self.ndesign, numpy.int64)
-        nchunk = numpy.zeros(self.ndesign, numpy.int32)
+        D = self.ndesign  # one buffer, one copy: offsets (8 bytes each), items, chunk counts
+        buf = numpy.zeros(2 * D + N.WORK_INTS * max(n, 1) + D, numpy.int32)
+        wbase, work, nchunk = buf[:2 * D], buf[2 * D:-D], buf[-D:]
         n2 = N.lib.cctamd_far_plan(*args, target, _np(work), _np(wbase), _np(nchunk))
         if n2 != n or n > plan.nwork:
             raise N.CctamdError(f"cctamd_far_plan: {n2} work items, {n} expected, {plan.nwork} at most")
-        dev = self.seg64.device
-        return FarPlan(n, torch.from_numpy(work).to(dev), torch.from_numpy(wbase).to(dev),
-                       torch.from_numpy(nchunk).to(dev))
+        on = torch.from_numpy(buf).to(self.seg64.device)
+        return FarPlan(n, on[2 * D:-D], on[:2 * D].view(torch.int64), on[-D:])
 
     def _track(self, plan: Plan, precision: int, state, kq, dt, nsteps, max_steps: int, scratch, partial, record,
                record_every: int, far_field: bool = True) -> None:
+        far = self.far_field(plan, precision, max_steps) if far_field and max_steps > 0 else None
+        self._call(N.lib.cctamd_track_rk4 if far is None else N.lib.cctamd_track_rk4_far, "cctamd_track_rk4", plan,
+                   precision, far, _p(state), plan.npt, _p(kq), _p(dt), _p(nsteps), int(max_steps), _p(scratch),
+                   _p(partial), _p(record), int(record_every))
+
+    def _call(self, function, name: str, plan: Plan, precision: int, far: Optional[FarField], *args) -> None:
+        """A library call on this segment set and plan, with its clusters where ``far`` gives them."""
         seg, org, near = self._seg(precision)
-        far = self.far_field(plan, precision, max_steps) if far_field else None
-        w = plan if far is None else plan.far[precision]
-        args = (_p(org), _p(near), _p(w.work), w.nwork, _p(w.wbase), _p(w.nchunk), _p(plan.design_pt_off),
-                self.ndesign, _p(self.qs), _p(self.design_qs_off), _p(self.bconst), _p(state), plan.npt, _p(kq),
-                _p(dt), _p(nsteps), int(max_steps), _p(scratch), _p(partial), _p(record), int(record_every),
-                _stream())
-        if far is None:
-            N.check(N.lib.cctamd_track_rk4(precision, plan.ppl, _p(seg), *args), "cctamd_track_rk4")
-        else:
-            rows = seg if far.rows is None else far.rows
-            N.check(N.lib.cctamd_track_rk4_far(_p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large),
-                                               _p(far.tiles), precision, plan.ppl, _p(rows), *args),
-                    "cctamd_track_rk4_far")
+        w, head = plan, ()
+        if far is not None:
+            w = plan.far[precision]
+            head = (_p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.tiles))
+            seg = seg if far.rows is None else far.rows
+        N.check(function(*head, precision, plan.ppl, _p(seg), _p(org), _p(near), _p(w.work), w.nwork, _p(w.wbase),
+                         _p(w.nchunk), _p(plan.design_pt_off), self.ndesign, _p(self.qs), _p(self.design_qs_off),
+                         _p(self.bconst), *args, _stream()), name)
 
     def _seg(self, precision: int):
         """(segment rows, tile origins, FP64 rows for near tiles) of a precision."""
@@ -424,11 +429,7 @@ class DeviceModel:
         soa = torch.from_numpy(numpy.ascontiguousarray(pts.T)).to(dev)
         out = torch.empty_like(soa)
         partial = torch.empty(max(plan.nwork * 3 * points_per_block(ppl), 1), dtype=torch.float64, device=dev)
-        seg, org, near = self._seg(precision)
-        N.check(N.lib.cctamd_bs_field(precision, ppl, _p(seg), _p(org), _p(near), _p(plan.work), plan.nwork, _p(plan.wbase),
-                                      _p(plan.nchunk), _p(plan.design_pt_off), self.ndesign, _p(self.qs),
-                                      _p(self.design_qs_off), _p(self.bconst), _p(soa), plan.npt, _p(partial),
-                                      _p(out), _stream()), "cctamd_bs_field")
+        self.field_tensors(plan, precision, soa, partial, out)
         return out.cpu().numpy().T.copy()
 
     # ---------------------------------------------------------- tracking
@@ -480,11 +481,10 @@ class DeviceModel:
     def field_tensors(self, plan: "Plan", precision: int, points: torch.Tensor, partial: torch.Tensor,
                       out: torch.Tensor) -> None:
         """B (3, P) at device points (3, P): Biot-Savart pass + fixed-order reduction + QS + uniform."""
-        seg, org, near = self._seg(precision)
-        N.check(N.lib.cctamd_bs_field(precision, plan.ppl, _p(seg), _p(org), _p(near), _p(plan.work), plan.nwork,
-                                      _p(plan.wbase), _p(plan.nchunk), _p(plan.design_pt_off), self.ndesign,
-                                      _p(self.qs), _p(self.design_qs_off), _p(self.bconst), _p(points), plan.npt,
-                                      _p(partial), _p(out), _stream()), "cctamd_bs_field")
+        # a map pays for its clusters in one call; on the FP32 path a field keeps the terms of every segment
+        far = self.far_field(plan, 64, 0) if precision == 64 and plan.pairs > _FAR[64]["pairs"] else None
+        self._call(N.lib.cctamd_bs_field if far is None else N.lib.cctamd_bs_field_far, "cctamd_bs_field", plan,
+                   precision, far, _p(points), plan.npt, _p(partial), _p(out))
 
     def bs_partial_tensors(self, plan: "Plan", precision: int, points: torch.Tensor, partial: torch.Tensor) -> None:
         """One launch of the split-K Biot-Savart kernel on device points (3, P)."""

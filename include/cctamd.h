@@ -203,8 +203,8 @@ int cctamd_track_rk4(int precision, int ppl, const void *seg, const double *tile
  *   cctamd_far_plan           work items as in cctamd_plan (host arrays), the tile range replaced
  *                             by the design's first small cluster and their number: an
  *                             item takes its share of what its block needs of them.
- * cctamd_track_rk4_far is cctamd_track_rk4 with these clusters (precision 33: ppl 1, 2, 4, -2;
- * precision 64: any ppl).
+ * cctamd_bs_field_far and cctamd_track_rk4_far are cctamd_bs_field and cctamd_track_rk4 with
+ * these clusters (precision 33: ppl 1, 2, 4, -2; precision 64: any ppl).
  */
 int64_t cctamd_far_coef_doubles(int precision);
 int cctamd_far_keys(const double *seg64, int unit, const int64_t *unit_off, int64_t ndesign, int64_t nunit,
@@ -216,6 +216,12 @@ int cctamd_far_build(int precision, const double *seg64, int unit, const float *
 int64_t cctamd_far_plan(int64_t ndesign, const int64_t *design_ntile, const int64_t *design_npt,
                         const int64_t *design_cluster_off, const int64_t *design_pt_off, int ppl,
                         int64_t target_items, int32_t *work, int64_t *design_wbase, int32_t *design_nchunk);
+int cctamd_bs_field_far(const double *geo, const double *geo_large, const double *coef, const double *coef_large,
+                        const int32_t *tiles, int precision, int ppl, const void *seg, const double *tile_org,
+                        const double *seg_near, const int32_t *work, int64_t nwork, const int64_t *design_wbase,
+                        const int32_t *design_nchunk, const int64_t *design_pt_off, int64_t ndesign,
+                        const double *qs, const int64_t *design_qs_off, const double *bconst, const double *points,
+                        int64_t npoints, double *partial, double *B, void *stream);
 int cctamd_track_rk4_far(const double *geo, const double *geo_large, const double *coef, const double *coef_large,
                          const int32_t *tiles, int precision, int ppl, const void *seg, const double *tile_org,
                          const double *seg_near, const int32_t *work, int64_t nwork, const int64_t *design_wbase,

@@ -98,3 +98,23 @@ def test_far_field_keeps_particles_apart(monkeypatch):
     assert np.isnan(got[:3, 7]).any()
     assert np.max(np.abs(got[:3, others] - want[:3, others])) <= 1e-13
     assert np.max(np.abs(got[3:, others] - want[3:, others])) <= 1e-13 * 1.8e8
+
+
+def test_far_field_of_a_map_matches_the_full_sum(monkeypatch):
+    """B of one evaluation: relative to its largest value both sums are within 1e-13 (10^5 terms in
+    another order, points from 3 mm to metres off the windings)."""
+    model = engine.DeviceModel(_specs(), fp32=False)
+    npt = [3, 130, 2, 40, 1, 257]
+    pts = torch.from_numpy(np.ascontiguousarray(_beam(npt)[:, :3].T)).to(engine.device())
+    for ppl in (1, 2, -2):
+        plan = model.plan(npt, ppl)
+        _, partial = model.workspace(plan)
+        out = []
+        for far in (True, False):
+            monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: far)
+            b = torch.full_like(pts, float("nan"))
+            model.field_tensors(plan, 64, pts, partial, b)
+            out.append(b.cpu().numpy())
+        assert np.all(np.isfinite(out[0]))
+        for d, (a, b) in enumerate(zip(*[np.split(o, np.cumsum(npt)[:-1], axis=1) for o in out])):
+            assert np.max(np.abs(a - b)) <= 1e-13 * max(np.max(np.abs(b)), 1e-300), (ppl, d)
