@@ -257,9 +257,9 @@ constexpr double kFp64Tile = 1.5;
 // VGPRs against 44 for k_bs_partial_f32k<1, 8>).  1 = no hint.
 constexpr int kKindF32 = 0, kKindF32k = 1, kKindF64 = 2;
 constexpr int fused_waves(int kind, int ppl, int s, bool far = false) {
-    // Far-field kernels: enough for two workgroups per CU (ppl 1, 2).  Their series hold 98 and
-    // 143 VGPRs by themselves; held to 96 and 128 they spill 1 and 13 outside its loop, and the
-    // 512-proton AG-CCT section's stage takes 58 instead of 67 us (FP32), one item per CU more.
+    // Far-field kernels: enough for two workgroups per CU (ppl 1, 2).  Held to 96 and 128 VGPRs they
+    // spill one register at most; unheld, the 512-proton AG-CCT section's stage took 67 instead of
+    // 58 us (FP32), one item per CU more.
     if (far) return ppl == 1 ? 5 : ppl == 2 ? 4 : 2;
     if (s < 0) return 1;
     if (kind == kKindF32) return ppl == 1 ? 6 : 4;
@@ -572,35 +572,21 @@ __device__ inline void tile_direct_term(const float4& a, const float4& b, const 
     bz += (a.x * ry - a.y * rx) * w3;
 }
 
-// A work item's share of its block's lists (far.hpp), for the scalar-load kernels: near tiles and
-// series are dealt out to all waves of the block's items, numbered so that neighbours in a
-// list go to different items.  A series is cut into NW shares (pairs of its rows m) as long
-// as the block has few series per wave: their lengths differ by a factor of ten, and one wave
-// alone takes 45,000 cycles for order 31 at two points per lane.  With many series each wave
-// takes whole ones, which saves the powers of X + iY that every sharer computes.
-constexpr int kFarShared = 4;  // series per wave of the block below which they are shared
-
-template <bool F64, int PPL, int NW, typename Tile>
+// A work item's share of its block's lists (far.hpp), for the scalar-load kernels: the segments of
+// the near clusters (near(list, its length, this wave's number, the number of waves)) and the
+// rows of the series are dealt out to all waves of the block's items.
+template <bool F64, int PPL, int NW, typename Near>
 __device__ __forceinline__ void far_scalar_walk(const FarSet& fs, const Work& w, int wave, int lane,
                                                 const double (&px)[PPL], const double (&py)[PPL],
                                                 const double (&pz)[PPL], double (&ax)[PPL], double (&ay)[PPL],
-                                                double (&az)[PPL], Tile&& tile) {
+                                                double (&az)[PPL], Near&& near) {
     __shared__ FarLists<NW> L;
     const Ball ball = block_ball<PPL>(px, py, pz);
     const int me = wave * w.nchunk + w.chunk, all = w.nchunk * NW;
     for (int base = 0; base * kParts < w.tile_count; base += FarLists<NW>::kRound) {
-        far_lists<F64, NW>(L, fs, w, ball, base, wave, lane);
-        const int ntile = __builtin_amdgcn_readfirstlane(L.nnear) * kSmallTiles;
-        for (int t = me; t < ntile; t += all)
-            tile(__builtin_amdgcn_readfirstlane(L.near[t / kSmallTiles]) * kSmallTiles + t % kSmallTiles);
-        // from the other end: the waves with one more near tile have one share less
-        const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
-        const int shares = nfar < kFarShared * all ? NW : 1;
-        for (int e = all - 1 - me; e < nfar * shares; e += all) {
-            const int s = e % shares;
-            far_entry<F64 ? kFarQ64 : kFarQ32, NW, PPL>(L, fs, e / shares, s, 2 * shares - 1 - s, 2 * shares, px, py, pz,
-                                                         ax, ay, az);
-        }
+        const FarCounts n = far_lists<F64, 1, NW>(L, fs, w, ball, base, wave, lane);
+        near(L.near, n.near, me, all);
+        far_share<F64 ? kFarQ64 : kFarQ32, 1>(L, n, fs, me, all, lane, px, py, pz, ax, ay, az);
         __syncthreads();  // before the next round's lists
     }
 }
@@ -669,9 +655,14 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
         }
     };
     if constexpr (FAR) {
-        far_scalar_walk<false, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az, [&](int place) {
-            const int t = __builtin_amdgcn_readfirstlane(fs.tiles[place]);
-            if (t >= 0) tile(t);
+        // whole tiles, neighbours to different items: their FP32 sums are those of the full sum
+        far_scalar_walk<false, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az,
+                                        [&](const int* list, int n, int me, int all) {
+            for (int k = me; k < n * kSmallTiles; k += all) {
+                const int place = __builtin_amdgcn_readfirstlane(list[k / kSmallTiles]) * kSmallTiles + k % kSmallTiles;
+                const int t = __builtin_amdgcn_readfirstlane(fs.tiles[place]);
+                if (t >= 0) tile(t);
+            }
         });
     } else {
         const int tend = w.tile_start + w.tile_count;
@@ -845,18 +836,15 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 6
         __shared__ FarLists<kWavesPerWG> L;
         const Ball ball = block_ball<2>(px, py, pz);
         for (int base = 0; base * kParts < w.tile_count; base += FarLists<kWavesPerWG>::kRound) {
-            far_lists<false, kWavesPerWG>(L, fs, w, ball, base, wave, lane);
-            const int ntile = L.nnear * kSmallTiles;
+            const int uwave = __builtin_amdgcn_readfirstlane(wave);
+            const FarCounts n = far_lists<false, 4, kWavesPerWG>(L, fs, w, ball, base, uwave, lane);
+            const int ntile = n.near * kSmallTiles;
             for (int t = w.chunk * NS + stream; t < ntile; t += w.nchunk * NS) {  // uniform within a row
                 const int id = fs.tiles[L.near[t / kSmallTiles] * kSmallTiles + t % kSmallTiles];
                 if (id >= 0) tile(id);
             }
-            // a series per wave, its rows m shared by the four rows of lanes
-            const int me = __builtin_amdgcn_readfirstlane(wave) * w.nchunk + w.chunk, all = w.nchunk * kWavesPerWG;
-            const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
             double ax[2] = {0.0, 0.0}, ay[2] = {0.0, 0.0}, az[2] = {0.0, 0.0};
-            for (int e = all - 1 - me; e < nfar; e += all)
-                far_entry<kFarQ32, kWavesPerWG, 2>(L, fs, e, lane / LG, 7 - lane / LG, 8, px, py, pz, ax, ay, az);
+            far_share<kFarQ32, 4>(L, n, fs, uwave * w.nchunk + w.chunk, w.nchunk * kWavesPerWG, lane, px, py, pz, ax, ay, az);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 acc[j][tid] += ax[j];
@@ -1081,9 +1069,10 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
         }
     };
     if constexpr (FAR) {
-        far_scalar_walk<true, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az, [&](int t) {
-            // packed rows {kl, m}, two pairs in turn (as the records of far_series)
-            ConstDoubles s = const_doubles(seg64 + (int64_t)t * kTile * 6);
+        // stretches of the near segments, in steps of four: with whole tiles a wave of 512 protons in the
+        // AG-CCT section had two or three of them
+        far_scalar_walk<true, PPL, NW>(fs, w, wave, lane, px, py, pz, ax, ay, az,
+                                       [&](const int* list, int n, int me, int all) {
             const auto terms = [&](const SegPair& p) {
 #pragma unroll
                 for (int i = 0; i < 12; i += 6) {
@@ -1099,17 +1088,27 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
                     }
                 }
             };
-            SegPair p = seg_pair(s), q;
+            constexpr int kCluster = kSmallTiles * kTile;
+            const int64_t fours = (int64_t)n * (kCluster / 4);
+            int k = (int)(fours * me / all) * 4;
+            const int end = (int)(fours * (me + 1) / all) * 4;
+            while (k < end) {
+                const int row = __builtin_amdgcn_readfirstlane(list[k / kCluster]) * kCluster + k % kCluster;
+                const int stop = end < (k / kCluster + 1) * kCluster ? end : (k / kCluster + 1) * kCluster;
+                // packed rows {kl, m}, two pairs in turn
+                ConstDoubles s = const_doubles(seg64 + (int64_t)row * 6);
+                SegPair p = seg_pair(s), q;
 #pragma unroll 1
-            for (int k = 0; k < kTile; k += 4, s += 24) {
-                loads_done();
-                q = seg_pair(s + 12);
-                __builtin_amdgcn_sched_barrier(0);
-                terms(p);
-                loads_done();
-                p = seg_pair(s + 24);  // past the last tile: kFarPad rows follow the array
-                __builtin_amdgcn_sched_barrier(0);
-                terms(q);
+                for (; k < stop; k += 4, s += 24) {
+                    loads_done();
+                    q = seg_pair(s + 12);
+                    __builtin_amdgcn_sched_barrier(0);
+                    terms(p);
+                    loads_done();
+                    p = seg_pair(s + 24);  // past the last tile: four rows follow the array
+                    __builtin_amdgcn_sched_barrier(0);
+                    terms(q);
+                }
             }
         });
     } else {
@@ -1161,73 +1160,53 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1
     const float4* src = reinterpret_cast<const float4*>(seg64);
     static_assert(NS * SEGS == kWG, "one segment per thread and staging round");
     const int st = (int)threadIdx.x / SEGS, sk = (int)threadIdx.x % SEGS;
-    // one round: every stream sums its own tile; tload: the tile this thread stages, tsum: the one
-    // of its stream (-1: none)
-    const auto tiles = [&](int tload, int tsum) {
-#pragma unroll 1
-        for (int h = 0; h < PARTS; ++h) {
-            float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0, v2 = v0, v3 = v0;  // absent tiles: not read
-            if (tload >= 0) {
-                if constexpr (FAR) {  // packed rows
-                    const float4* g = src + ((int64_t)tload * kTile + h * SEGS + sk) * 3;
-                    v0 = g[0];
-                    v1 = g[1];
-                    v2 = g[2];
-                } else {
-                    const float4* g = src + (int64_t)tload * ROW + (h * SEGS + sk) * 4;
-                    v0 = g[0];  // kl.x, kl.y
-                    v1 = g[1];  // kl.z, pad
-                    v2 = g[2];  // m.x, m.y
-                    v3 = g[3];  // m.z, pad
-                }
-            }
-            lds[st][3 * sk] = v0;
-            lds[st][3 * sk + 1] = FAR ? v1 : make_float4(v1.x, v1.y, v2.x, v2.y);
-            lds[st][3 * sk + 2] = FAR ? v2 : make_float4(v2.z, v2.w, v3.x, v3.y);
-            __syncthreads();
-            if (tsum >= 0) {  // uniform within a lane group
-                const double2* r = reinterpret_cast<const double2*>(lds[stream]);
+    // the first n rows staged for this lane group's stream
+    const auto sum = [&](int n) {
+        const double2* r = reinterpret_cast<const double2*>(lds[stream]);
 #pragma unroll CCTAMD_F64G_UNROLL
-                for (int k = 0; k < SEGS; ++k) {
-                    const double2 k01 = r[3 * k], k2m0 = r[3 * k + 1], m12 = r[3 * k + 2];
+        for (int k = 0; k < n; ++k) {
+            const double2 k01 = r[3 * k], k2m0 = r[3 * k + 1], m12 = r[3 * k + 2];
 #pragma unroll
-                    for (int j = 0; j < PL; ++j) {
-                        const double rx = px[j] - k2m0.y, ry = py[j] - m12.x, rz = pz[j] - m12.y;
-                        const double r2 = rx * rx + ry * ry + rz * rz;
-                        const double inv = rsqrt_f64(r2);
-                        const double inv3 = inv * inv * inv;
-                        ax[j] += (k01.y * rz - k2m0.x * ry) * inv3;
-                        ay[j] += (k2m0.x * rx - k01.x * rz) * inv3;
-                        az[j] += (k01.x * ry - k01.y * rx) * inv3;
-                    }
-                }
+            for (int j = 0; j < PL; ++j) {
+                const double rx = px[j] - k2m0.y, ry = py[j] - m12.x, rz = pz[j] - m12.y;
+                const double r2 = rx * rx + ry * ry + rz * rz;
+                const double inv = rsqrt_f64(r2);
+                const double inv3 = inv * inv * inv;
+                ax[j] += (k01.y * rz - k2m0.x * ry) * inv3;
+                ay[j] += (k2m0.x * rx - k01.x * rz) * inv3;
+                az[j] += (k01.x * ry - k01.y * rx) * inv3;
             }
-            __syncthreads();
         }
     };
     if constexpr (FAR) {
         __shared__ FarLists<kWavesPerWG> L;
         const Ball ball = block_ball<PL>(px, py, pz);
         for (int base = 0; base * kParts < w.tile_count; base += FarLists<kWavesPerWG>::kRound) {
-            far_lists<true, kWavesPerWG>(L, fs, w, ball, base, wave, lane);
-            const int ntile = __builtin_amdgcn_readfirstlane(L.nnear) * kSmallTiles;
-            const auto near = [&](int t) {
-                return t < ntile ? L.near[t / kSmallTiles] * kSmallTiles + t % kSmallTiles : -1;
-            };
-            for (int t = w.chunk * NS; t < ntile; t += w.nchunk * NS) tiles(near(t + st), near(t + stream));
-            // the 16-lane rows of the workgroup share a series (groups of 8 lanes: the first of a row
-            // takes its sum), or those of a wave where there are many; a share per wave as in
-            // far_scalar_walk measured up to 8 % slower here
-            const int me = w.chunk * kWavesPerWG + __builtin_amdgcn_readfirstlane(wave), all = w.nchunk * kWavesPerWG;
-            const int nfar = __builtin_amdgcn_readfirstlane(L.nfar);
-            const bool shared = nfar < kFarShared * all;
-            const int from = shared ? w.nchunk - 1 - w.chunk : all - 1 - me, by = shared ? w.nchunk : all;
-            const int row = shared ? (int)threadIdx.x / 16 : lane / 16, rows = shared ? kWG / 16 : kWave / 16;
+            const int uwave = __builtin_amdgcn_readfirstlane(wave);
+            const FarCounts n = far_lists<true, 4, kWavesPerWG>(L, fs, w, ball, base, uwave, lane);
+            // a stretch of the near segments (packed rows {kl, m}), every stream with as many of them
+            constexpr int kCluster = kSmallTiles * kTile;
+            const int64_t units = (int64_t)n.near * (kCluster / NS);
+            const int end = (int)(units * (w.chunk + 1) / w.nchunk) * NS;
+            for (int k0 = (int)(units * w.chunk / w.nchunk) * NS; k0 < end; k0 += kWG) {
+                const int k = k0 + (int)threadIdx.x;
+                if (k < end) {
+                    const float4* g = src + ((int64_t)L.near[k / kCluster] * kCluster + k % kCluster) * 3;
+                    const float4 v0 = g[0], v1 = g[1], v2 = g[2];
+                    float4* to = &lds[threadIdx.x % NS][3 * (threadIdx.x / NS)];
+                    to[0] = v0;
+                    to[1] = v1;
+                    to[2] = v2;
+                }
+                __syncthreads();
+                sum((end - k0 < kWG ? end - k0 : kWG) / NS);
+                __syncthreads();
+            }
+            // the four rows of lanes share a series (groups of 8 lanes: the first of a row takes its sum)
             double fx[PL], fy[PL], fz[PL];
 #pragma unroll
             for (int j = 0; j < PL; ++j) fx[j] = fy[j] = fz[j] = 0.0;
-            for (int e = from; e < nfar; e += by)
-                far_entry<kFarQ64, kWavesPerWG, PL>(L, fs, e, row, 2 * rows - 1 - row, 2 * rows, px, py, pz, fx, fy, fz);
+            far_share<kFarQ64, 4>(L, n, fs, uwave * w.nchunk + w.chunk, w.nchunk * kWavesPerWG, lane, px, py, pz, fx, fy, fz);
             const bool mine = LG >= 16 || (lane & 8) == 0;
 #pragma unroll
             for (int j = 0; j < PL; ++j) {
@@ -1239,8 +1218,25 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1
         }
     } else {
         const int tend = w.tile_start + w.tile_count;
-        for (int t0 = w.tile_start; t0 < tend; t0 += NS)
-            tiles(t0 + st < tend ? t0 + st : -1, t0 + stream < tend ? t0 + stream : -1);
+        for (int t0 = w.tile_start; t0 < tend; t0 += NS) {
+#pragma unroll 1
+            for (int h = 0; h < PARTS; ++h) {
+                float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0, v2 = v0, v3 = v0;  // absent tiles: not read
+                if (t0 + st < tend) {
+                    const float4* g = src + (int64_t)(t0 + st) * ROW + (h * SEGS + sk) * 4;
+                    v0 = g[0];  // kl.x, kl.y
+                    v1 = g[1];  // kl.z, pad
+                    v2 = g[2];  // m.x, m.y
+                    v3 = g[3];  // m.z, pad
+                }
+                lds[st][3 * sk] = v0;
+                lds[st][3 * sk + 1] = make_float4(v1.x, v1.y, v2.x, v2.y);
+                lds[st][3 * sk + 2] = make_float4(v2.z, v2.w, v3.x, v3.y);
+                __syncthreads();
+                if (t0 + stream < tend) sum(SEGS);  // uniform within a lane group
+                __syncthreads();
+            }
+        }
     }
 #pragma unroll
     for (int j = 0; j < PL; ++j) {

@@ -316,7 +316,7 @@ __device__ inline void analytic_fields(int64_t d, const double* __restrict__ qs,
 struct FarSet {
     const double *geo, *geo_large;    // [C][kFarGeo] small clusters, [C / 4][kFarGeo] large ones
     const double *coef, *coef_large;  // [C][far_records(Q)][kFarRec], [C / 4][far_records(Q)][kFarRec]
-    const int32_t* tiles;             // [C][kSmall * kNodeTiles] tile of each place, -1 for none (FP32 path); NULL:
+    const int32_t* tiles;             // [C][kSmallTiles] tile of each place, -1 for none (FP32 path); NULL:
                                       // places are tiles of the packed rows passed beside this set (FP64 path)
 };
 

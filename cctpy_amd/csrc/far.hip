@@ -683,7 +683,8 @@ int64_t cctamd_far_plan(int64_t ndesign, const int64_t* design_ntile, const int6
         // tile (what an item deals in)
         int64_t nc = nb > 0 ? std::max<int64_t>(1, ns * target_items / std::max<int64_t>(total, 1)) : 0;
         nc = std::min(nc, std::max<int64_t>(design_ntile[d], nb > 0 ? 1 : 0));
-        if (nc > kXcds) nc -= nc % kXcds;  // items that read the same rows share an XCD (as in cctamd_plan)
+        // the blocks' items that read the same rows share an XCD (as in cctamd_plan)
+        if (nb > 1 && nc > kXcds) nc -= nc % kXcds;
         if (work) {
             if (!design_cluster_off || !design_pt_off || !design_wbase || !design_nchunk) return CCTAMD_EINVAL;
             if (nc > 0x7fffffff) return CCTAMD_ERANGE;

@@ -114,114 +114,149 @@ __device__ __forceinline__ Ball block_ball(const double (&px)[PL], const double 
     return b;
 }
 
-// Order of the series that serves a cluster for a block, 0 if the cluster is too close (its
-// segments are then summed one by one).  Every wave and workgroup of a block gets the same
-// answer: the same operations on the same values, each rounded by itself.
+// Cost of a series in quarters of a block of four terms, for dealing it out.  A wave of one point
+// set takes row after row (LR = 1), one whose four rows of lanes hold the same points takes four
+// rows m at a time (LR = 4), a unit either way.  A unit's start: the blocks of those before it, a
+// row's own start and end (kFarRowCost each) and what a series needs before its first row.
+constexpr int kFarRowCost = 3, kFarSeriesCost = 12;
+template <int LR>
+__host__ __device__ constexpr int far_units(int N) { return LR == 1 ? N + 1 : (N >> 2) + 1; }
+template <int LR>
+__host__ __device__ constexpr int far_unit_blocks(int N, int u) {
+    return LR == 1 ? (N - u + 4) >> 2 : (N >> 2) - u + 1;
+}
+__host__ __device__ constexpr int far_blocks_upto(int l) {  // sum of ceil(k / 4) over k = 1 .. l
+    return ((l >> 2) + 1) * (2 * (l >> 2) + (l & 3));
+}
+template <int LR>
+__host__ __device__ constexpr int far_unit_start(int N, int u) {  // 0 for u = 0
+    const int blocks = LR == 1 ? far_blocks_upto(N + 1) - far_blocks_upto(N + 1 - u)
+                               : u * far_units<4>(N) - u * (u - 1) / 2;
+    return u == 0 ? 0 : kFarSeriesCost + kFarRowCost * u + 4 * blocks;
+}
+// Order and cost of a series in one value, as the lists carry them about.
+template <int LR>
+__host__ __device__ constexpr int far_pack(int N) {
+    return far_unit_start<LR>(N, far_units<LR>(N)) << 5 | N;
+}
+
+// Order and cost (far_pack) of the series that serves a cluster for a block, 0 if the cluster is too
+// close (its segments are then summed one by one).  Every wave and workgroup of a block gets the
+// same answer: the same operations on the same values, each rounded by itself.
 #pragma clang fp contract(off)
-template <bool F64>
+template <bool F64, int LR>
 __device__ __forceinline__ int far_order(const double* __restrict__ geo, const Ball& b) {
     const double dx = geo[0] - b.x, dy = geo[1] - b.y, dz = geo[2] - b.z;
-    const double ratio = (__builtin_sqrt(dx * dx + dy * dy + dz * dz) - b.r) * geo[3];
+    const float d = __builtin_amdgcn_sqrtf((float)(dx * dx + dy * dy + dz * dz));
+    const float ratio = (d - (float)b.r) * (float)geo[3];
     using T = FarOrders<F64>;
     int n = 0;
 #pragma unroll
-    for (int k = 0; k < T::n; ++k) n = ratio >= T::ratio[k] ? T::order[k] : n;
+    for (int k = 0; k < T::n; ++k) n = ratio >= (float)T::ratio[k] ? far_pack<LR>(T::order[k]) : n;
     return n;
 }
 #pragma clang fp contract(fast)
 
-// Work lists of a workgroup for its point block, in LDS: the small clusters whose segments are
-// summed one by one, and the clusters, small or large, that act through their series.  Every
-// workgroup of a block makes the same lists; each takes its share of them (the tiles of the
-// near clusters and the series are dealt out over all waves of the block's work items, so
-// that the near part, a few percent of the segments, does not fall to a few of them).
-template <int NW>
-struct FarLists {
-    static constexpr int kRound = kWave * NW;  // large clusters per round
-    int near[kParts * kRound];                 // small cluster
-    int far[kParts * kRound];                  // cluster << 6 | order << 1 | large
-    unsigned short close[kRound];              // large clusters of the round that are not far
-    alignas(16) int count[2][kParts * NW];
-    int nnear, nfar;
-};
+// Sum of v over the lanes of the wave up to and with this one: within the 16-lane rows, then the
+// rows' last lanes into the next rows.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
 
 __device__ __forceinline__ int lane_rank(uint64_t mask) {  // set bits below this lane
     return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
 }
 
+// Work lists of a workgroup for its point block, in LDS: the small clusters whose segments are
+// summed one by one, and the clusters, small or large, that act through their series.  Every
+// workgroup of a block makes the same lists; each takes its share of them (the segments of the
+// near clusters and the rows of the series are dealt out over all waves of the block's work
+// items, so that neither falls to a few of them).
+template <int NW>
+struct FarLists {
+    static constexpr int kRound = kWave * NW;  // large clusters per round
+    int near[kParts * kRound];                 // small cluster
+    int far[kParts * kRound];                  // cluster << 6 | order << 1 | large
+    int start[kParts * kRound];                // cost of the series before this one in the list
+    unsigned short close[kRound];              // large clusters of the round that are not far
+    int tally[2][(kParts + 1) * NW];           // of a wave: series | other clusters << 16, cost of the series
+};
+
+struct FarCounts {
+    int near, far, cost;
+};
+
 // Lists of the large clusters [base, base + kRound) of a work item's design (w.tile_start: its
-// first small cluster, w.tile_count: its small clusters).
-template <bool F64, int NW>
-__device__ __forceinline__ void far_lists(FarLists<NW>& L, const FarSet& fs, const Work& w, const Ball& ball, int base,
-                                          int wave, int lane) {
-    const int nlarge = (w.tile_count + kParts - 1) / kParts;
-    // sum of the counts of round r, all and those of the waves before this one
-    const auto add = [&](int which, int r, int& mine, int& all) {
-        const int4* c = reinterpret_cast<const int4*>(&L.count[which][r * NW]);
-#pragma unroll
-        for (int i = 0; i < NW / 4; ++i) {
-            const int4 v = c[i];
-            mine += (4 * i < wave ? v.x : 0) + (4 * i + 1 < wave ? v.y : 0) + (4 * i + 2 < wave ? v.z : 0) +
-                    (4 * i + 3 < wave ? v.w : 0);
-            all += v.x + v.y + v.z + v.w;
+// first small cluster, w.tile_count: its small clusters).  All waves of all workgroups run through
+// this at once, so its instructions count: with FP64 roots, orders and costs of four rounds kept in
+// registers and every tally added up by every lane it took 2.5 us, a tenth of a stage of the AG-CCT
+// section; now 1.5.
+template <bool F64, int LR, int NW>
+__device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs, const Work& w, const Ball& ball,
+                                               int base, int wave, int lane) {
+    FarCounts n{0, 0, 0};
+    // a cluster per lane: it joins the series, or put(its place among the others) takes it
+    const auto round = [&](int slot, bool valid, int cl, const double* geo, int large, auto&& put) {
+        int order = 0, upto = 0;
+        uint64_t far = 0, other = 0;
+        if (__any(valid)) {  // wave-uniform
+            order = valid ? far_order<F64, LR>(geo + (int64_t)cl * kFarGeo, ball) : 0;
+            far = __ballot(order != 0);
+            other = __ballot(valid && order == 0);
+            upto = wave_scan(order >> 5);
         }
+        const int own = __popcll(far) | __popcll(other) << 16;
+        if (lane == kWave - 1) {
+            L.tally[0][slot * NW + wave] = own;
+            L.tally[1][slot * NW + wave] = upto;
+        }
+        __syncthreads();
+        // sums up to each wave in lanes 0 .. NW - 1
+        int count = L.tally[0][slot * NW + (lane & (NW - 1))], cost = L.tally[1][slot * NW + (lane & (NW - 1))];
+        // one block, with the two wait states between a write and its read by lane moves written out
+#define CCTAMD_SCAN(N)                                                                           \
+    "s_nop 0\n\t"                                                                                \
+    "v_add_u32_dpp %0, %0, %0 row_shr:" #N " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"         \
+    "v_add_u32_dpp %1, %1, %1 row_shr:" #N " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+        asm volatile("s_nop 0\n\t" CCTAMD_SCAN(1) CCTAMD_SCAN(2) CCTAMD_SCAN(4) "s_nop 1" : "+v"(count), "+v"(cost));
+#undef CCTAMD_SCAN
+        static_assert(NW <= 8, "tallies of a round within a scan of eight lanes");
+        const int before = __builtin_amdgcn_readlane(count, wave) - own;
+        if (order != 0) {
+            const int at = n.far + (before & 0xffff) + lane_rank(far);
+            L.far[at] = cl << 6 | (order & 31) << 1 | large;
+            L.start[at] = n.cost + __builtin_amdgcn_readlane(cost, wave) - __builtin_amdgcn_readlane(upto, kWave - 1) +
+                          upto - (order >> 5);
+        } else if (valid) {
+            put(n.near + (before >> 16) + lane_rank(other));
+        }
+        const int all = __builtin_amdgcn_readlane(count, NW - 1);
+        n.far += all & 0xffff;
+        n.near += all >> 16;
+        n.cost += __builtin_amdgcn_readlane(cost, NW - 1);
     };
-    int nfar, nclose;
-    {
-        const int l = base + wave * kWave + lane;
-        const bool valid = l < nlarge;
-        const int cl = w.tile_start / kParts + (valid ? l : 0);
-        const int order = far_order<F64>(fs.geo_large + (int64_t)cl * kFarGeo, ball);
-        const uint64_t far = __ballot(valid && order != 0), close = __ballot(valid && order == 0);
-        if (lane == 0) {
-            L.count[0][wave] = __popcll(far);
-            L.count[1][wave] = __popcll(close);
-        }
-        __syncthreads();
-        int f = 0, c = 0;
-        nfar = nclose = 0;
-        add(0, 0, f, nfar);
-        add(1, 0, c, nclose);
-        if (valid && order != 0) L.far[f + lane_rank(far)] = cl << 6 | order << 1 | 1;
-        if (valid && order == 0) L.close[c + lane_rank(close)] = (unsigned short)(l - base);
-        __syncthreads();
-    }
-    int order[kParts], cl[kParts];
-    uint64_t far[kParts], near[kParts];
-    const int rounds = (kParts * nclose + FarLists<NW>::kRound - 1) / FarLists<NW>::kRound;
-#pragma unroll
-    for (int r = 0; r < kParts; ++r) {
-        far[r] = near[r] = 0;
-        if (r >= rounds) continue;
+    const int nlarge = (w.tile_count + kParts - 1) / kParts;
+    const int l = base + wave * kWave + lane;
+    round(0, l < nlarge, w.tile_start / kParts + l, fs.geo_large, 1,
+          [&](int at) { L.close[at] = (unsigned short)(l - base); });
+    __syncthreads();
+    const int parts = kParts * n.near;
+    n.near = 0;
+#pragma unroll 1
+    for (int r = 0; r * FarLists<NW>::kRound < parts; ++r) {
         const int j = (r * NW + wave) * kWave + lane;
-        const int part = j < kParts * nclose ? (base + L.close[j / kParts]) * kParts + j % kParts : 0;
-        const bool valid = j < kParts * nclose && part < w.tile_count;
-        cl[r] = w.tile_start + (valid ? part : 0);
-        order[r] = far_order<F64>(fs.geo + (int64_t)cl[r] * kFarGeo, ball);
-        far[r] = __ballot(valid && order[r] != 0);
-        near[r] = __ballot(valid && order[r] == 0);
-        if (lane == 0) {
-            L.count[0][r * NW + wave] = __popcll(far[r]);
-            L.count[1][r * NW + wave] = __popcll(near[r]);
-        }
+        const int part = j < parts ? (base + L.close[j / kParts]) * kParts + j % kParts : w.tile_count;
+        const int cl = w.tile_start + part;
+        round(r + 1, part < w.tile_count, cl, fs.geo, 0, [&](int at) { L.near[at] = cl; });
     }
     __syncthreads();
-    int nnear = 0;
-    const uint64_t me = 1ull << lane;
-#pragma unroll
-    for (int r = 0; r < kParts; ++r) {
-        if (r >= rounds) continue;
-        int f = nfar, n = nnear;
-        add(0, r, f, nfar);
-        add(1, r, n, nnear);
-        if (far[r] & me) L.far[f + lane_rank(far[r])] = cl[r] << 6 | order[r] << 1;
-        if (near[r] & me) L.near[n + lane_rank(near[r])] = cl[r];
-    }
-    if (wave == 0 && lane == 0) {
-        L.nnear = nnear;
-        L.nfar = nfar;
-    }
-    __syncthreads();
+    return n;
 }
 
 // Read-only memory: wave-uniform addresses are read by scalar loads.
@@ -241,8 +276,6 @@ __device__ __forceinline__ ConstDoubles apart(ConstDoubles p) {
     asm volatile("" : "+s"(p));
     return p;
 }
-
-constexpr int kFarPad = 16;  // records that may be read past the last one
 
 // One (n, m) of the series at one point.  Record I (0 or 1) of the two that a 16-lane row
 // holds, lane i with double i of them; each coefficient reaches the row's lanes through the
@@ -268,134 +301,176 @@ __device__ __forceinline__ void far_term(double rec, double Z, double rho, doubl
     t = tn;
 }
 
-// Adds the series of a cluster (wave-uniform) at the lane's PL points: rows m = a0, a0 + step, ...
-// and b0, b0 + step, ... up to order N (a0, b0 < step, step a power of two), which may differ
-// between the 16-lane rows of the wave.  Waves or rows of lanes share a cluster by their a0
-// and b0; pairing row w with row step - 1 - w gives all of them about as many terms (row m has
-// N - m + 1).  9 FP64 instructions per (n, m) and point.
+// Adds units u0 .. u1 - 1 of the series of a cluster (wave-uniform) at the lane's PL points: rows m
+// of the unit's number (LR = 1), or row 4 u + i in the wave's row i of lanes (LR = 4).  9 FP64
+// instructions per (n, m) and point.
 // The coefficients of a cluster (up to 35 KB) are read once per block and stage, from L2 at
 // best, and a term uses them up quickly: with scalar loads, which a wave can only wait for all
 // at once, the AG-CCT section's FP64 stage spent two thirds of its time waiting.  Vector loads
-// of 16 doubles (two records) return in order, and three pairs of them are on their way.
-template <int Q, int PL>
-__device__ __forceinline__ void far_series(ConstDoubles geo, const double* __restrict__ coef, int N, int a0, int b0,
-                                           int step, const double (&px)[PL], const double (&py)[PL],
-                                           const double (&pz)[PL], double (&ax)[PL], double (&ay)[PL],
-                                           double (&az)[PL]) {
-    double X[PL], Y[PL], Z[PL], rho[PL], ri[PL], ac[PL], as[PL], bc[PL], bs[PL], sc[PL], ss[PL];
-    const double gx = geo[0], gy = geo[1], gz = geo[2], inv = geo[3];
-    coef += threadIdx.x & 15;
-#pragma unroll
-    for (int j = 0; j < PL; ++j) {
-        const double x = (px[j] - gx) * inv, y = (py[j] - gy) * inv, z = (pz[j] - gz) * inv;
-        const double r2 = x * x + y * y + z * z;
-        const double h = __builtin_amdgcn_rsq(r2);  // refined as in rsqrt_f64
-        const double e = __builtin_fma(-r2 * h, h, 1.0);
-        ri[j] = __builtin_fma(h * e, __builtin_fma(e, 0.375, 0.5), h);
-        rho[j] = ri[j] * ri[j];
-        X[j] = x * rho[j];
-        Y[j] = y * rho[j];
-        Z[j] = z * rho[j];
-        ac[j] = bc[j] = 1.0;
-        as[j] = bs[j] = 0.0;
-        sc[j] = X[j];
-        ss[j] = Y[j];
-    }
-#pragma unroll 1
-    for (int bit = 1; bit < step; bit <<= 1) {  // (X + iY)^a0, ^b0 and, at the end, ^step
-        const bool ua = (a0 & bit) != 0, ub = (b0 & bit) != 0;
+// of 16 doubles (two records) return in order; those of the two blocks after the one in use are on
+// their way, across the ends of rows too.
+template <int Q, int PL, int LR>
+__device__ __forceinline__ void far_rows(ConstDoubles geo, const double* __restrict__ coef, int N, int u0, int u1,
+                                         const double (&px)[PL], const double (&py)[PL], const double (&pz)[PL],
+                                         double (&ax)[PL], double (&ay)[PL], double (&az)[PL]) {
+    const int lrow = LR == 1 ? 0 : (int)(threadIdx.x >> 4) & 3;
+    const double* lanes = coef + (threadIdx.x & 15);
+    const auto unit = [&](int u) {  // this lane's first record of a unit
+        return LR == 1 ? lanes + far_row(Q, u) * kFarRec
+                       : lanes + (far_row(Q, 4 * u) + lrow * 4 * (Q - u)) * kFarRec;
+    };
+    // loads of the next block in the order of use; past the last one it is loaded again
+    int fu = u0, fk = far_unit_blocks<LR>(N, u0);
+    const double* next = unit(u0);
+    const auto fetch = [&](double& p, double& q) {
+        p = next[0];
+        q = next[16];
+        if (--fk > 0) {
+            next += 32;
+        } else if (fu + 1 < u1) {
+            next = unit(++fu);
+            fk = far_unit_blocks<LR>(N, fu);
+        }
+    };
+    double a0, a1, b0, b1, d0, d1;
+    fetch(a0, a1);
+    fetch(b0, b1);
+
+    double Z[PL], rho[PL], ri[PL], wc[PL], ws[PL], sc[PL], ss[PL];
+    {
+        const double gx = geo[0], gy = geo[1], gz = geo[2], inv = geo[3];
+        double bc[PL], bs[PL];
 #pragma unroll
         for (int j = 0; j < PL; ++j) {
-            const double c = sc[j], s = ss[j];
-            if (ua) {
-                const double t = ac[j] * c - as[j] * s;
-                as[j] = ac[j] * s + as[j] * c;
-                ac[j] = t;
+            const double x = (px[j] - gx) * inv, y = (py[j] - gy) * inv, z = (pz[j] - gz) * inv;
+            const double r2 = x * x + y * y + z * z;
+            const double h = __builtin_amdgcn_rsq(r2);  // refined as in rsqrt_f64
+            const double e = __builtin_fma(-r2 * h, h, 1.0);
+            ri[j] = __builtin_fma(h * e, __builtin_fma(e, 0.375, 0.5), h);
+            rho[j] = ri[j] * ri[j];
+            Z[j] = z * rho[j];
+            sc[j] = bc[j] = x * rho[j];
+            ss[j] = bs[j] = y * rho[j];
+            wc[j] = 1.0;
+            ws[j] = 0.0;
+        }
+        const auto times = [](double& c, double& s, double bc, double bs) {
+            const double t = c * bc - s * bs;
+            s = c * bs + s * bc;
+            c = t;
+        };
+        if constexpr (LR == 4) {  // (X + iY)^lrow, and the step (X + iY)^4
+#pragma unroll
+            for (int j = 0; j < PL; ++j) {
+                double c2 = sc[j], s2 = ss[j];
+                times(c2, s2, sc[j], ss[j]);
+                wc[j] = lrow & 1 ? sc[j] : 1.0;
+                ws[j] = lrow & 1 ? ss[j] : 0.0;
+                double c = wc[j], s = ws[j];
+                times(c, s, c2, s2);
+                wc[j] = lrow & 2 ? c : wc[j];
+                ws[j] = lrow & 2 ? s : ws[j];
+                times(c2, s2, c2, s2);
+                sc[j] = bc[j] = c2;
+                ss[j] = bs[j] = s2;
             }
-            if (ub) {
-                const double t = bc[j] * c - bs[j] * s;
-                bs[j] = bc[j] * s + bs[j] * c;
-                bc[j] = t;
+        }
+#pragma unroll 1
+        for (int bits = u0; bits; bits >>= 1) {  // times the step's power u0
+            if (bits & 1) {
+#pragma unroll
+                for (int j = 0; j < PL; ++j) times(wc[j], ws[j], bc[j], bs[j]);
             }
-            sc[j] = c * c - s * s;
-            ss[j] = 2.0 * c * s;
+#pragma unroll
+            for (int j = 0; j < PL; ++j) {
+                const double c = bc[j], s = bs[j];
+                bc[j] = c * c - s * s;
+                bs[j] = 2.0 * c * s;
+            }
         }
     }
-    const auto row = [&](int m, const double (&wc)[PL], const double (&ws)[PL]) {
-        const double* rec = coef + (int64_t)far_row(Q, m) * kFarRec;
-        double t[PL], u[PL], c0[PL], c1[PL], c2[PL], s0[PL], s1[PL], s2[PL];
+    double t[PL], u[PL], c0[PL], c1[PL], c2[PL], s0[PL], s1[PL], s2[PL];
+    const auto begin = [&]() {
 #pragma unroll
         for (int j = 0; j < PL; ++j) {
             t[j] = ri[j];
             u[j] = c0[j] = c1[j] = c2[j] = s0[j] = s1[j] = s2[j] = 0.0;
         }
-        const auto four = [&](double p, double q) {  // four records, two per register
+    };
+    begin();
+    int at = u0, left = far_unit_blocks<LR>(N, u0);
+    const auto block = [&](double p, double q) {  // four records, two per register; true after the last row
 #pragma unroll
-            for (int j = 0; j < PL; ++j)
-                far_term<0>(p, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
+        for (int j = 0; j < PL; ++j)
+            far_term<0>(p, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
 #pragma unroll
-            for (int j = 0; j < PL; ++j)
-                far_term<1>(p, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
+        for (int j = 0; j < PL; ++j)
+            far_term<1>(p, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
 #pragma unroll
-            for (int j = 0; j < PL; ++j)
-                far_term<0>(q, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
+        for (int j = 0; j < PL; ++j)
+            far_term<0>(q, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
 #pragma unroll
-            for (int j = 0; j < PL; ++j)
-                far_term<1>(q, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
-        };
-        // past the row's end the next row's records are loaded and not used (kFarPad follow the array)
-        double p0 = rec[0], p1 = rec[16], q0 = rec[32], q1 = rec[48], r0, r1;
-#pragma unroll 1
-        for (int n = m;;) {
-            r0 = rec[64];
-            r1 = rec[80];
-            four(p0, p1);
-            if ((n += 4) > N) break;
-            p0 = rec[96];
-            p1 = rec[112];
-            four(q0, q1);
-            if ((n += 4) > N) break;
-            q0 = rec[128];
-            q1 = rec[144];
-            four(r0, r1);
-            if ((n += 4) > N) break;
-            rec += 96;
-        }
+        for (int j = 0; j < PL; ++j)
+            far_term<1>(q, Z[j], rho[j], t[j], u[j], c0[j], c1[j], c2[j], s0[j], s1[j], s2[j]);
+        if (--left > 0) return false;
 #pragma unroll
         for (int j = 0; j < PL; ++j) {
             ax[j] = __builtin_fma(wc[j], c0[j], __builtin_fma(ws[j], s0[j], ax[j]));
             ay[j] = __builtin_fma(wc[j], c1[j], __builtin_fma(ws[j], s1[j], ay[j]));
             az[j] = __builtin_fma(wc[j], c2[j], __builtin_fma(ws[j], s2[j], az[j]));
-        }
-    };
-    const auto ahead = [&](double (&wc)[PL], double (&ws)[PL]) {
-#pragma unroll
-        for (int j = 0; j < PL; ++j) {
-            const double t = wc[j] * sc[j] - ws[j] * ss[j];
+            const double c = wc[j] * sc[j] - ws[j] * ss[j];
             ws[j] = wc[j] * ss[j] + ws[j] * sc[j];
-            wc[j] = t;
+            wc[j] = c;
         }
+        if (++at == u1) return true;
+        left = far_unit_blocks<LR>(N, at);
+        begin();
+        return false;
     };
 #pragma unroll 1
-    for (int m = a0, m2 = b0; m <= N || m2 <= N; m += step, m2 += step) {
-        if (m <= N) row(m, ac, as);
-        if (m2 <= N) row(m2, bc, bs);
-        ahead(ac, as);
-        ahead(bc, bs);
+    for (;;) {
+        fetch(d0, d1);
+        if (block(a0, a1)) break;
+        fetch(a0, a1);
+        if (block(b0, b1)) break;
+        fetch(b0, b1);
+        if (block(d0, d1)) break;
     }
 }
 
-// The series of entry e of a block's list.
-template <int Q, int NW, int PL>
-__device__ __forceinline__ void far_entry(const FarLists<NW>& L, const FarSet& fs, int e, int a0, int b0, int step,
+// Share `me` of `all` equal shares of a block's series, by cost: a wave takes a stretch of the
+// rows of the whole list, so that every wave of the block has as much to do to within a row, and
+// starts few series (those of its stretch).  Dealt out by series, or by eighths of one where there
+// were few, waves had two or three pieces of very different lengths, and each piece began with
+// powers of X + iY: 4,096 protons in the gantry spent 37 us of a stage here, now 18; a stage of 512
+// in the AG-CCT section (FP64) took 49.8 us, now 44.5.
+template <int Q, int LR, int NW, int PL>
+__device__ __forceinline__ void far_share(const FarLists<NW>& L, const FarCounts& n, const FarSet& fs, int me, int all, int lane,
                                           const double (&px)[PL], const double (&py)[PL], const double (&pz)[PL],
                                           double (&ax)[PL], double (&ay)[PL], double (&az)[PL]) {
-    const int entry = __builtin_amdgcn_readfirstlane(L.far[e]);
-    const bool large = entry & 1;
-    const int64_t cl = entry >> 6;
-    far_series<Q, PL>(const_doubles((large ? fs.geo_large : fs.geo) + cl * kFarGeo),
-                      (large ? fs.coef_large : fs.coef) + cl * far_records(Q) * kFarRec, entry >> 1 & 31, a0, b0, step,
-                      px, py, pz, ax, ay, az);
+    const int nfar = n.far;
+    const int from = (int)((int64_t)n.cost * me / all), to = (int)((int64_t)n.cost * (me + 1) / all);
+    if (from == to) return;
+    int e = -1;  // the last series that starts at or before `from`
+    for (int k = 0; k < nfar; k += kWave) {
+        const bool before = k + lane < nfar && L.start[k + lane] <= from;
+        e += __popcll(__ballot(before));
+    }
+    for (; e < nfar; ++e) {
+        const int at = __builtin_amdgcn_readfirstlane(L.start[e]);
+        if (at >= to) break;
+        const int entry = __builtin_amdgcn_readfirstlane(L.far[e]);
+        const int N = entry >> 1 & 31;
+        const bool is = lane < far_units<LR>(N);
+        const int start = far_unit_start<LR>(N, lane);
+        const int u0 = __popcll(__ballot(is && start < from - at)), u1 = __popcll(__ballot(is && start < to - at));
+        if (u0 == u1) continue;
+        const bool large = entry & 1;
+        const int64_t cl = entry >> 6;
+        far_rows<Q, PL, LR>(const_doubles((large ? fs.geo_large : fs.geo) + cl * kFarGeo),
+                            (large ? fs.coef_large : fs.coef) + cl * far_records(Q) * kFarRec, N, u0, u1, px, py, pz,
+                            ax, ay, az);
+    }
 }
 
 }  // namespace cctamd_detail

@@ -44,7 +44,7 @@ _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # 158 / 45-60.  FP32: 2,048 protons in the CCT of 1,440 tiles (9.4e7, 23) 53 / 45-55, 400 in the gantry at
 # 60 (4.1e7, 31) 37 / 29, 64 in the section at 360 (1.2e7, 90) 18 / 18-23, 128 at 720 (4.7e7, 180) 37-40 /
 # 24-34, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 300.
-_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.6, share=11),
+_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.6, share=24),
         33: dict(pairs=4.0e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
 
 
@@ -166,7 +166,7 @@ class FarField:
         self.rows = empty(6 * (C * 512 + 4)) if precision == 64 else None
         self.tiles = empty(C * 16, torch.int32) if precision != 64 else None
         self.geo, self.geo_large = empty(8 * C), empty(2 * C)
-        self.coef, self.coef_large = empty(C * per + 128), empty(C // 4 * per + 128)
+        self.coef, self.coef_large = empty(C * per), empty(C // 4 * per)
         mom = empty(2 * C * per // 4 * 3)
         N.check(N.lib.cctamd_far_build(precision, _p(model.seg64), unit, _p(centre), _p(uo), _p(so), int(chunk_off[-1]),
                                        _p(co), model.ndesign, C, _p(perm), _p(self.rows), _p(self.tiles),
@@ -357,14 +357,18 @@ class DeviceModel:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
         npt = numpy.asarray(plan.design_npt, numpy.int64)
         pt_off = numpy.concatenate([[0], numpy.cumsum(npt)]).astype(numpy.int64)
-        # Work items: one per CU for a small beam in one design (its lists cost each item 5 us), more where
-        # there is more to deal out, up to two resident per CU; several designs differ in what their
-        # blocks need and balance over smaller items.  512 protons in the AG-CCT section: 256 items 60 us,
-        # 1,024 69 us; 24 designs x 32: 256 items 153 us, 1,440 84 us.
+        # Work items.  Designs alike: one or two per CU, as all their items take the same time and between
+        # the two some CUs have twice the work of others (512 protons in the AG-CCT section, FP32: 256 items 35.7
+        # us per stage, 320 42.4, 480 35.3, 512 33.9, 640 42.4, 1,024 44.3; 128 protons: 21.5, 25.1, 24.4, 24.4,
+        # 33.2; FP64 8 gantries x 80: 256 items 23.4, 448 26.6, 512 26.4, 640 33.2).  Designs that differ in what
+        # their blocks need balance over smaller items (24 designs x 32, FP32: 498 items 70, 754 59, 1,012 64).
+        tiles = -(-npt // points_per_block(plan.ppl)) * nt
         clusters = int((-(-npt // points_per_block(plan.ppl)) * -(-nt // 16)).sum())
         cus = cu_count()
-        target = min(max(clusters // 5, cus), 6 * cus) if self.ndesign > 1 else \
-            min(max(clusters // _FAR[precision]["share"], cus), 2 * cus)
+        if tiles.max() <= 1.05 * tiles.min():
+            target = cus if clusters <= _FAR[precision]["share"] * cus else 2 * cus
+        else:
+            target = min(max(clusters // 5, cus), 6 * cus)
         target = min(plan.nwork, target)
         while True:  # the caller's partial sums hold plan.nwork items (every point block has one)
             args = (self.ndesign, _np(nt), _np(npt), _np(far.cluster_off), _np(pt_off), plan.ppl)

@@ -196,8 +196,7 @@ int cctamd_track_rk4(int precision, int ppl, const void *seg, const double *tile
  *                             clusters (a multiple of 4 per design, C in all), chunk_off
  *                             int64[D+1] stretches of 16,384 units (the last one of a design
  *                             may be shorter).  Writes geo double[C][8], geo_large
- *                             double[C/4][8], coef and coef_large (allocated with 128 doubles more
- *                             than their clusters), and rows double[C*512 + 4][6] (precision 64:
+ *                             double[C/4][8], coef, coef_large, and rows double[C*512 + 4][6] (precision 64:
  *                             {kl, m} in cluster order, passed as `seg` when tracking) or
  *                             tiles int32[C*16] (precision 33); mom is scratch for 2 C clusters.
  *   cctamd_far_plan           work items as in cctamd_plan (host arrays), the tile range replaced

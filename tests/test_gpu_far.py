@@ -118,3 +118,25 @@ def test_far_field_of_a_map_matches_the_full_sum(monkeypatch):
         assert np.all(np.isfinite(out[0]))
         for d, (a, b) in enumerate(zip(*[np.split(o, np.cumsum(npt)[:-1], axis=1) for o in out])):
             assert np.max(np.abs(a - b)) <= 1e-13 * max(np.max(np.abs(b)), 1e-300), (ppl, d)
+
+@pytest.mark.parametrize("precision,ppl", [(64, 1), (64, 2), (64, -2), (64, -4), (33, 1), (33, 2), (33, -2)])
+def test_the_number_of_items_does_not_change_the_sum(precision, ppl, monkeypatch):
+    """The series' rows and the near segments dealt out to the waves of few items or of many (more waves
+    than rows in the designs of few tiles): the same terms, added up in another order.  The FP32 path
+    sums whole tiles, so its tile sums are the same too."""
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    npt = [3, 130, 2, 40, 1, 257]
+    model = engine.DeviceModel(_specs(), fp32=precision != 64)
+    state = _beam(npt)
+    results, items = [], []
+    for cus in (1, 3, 100, 1000):  # items per block from one to one per tile
+        monkeypatch.setattr(engine, "cu_count", lambda: cus)
+        model._plans.clear()
+        plan = model.plan(npt, ppl, 8192)
+        results.append(_track(model, plan, precision, state, 1, True))
+        items.append(plan.far[precision].nwork)
+    assert items == sorted(items) and items[-1] > 2 * items[0]
+    for r in results[1:]:
+        np.testing.assert_allclose(r[:3], results[0][:3], rtol=0, atol=1e-13)
+        v = np.linalg.norm(results[0][3:], axis=0)
+        assert (np.abs(r[3:] - results[0][3:]) <= 1e-13 * v).all()
