@@ -170,12 +170,12 @@ __device__ __forceinline__ void tile_terms_f64(const double* __restrict__ seg64,
                                                const double (&py)[NP], const double (&pz)[NP], double (&ax)[NP],
                                                double (&ay)[NP], double (&az)[NP]) {
     const double2* s = reinterpret_cast<const double2*>(seg64) + t * kTile * 4;
-    // one point at a time and no unrolling: this path is rare, and its registers count
+    // one point at a time and two segments: this path is rare, and its registers count
     // against the occupancy of the FP32 loop of the same kernel
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
         double bx = ax[j], by = ay[j], bz = az[j];
-#pragma unroll 1
+#pragma unroll 2
         for (int k = 0; k < kTile; ++k) {
             const double2 k01 = s[4 * k], k2_ = s[4 * k + 1], m01 = s[4 * k + 2], m2_ = s[4 * k + 3];
             const double rx = px[j] - m01.x, ry = py[j] - m01.y, rz = pz[j] - m2_.x;
@@ -254,14 +254,16 @@ constexpr double kFp64Tile = 1.5;
 // Occupancy (waves per SIMD) of the scalar-load Biot-Savart kernels without the
 // fused stage, which their fused variants (S >= 0) are held to: the stage
 // update at the end alone would otherwise set their register count (~120-160
-// VGPRs against 44 for k_bs_partial_f32k<1, 8>).  1 = no hint.
+// VGPRs against 58 for k_bs_partial_f32k<1, 8>).  1 = no hint.
 constexpr int kKindF32 = 0, kKindF32k = 1, kKindF64 = 2;
 constexpr int fused_waves(int kind, int ppl, int s, bool far = false) {
     // Far-field kernels: enough for two workgroups per CU (ppl 1, 2).  Held to 96 and 128 VGPRs they
     // spill one register at most; unheld, the 512-proton AG-CCT section's stage took 67 instead of
     // 58 us (FP32), one item per CU more.
     if (far) return ppl == 1 ? 5 : ppl == 2 ? 4 : 2;
-    if (s < 0) return 1;
+    // 84 VGPRs: the direct tiles in fours would take 100 (256 protons in the AG-CCT section 51.3 instead of
+    // 49.7 us per stage)
+    if (s < 0) return kind == kKindF32k && ppl == 2 ? 6 : 1;
     if (kind == kKindF32) return ppl == 1 ? 6 : 4;
     if (kind == kKindF32k) return ppl == 1 ? 8 : ppl == 2 ? 6 : 4;
     return ppl == 1 ? 8 : ppl == 2 ? 5 : 4;
@@ -631,7 +633,10 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
             return;
         }
         if (__any(near)) {  // wave-uniform: FP32 direct form
-#pragma unroll 1
+            // a wave waits for all its scalar loads at once: per segment, one by one, a direct tile took
+            // three times a K/C tile (64 protons in the single CCT, where most are direct: 10.1 us per stage, in
+            // fours 8.7; 64 in the AG-CCT section 25.7 and 23.3)
+#pragma unroll 4
             for (int k = 0; k < kTile; ++k) {
                 const float4 a = s[3 * k], b = s[3 * k + 1], c = s[3 * k + 2];
 #pragma unroll
