@@ -302,7 +302,7 @@ __device__ inline int* arrival_counters(const StageArgs& sa) { return (int*)(sa.
 // Y1 = Y0 + dt/2 k1, Y2 = Y0 + dt/2 k2, Y3 = Y0 + dt k3,
 // Y0 += dt/6 (((k1 + 2 k2) + 2 k3) + k4).
 // LEAN (the fused epilogue): the chunk sum first, with two loads in flight per
-// lane, and the particle's state loaded by lane 0 only after it, so that the
+// lane, and the particle's state loaded only after it, so that the
 // stage update needs few registers beside the Biot-Savart loop's.  Otherwise
 // every load is issued before the chunk sum (latency first, registers are
 // plentiful in k_rk4_stage).  Both forms compute the same values.
@@ -337,7 +337,6 @@ __device__ inline void rk4_stage_point(const StageArgs& sa, int64_t g) {
     };
     if (LEAN) {
         chunk_sum<2>(sl, b, sa.scratch);
-        if ((threadIdx.x & (kWave - 1)) != 0) return;
         load_state();
         if (sa.step >= ns) return;
     } else {
@@ -347,9 +346,9 @@ __device__ inline void rk4_stage_point(const StageArgs& sa, int64_t g) {
         load_state();
         chunk_sum(sl, b, sa.scratch);
         if (sa.step >= ns) return;
-        if ((threadIdx.x & (kWave - 1)) != 0) return;
     }
     analytic_fields(an, sa.qs, p, b);
+    if ((threadIdx.x & (kWave - 1)) != 0) return;
     if (sa.tape) {  // stage point, velocity and field for the adjoint
         double* t = sa.tape + S * 9 * P;
         for (int c = 0; c < 3; ++c) {
@@ -1284,8 +1283,8 @@ __global__ __launch_bounds__(kWG) void k_field_reduce(int ppl, const double* __r
     const PointSlot sl = point_slot(g, ppl, partial, design_wbase, design_nchunk, design_pt_off, nd);
     double b[3];
     chunk_sum(sl, b, pts);
-    if ((threadIdx.x & (kWave - 1)) != 0) return;
     analytic_fields(sl.design, qs, design_qs_off, bconst, p, b);
+    if ((threadIdx.x & (kWave - 1)) != 0) return;
     B[g] = b[0];
     B[ptot + g] = b[1];
     B[2 * ptot + g] = b[2];
