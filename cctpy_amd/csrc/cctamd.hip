@@ -747,9 +747,11 @@ __device__ __forceinline__ void direct_row_steps(const KCRow& g, const float (&q
 }
 
 // 6 waves per SIMD (80 VGPRs): hints of 7 (72 VGPRs, 10 spilled) and 8 (64, 23
-// spilled) measured 8 % and 11 % slower on the 64-design population.
+// spilled) measured 8 % and 11 % slower on the 64-design population.  With the far field
+// 4, so that the four items per CU of a population are all under way at once (64 designs x 32:
+// 134 instead of 142 us per stage; FP64 split-wave kernels: no faster at 4 than at 3).
 template <bool FAR>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 6))) void k_bs_partial_f32k_row(const float* __restrict__ seg32k,
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 4 : 6))) void k_bs_partial_f32k_row(const float* __restrict__ seg32k,
                                                              const double* __restrict__ tile_org,
                                                              const double* __restrict__ seg64,
                                                              const Work* __restrict__ work,
