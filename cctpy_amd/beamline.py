@@ -156,9 +156,10 @@ class Beamline(Line2, Magnet, ApertureObject):
         old = self.trajectory.get_length()
         cct_length = big_r * abs(BaseUtils.angle_to_radian(bending_angle))
         self.trajectory.add_arc_line(radius=big_r, clockwise=bending_angle < 0, angle_deg=abs(bending_angle))
+        place = CCT._place_along(self.trajectory, old, big_r, abs(bending_angle))
         for small_r, sign in ((small_r_inner, 1), (small_r_outer, -1)):
-            cct = CCT.create_cct_along(
-                trajectory=self.trajectory, s=old, big_r=big_r, small_r=small_r, bending_angle=abs(bending_angle),
+            cct = CCT._create_at(
+                place, big_r=big_r, small_r=small_r, bending_angle=abs(bending_angle),
                 tilt_angles=tilt_angles if sign == 1 else BaseUtils.list_multiply(tilt_angles, -1),
                 winding_number=winding_number, current=current,
                 starting_point_in_ksi_phi_coordinate=P2.origin(),
@@ -189,10 +190,11 @@ class Beamline(Line2, Magnet, ApertureObject):
         n = disperse_number_per_winding
         wd = winding_numbers[0][0]
         total_rad = BaseUtils.angle_to_radian(total)
+        place = CCT._place_along(self.trajectory, old, big_r, abs(total))
         for small_r, tilts, sign in ((small_rs[0], BaseUtils.list_multiply(tilt_angles[0], -1), -1),
                                      (small_rs[1], tilt_angles[0], 1)):
-            cct = CCT.create_cct_along(self.trajectory, old, big_r, small_r, abs(total), tilts, wd, currents[0],
-                                       P2.origin(), P2(sign * 2 * math.pi * wd, total_rad), n)
+            cct = CCT._create_at(place, big_r, small_r, abs(total), tilts, wd, currents[0], P2.origin(),
+                                 P2(sign * 2 * math.pi * wd, total_rad), n)
             self.magnets.append(cct)
             self.elements.append((old, cct, length))
         ws = winding_numbers[1]
@@ -211,10 +213,11 @@ class Beamline(Line2, Magnet, ApertureObject):
                 end_in = start_in + P2(((-1) ** k) * 2 * math.pi * ws[k], rads[k])
                 end_out = start_out + P2(((-1) ** (k + 1)) * 2 * math.pi * ws[k], rads[k])
             part_length = big_r * BaseUtils.angle_to_radian(abs(bending_angles[k]))
+            place = CCT._place_along(self.trajectory, old, big_r, abs(bending_angles[k]))
             for small_r, tilts, st, en in ((small_rs[3], BaseUtils.list_multiply(ag_tilts, -1), start_in, end_in),
                                            (small_rs[2], ag_tilts, start_out, end_out)):
-                cct = CCT.create_cct_along(self.trajectory, old, big_r, small_r, abs(bending_angles[k]), tilts,
-                                           ws[k], currents[1], st, en, n)
+                cct = CCT._create_at(place, big_r, small_r, abs(bending_angles[k]), tilts, ws[k], currents[1], st,
+                                     en, n)
                 self.magnets.append(cct)
                 self.elements.append((s_part, cct, part_length))
             s_part += part_length
