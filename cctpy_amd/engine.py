@@ -38,14 +38,17 @@ _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # which it does, or the lanes x segments from which it does whatever the clusters; the pair terms per
 # second of the full sum (64-point blocks and larger, smaller blocks), the share of their time that it
 # saves at the least, and the work items per cluster and block of a single design.
-# Measured per RK4 stage, full sum / far field.  FP64: 64 protons in one CCT of 360 tiles (2.9e6, 12
-# clusters) 13 / 20 us, 300 in one of 1,440 (1.8e7, 23) 34 / 22-28, 24 in two gantries at 120 segments per
-# winding (1.0e7, 79) 21 / 15, 64 in the AG-CCT section at 360 (1.2e7, 90) 24 / 16-21, 512 at 720 (1.9e8, 180)
-# 158 / 45-60.  FP32: 2,048 protons in the CCT of 1,440 tiles (9.4e7, 23) 53 / 45-55, 400 in the gantry at
-# 60 (4.1e7, 31) 37 / 29, 64 in the section at 360 (1.2e7, 90) 18 / 18-23, 128 at 720 (4.7e7, 180) 37-40 /
-# 24-34, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 300.
-_FAR = {64: dict(pairs=1.0e7, large=60, any_pairs=4.0e7, rate=(1.25e12, 0.9e12), saved=0.6, share=24),
-        33: dict(pairs=4.0e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
+# Measured per RK4 stage in us, full sum / far field.  FP64: 200 protons in one CCT of 720 tiles (5.9e6 pairs,
+# 11 clusters) 15.3 / 15.4, 300 (8.8e6) 20.0 / 17.0, 64 in the AG-CCT section at 60 segments per winding (2.0e6,
+# 15) 10.2 / 12.6, 16 at 120 (9.8e5, 30) 12.7 / 13.7, one in the gantry at 60 (1.3e6, 39) 11.5 / 10.8, 16 at 120
+# (2.6e6, 78) 15.9 / 12.3, 512 in the section at 720 (1.9e8, 180) 158 / 44.  FP32: 128 in the gantry at 60 (1.0e7,
+# 39) 18.0 / 17.3, 32 in the section at 720 (1.2e7, 180) 19.9 / 20.4, 32 in the gantry at 360 (1.5e7, 234) 19.6 /
+# 18.9, two designs x 32 (2.1e7, 158) 26.5 / 23.3, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 230; single CCTs
+# stay with the full sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3, and nearer to the bound of
+# what the far field may move a track by).
+_FAR = {64: dict(pairs=1.25e6, large=36, any_pairs=8.5e6, rate=(1.25e12, 0.9e12), saved=0.6, share=24),
+        33: dict(pairs=1.3e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
+_FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters (0.35 ms at the rates above)
 
 
 def device() -> torch.device:
@@ -486,7 +489,7 @@ class DeviceModel:
                       out: torch.Tensor) -> None:
         """B (3, P) at device points (3, P): Biot-Savart pass + fixed-order reduction + QS + uniform."""
         # a map pays for its clusters in one call; on the FP32 path a field keeps the terms of every segment
-        far = self.far_field(plan, 64, 0) if precision == 64 and plan.pairs > _FAR[64]["pairs"] else None
+        far = self.far_field(plan, 64, 0) if precision == 64 and plan.pairs > _FAR_MAP_PAIRS else None
         self._call(N.lib.cctamd_bs_field if far is None else N.lib.cctamd_bs_field_far, "cctamd_bs_field", plan,
                    precision, far, _p(points), plan.npt, _p(partial), _p(out))
 
