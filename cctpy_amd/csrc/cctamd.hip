@@ -13,6 +13,8 @@
 //                       in VGPRs (N per lane)
 //   k_bs_partial_f32k_row  32-point blocks: 16-lane rows walk their own tiles,
 //                       segments broadcast within a row by DPP
+//   ...<.., FAR>        with the far field of segment clusters (far.hpp, built by
+//                       far.hip): near segments one by one, the rest as series
 //   k_field_reduce      fixed-order sum of the chunk partials + QS + uniform
 //   k_rk4_stage<S>      same reduction, then RK4 stage S of each particle
 //
@@ -1445,7 +1447,8 @@ int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, do
 // waves sum their points' chunk partials one point after another (the chunk
 // order of k_rk4_stage), a serial tail of ~45 us per launch on the 23,040-segment
 // single CCT whatever the item count (6x slower there; 2.9x on the
-// 368,640-segment AG-CCT section), against ~5 us for the stage kernel.
+// 368,640-segment AG-CCT section, both full sums), against ~4 us for the stage
+// kernel.
 bool fused_stages(const DeviceSet& ds) {
     if (ds.ppl <= 0 || ds.nwork == 0 || ds.far.geo) return false;
     const char* env = getenv("CCTAMD_FUSED_STAGES");
