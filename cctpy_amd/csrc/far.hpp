@@ -13,16 +13,19 @@
 // (the recurrence of the associated Legendre functions in n, with the double factorial
 // (2n - 1)!! taken into beta).  The coefficients are the curl of the multipole series of the
 // vector potential sum kl / |q - m| (addition theorem of 1 / |x - y| in regular and exterior
-// solid harmonics), built once per segment set.  Cut at order N the series is off by about
-// (E / |q - c|)^N of the cluster's sum of |terms|.  A block takes a large cluster's
+// solid harmonics), built once per segment set.  A block takes a large cluster's
 // series where the large one is far enough, else the series of those of its four parts that
 // are, and sums the other parts' segments one by one.
 //
-// Orders per distance (FarOrders): the smallest N whose cut lies below the rounding of the
-// sum it replaces.  Measured against an extended-precision sum over random segments in a
-// ball, relative to the sum of |terms|: ratio 3.0, N = 31: 8e-17; 3.3, 28: 1.2e-16; 4.0, 24:
-// 2.2e-16; 6.0, 20: 1e-17; 10, 15: 5e-17.  The FP32 path cuts at 1e-10 to 1e-11 (its own
-// terms are rounded at 6e-8) and evaluates the series in FP64.
+// Orders per distance (FarOrders), for the worst cluster: one element with all the current on
+// the rim, towards the point.  Relative to that element's term the cut is at most
+// (N + 1) (E / |q - c|)^N or so: below 4e-16 at every distance of the FP64 table (a term of the
+// full sum is rounded by as much), 2e-9 of the FP32 one (terms rounded at 6e-8); other clusters'
+// cuts are smaller against their sum of |terms| (random elements in a ball: by 100 or more).  With the
+// rounding of the series, which are evaluated in FP64 on both paths, worst of elements on the rim,
+// bars, rings and balls at every distance of the tables, against extended precision: 1.1e-15 and
+// 1.0e-9.  FP64 from 3.55 radii on with order 31 at the most keeps the same bound but sums more
+// segments one by one: 512 protons in the AG-CCT section 52 us per stage, with order 35 48.
 #pragma once
 
 #include "common.hpp"
@@ -33,7 +36,7 @@ constexpr int kSmallTiles = 16;           // tiles of a small cluster
 constexpr int kParts = 4;                 // small clusters of a large one
 constexpr int kFarGeo = 8;                // doubles per cluster: centre, 1 / E, E, 0, 0, 0
 constexpr int kFarRec = 8;                // doubles per record: beta_c xyz, beta_s xyz, -kappa, 0
-constexpr int kFarQ64 = 8, kFarQ32 = 5;   // highest order + 1 = 4 Q: 32 on the FP64 path, 20 on the FP32 path
+constexpr int kFarQ64 = 9, kFarQ32 = 5;   // highest order + 1 = 4 Q: 36 on the FP64 path, 20 on the FP32 path
 
 // Record (m, n) of a cluster is at far_row(Q, m) + (n - m); rows hold a multiple of four
 // records (zero beyond the highest order), so that the row loops need no remainder.
@@ -46,9 +49,9 @@ template <bool F64>
 struct FarOrders;
 template <>
 struct FarOrders<true> {
-    static constexpr int n = 9;
-    static constexpr double ratio[n] = {3.0, 3.4, 4.2, 6.0, 8.0, 12.0, 20.0, 40.0, 100.0};
-    static constexpr int order[n] = {31, 28, 24, 19, 17, 14, 12, 10, 8};
+    static constexpr int n = 10;
+    static constexpr double ratio[n] = {3.1, 3.55, 4.05, 5.1, 7.05, 9.85, 13.3, 25.0, 47.0, 120.0};
+    static constexpr int order[n] = {35, 31, 28, 24, 20, 17, 15, 12, 10, 8};
 };
 template <>
 struct FarOrders<false> {
@@ -135,9 +138,10 @@ __host__ __device__ constexpr int far_unit_start(int N, int u) {  // 0 for u = 0
     return u == 0 ? 0 : kFarSeriesCost + kFarRowCost * u + 4 * blocks;
 }
 // Order and cost of a series in one value, as the lists carry them about.
+constexpr int kFarOrderBits = 6;
 template <int LR>
 __host__ __device__ constexpr int far_pack(int N) {
-    return far_unit_start<LR>(N, far_units<LR>(N)) << 5 | N;
+    return far_unit_start<LR>(N, far_units<LR>(N)) << kFarOrderBits | N;
 }
 
 // Order and cost (far_pack) of the series that serves a cluster for a block, 0 if the cluster is too
@@ -182,7 +186,7 @@ template <int NW>
 struct FarLists {
     static constexpr int kRound = kWave * NW;  // large clusters per round
     int near[kParts * kRound];                 // small cluster
-    int far[kParts * kRound];                  // cluster << 6 | order << 1 | large
+    int far[kParts * kRound];                  // cluster << 7 | order << 1 | large
     int start[kParts * kRound];                // cost of the series before this one in the list
     unsigned short close[kRound];              // large clusters of the round that are not far
     int tally[2][(kParts + 1) * NW];           // of a wave: series | other clusters << 16, cost of the series
@@ -209,7 +213,7 @@ __device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs
             order = valid ? far_order<F64, LR>(geo + (int64_t)cl * kFarGeo, ball) : 0;
             far = __ballot(order != 0);
             other = __ballot(valid && order == 0);
-            upto = wave_scan(order >> 5);
+            upto = wave_scan(order >> kFarOrderBits);
         }
         const int own = __popcll(far) | __popcll(other) << 16;
         if (lane == kWave - 1) {
@@ -230,9 +234,9 @@ __device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs
         const int before = __builtin_amdgcn_readlane(count, wave) - own;
         if (order != 0) {
             const int at = n.far + (before & 0xffff) + lane_rank(far);
-            L.far[at] = cl << 6 | (order & 31) << 1 | large;
+            L.far[at] = cl << (kFarOrderBits + 1) | (order & ((1 << kFarOrderBits) - 1)) << 1 | large;
             L.start[at] = n.cost + __builtin_amdgcn_readlane(cost, wave) - __builtin_amdgcn_readlane(upto, kWave - 1) +
-                          upto - (order >> 5);
+                          upto - (order >> kFarOrderBits);
         } else if (valid) {
             put(n.near + (before >> 16) + lane_rank(other));
         }
@@ -304,7 +308,7 @@ __device__ __forceinline__ void far_term(double rec, double Z, double rho, doubl
 // Adds units u0 .. u1 - 1 of the series of a cluster (wave-uniform) at the lane's PL points: rows m
 // of the unit's number (LR = 1), or row 4 u + i in the wave's row i of lanes (LR = 4).  9 FP64
 // instructions per (n, m) and point.
-// The coefficients of a cluster (up to 35 KB) are read once per block and stage, from L2 at
+// The coefficients of a cluster (up to 46 KB) are read once per block and stage, from L2 at
 // best, and a term uses them up quickly: with scalar loads, which a wave can only wait for all
 // at once, the AG-CCT section's FP64 stage spent two thirds of its time waiting.  Vector loads
 // of 16 doubles (two records) return in order; those of the two blocks after the one in use are on
@@ -460,13 +464,13 @@ __device__ __forceinline__ void far_share(const FarLists<NW>& L, const FarCounts
         const int at = __builtin_amdgcn_readfirstlane(L.start[e]);
         if (at >= to) break;
         const int entry = __builtin_amdgcn_readfirstlane(L.far[e]);
-        const int N = entry >> 1 & 31;
+        const int N = entry >> 1 & ((1 << kFarOrderBits) - 1);
         const bool is = lane < far_units<LR>(N);
         const int start = far_unit_start<LR>(N, lane);
         const int u0 = __popcll(__ballot(is && start < from - at)), u1 = __popcll(__ballot(is && start < to - at));
         if (u0 == u1) continue;
         const bool large = entry & 1;
-        const int64_t cl = entry >> 6;
+        const int64_t cl = entry >> (kFarOrderBits + 1);
         far_rows<Q, PL, LR>(const_doubles((large ? fs.geo_large : fs.geo) + cl * kFarGeo),
                             (large ? fs.coef_large : fs.coef) + cl * far_records(Q) * kFarRec, N, u0, u1, px, py, pz,
                             ax, ay, az);
