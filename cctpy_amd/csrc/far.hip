@@ -696,8 +696,9 @@ int64_t cctamd_far_plan(int64_t ndesign, const int64_t* design_ntile, const int6
                 for (int64_t c = 0; c < nc; ++c) {
                     const int64_t ps = design_pt_off[d] + b * pb;
                     const int64_t pc = std::min(pb, design_npt[d] - b * pb);
-                    // cluster numbers are kept shifted by 7 bits (FarLists), their tiles in 31
-                    if (ps + pc > 0x7fffffff || (design_cluster_off[d] + ns) > (0x7fffffff >> (kFarOrderBits + 1))) return CCTAMD_ERANGE;
+                    // cluster numbers are kept shifted by up to 7 bits (FarLists), their tiles in 31
+                    if (ps + pc > 0x7fffffff || design_cluster_off[d] + ns > 0x7fffffff >> (far_order_bits(kFarQ64) + 1))
+                        return CCTAMD_ERANGE;
                     int32_t* w = work + CCTAMD_WORK_INTS * (n + b * nc + c);
                     w[0] = (int32_t)d;
                     w[1] = (int32_t)ps;

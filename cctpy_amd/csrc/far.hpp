@@ -137,11 +137,12 @@ __host__ __device__ constexpr int far_unit_start(int N, int u) {  // 0 for u = 0
                                : u * far_units<4>(N) - u * (u - 1) / 2;
     return u == 0 ? 0 : kFarSeriesCost + kFarRowCost * u + 4 * blocks;
 }
-// Order and cost of a series in one value, as the lists carry them about.
-constexpr int kFarOrderBits = 6;
-template <int LR>
+// Order and cost of a series in one value, as the lists carry them about; the order takes as many
+// bits as the path's highest one needs (6 on the FP32 path too: its gantry stage 4 % slower).
+constexpr int far_order_bits(int q) { return q > 8 ? 6 : 5; }
+template <bool F64, int LR>
 __host__ __device__ constexpr int far_pack(int N) {
-    return far_unit_start<LR>(N, far_units<LR>(N)) << kFarOrderBits | N;
+    return far_unit_start<LR>(N, far_units<LR>(N)) << far_order_bits(F64 ? kFarQ64 : kFarQ32) | N;
 }
 
 // Order and cost (far_pack) of the series that serves a cluster for a block, 0 if the cluster is too
@@ -156,7 +157,7 @@ __device__ __forceinline__ int far_order(const double* __restrict__ geo, const B
     using T = FarOrders<F64>;
     int n = 0;
 #pragma unroll
-    for (int k = 0; k < T::n; ++k) n = ratio >= (float)T::ratio[k] ? far_pack<LR>(T::order[k]) : n;
+    for (int k = 0; k < T::n; ++k) n = ratio >= (float)T::ratio[k] ? far_pack<F64, LR>(T::order[k]) : n;
     return n;
 }
 #pragma clang fp contract(fast)
@@ -186,7 +187,7 @@ template <int NW>
 struct FarLists {
     static constexpr int kRound = kWave * NW;  // large clusters per round
     int near[kParts * kRound];                 // small cluster
-    int far[kParts * kRound];                  // cluster << 7 | order << 1 | large
+    int far[kParts * kRound];                  // cluster | order (far_order_bits) | large (1 bit)
     int start[kParts * kRound];                // cost of the series before this one in the list
     unsigned short close[kRound];              // large clusters of the round that are not far
     int tally[2][(kParts + 1) * NW];           // of a wave: series | other clusters << 16, cost of the series
@@ -204,6 +205,7 @@ struct FarCounts {
 template <bool F64, int LR, int NW>
 __device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs, const Work& w, const Ball& ball,
                                                int base, int wave, int lane) {
+    constexpr int bits = far_order_bits(F64 ? kFarQ64 : kFarQ32);
     FarCounts n{0, 0, 0};
     // a cluster per lane: it joins the series, or put(its place among the others) takes it
     const auto round = [&](int slot, bool valid, int cl, const double* geo, int large, auto&& put) {
@@ -213,7 +215,7 @@ __device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs
             order = valid ? far_order<F64, LR>(geo + (int64_t)cl * kFarGeo, ball) : 0;
             far = __ballot(order != 0);
             other = __ballot(valid && order == 0);
-            upto = wave_scan(order >> kFarOrderBits);
+            upto = wave_scan(order >> bits);
         }
         const int own = __popcll(far) | __popcll(other) << 16;
         if (lane == kWave - 1) {
@@ -234,9 +236,9 @@ __device__ __forceinline__ FarCounts far_lists(FarLists<NW>& L, const FarSet& fs
         const int before = __builtin_amdgcn_readlane(count, wave) - own;
         if (order != 0) {
             const int at = n.far + (before & 0xffff) + lane_rank(far);
-            L.far[at] = cl << (kFarOrderBits + 1) | (order & ((1 << kFarOrderBits) - 1)) << 1 | large;
+            L.far[at] = cl << (bits + 1) | (order & ((1 << bits) - 1)) << 1 | large;
             L.start[at] = n.cost + __builtin_amdgcn_readlane(cost, wave) - __builtin_amdgcn_readlane(upto, kWave - 1) +
-                          upto - (order >> kFarOrderBits);
+                          upto - (order >> bits);
         } else if (valid) {
             put(n.near + (before >> 16) + lane_rank(other));
         }
@@ -452,6 +454,7 @@ template <int Q, int LR, int NW, int PL>
 __device__ __forceinline__ void far_share(const FarLists<NW>& L, const FarCounts& n, const FarSet& fs, int me, int all, int lane,
                                           const double (&px)[PL], const double (&py)[PL], const double (&pz)[PL],
                                           double (&ax)[PL], double (&ay)[PL], double (&az)[PL]) {
+    constexpr int bits = far_order_bits(Q);
     const int nfar = n.far;
     const int from = (int)((int64_t)n.cost * me / all), to = (int)((int64_t)n.cost * (me + 1) / all);
     if (from == to) return;
@@ -464,13 +467,13 @@ __device__ __forceinline__ void far_share(const FarLists<NW>& L, const FarCounts
         const int at = __builtin_amdgcn_readfirstlane(L.start[e]);
         if (at >= to) break;
         const int entry = __builtin_amdgcn_readfirstlane(L.far[e]);
-        const int N = entry >> 1 & ((1 << kFarOrderBits) - 1);
+        const int N = entry >> 1 & ((1 << bits) - 1);
         const bool is = lane < far_units<LR>(N);
         const int start = far_unit_start<LR>(N, lane);
         const int u0 = __popcll(__ballot(is && start < from - at)), u1 = __popcll(__ballot(is && start < to - at));
         if (u0 == u1) continue;
         const bool large = entry & 1;
-        const int64_t cl = entry >> (kFarOrderBits + 1);
+        const int64_t cl = entry >> (bits + 1);
         far_rows<Q, PL, LR>(const_doubles((large ? fs.geo_large : fs.geo) + cl * kFarGeo),
                             (large ? fs.coef_large : fs.coef) + cl * far_records(Q) * kFarRec, N, u0, u1, px, py, pz,
                             ax, ay, az);
