@@ -136,7 +136,35 @@ class Plan:
     design_npt: tuple = ()
     pairs: float = 0.0  # lanes x segments of a launch
     large: float = 0.0  # large segment clusters per block, in the mean
-    far: Dict[int, FarPlan] = dc_field(default_factory=dict)  # by precision
+    # by precision for tracking, by (precision, 0) for single evaluations
+    far: Dict[object, FarPlan] = dc_field(default_factory=dict)
+
+
+def far_items(clusters: int, alike: bool, single: bool, precision: int, ppl: int, cus: int, most: int) -> int:
+    """Work items of a far-field launch: ``clusters`` (of every block together), ``alike`` where the blocks'
+    designs have as many tiles, ``single`` for one evaluation (a map) instead of a track's stages; at ``most`` so
+    many.
+
+    Tracks through designs alike: one or two per CU, as all their items take the same time and between the two
+    some CUs have twice the work of others (512 protons in the AG-CCT section, FP32: 256 items 35.7 us per stage,
+    320 42.4, 480 35.3, 512 33.9, 640 42.4, 1,024 44.3; 128 protons: 21.5, 25.1, 24.4, 24.4, 33.2; FP64 8 gantries
+    x 80: 256 items 23.4, 448 26.6, 512 26.4, 640 33.2).
+
+    Designs that differ balance over smaller items, but over whole rounds of what a CU has under way (two 8-wave
+    items; of the 4-wave ones three or four): the items past a round wait for its slowest.  us per stage of a
+    bunch / of particles all along the orbit, FP64: 4 designs x 48 protons 530 items 37 / 119, 510 31 / 96; 8 x 48
+    852 items 49 / 157, 507 44 / 146; 5 x 100 606 items 60 / 206, 509 56 / 171; 32 x 64 1,025 items 155 / 641,
+    1,006 156 / 492; 4 x 32 530 items 27 / 68, 510 25 / 55; FP32: 4 x 48 44 / 101 and 33 / 67.
+
+    A map's blocks see clusters from next to all around, whatever the designs: four per CU (5,003 points in the
+    section: 320 items 549 us, 640 375, 960 357; 20,000: 471 items 1,446, 942 1,213)."""
+    if single:
+        return min(4 * cus, most)
+    if alike:
+        return min(cus if clusters <= _FAR[precision]["share"] * cus else 2 * cus, most)
+    each = 2 * cus if ppl > 0 else cus
+    whole = int(min(max(clusters // 5, 2 * cus), 6 * cus, most) / each + 0.3) * each  # 0.3: a round that is nearly full
+    return whole if 0 < whole <= most else most
 
 
 class FarField:
@@ -320,16 +348,17 @@ class DeviceModel:
         return p
 
     # --------------------------------------------------------- far field
-    def far_field(self, plan: Plan, precision: int, max_steps: int) -> Optional[FarField]:
+    def far_field(self, plan: Plan, precision: int, max_steps: int) -> Optional[Tuple[FarField, FarPlan]]:
         """The segment clusters that tracking ``plan`` for ``max_steps`` steps uses (0: one field
-        evaluation), built on first need, with their work items in ``plan.far``; None where every
+        evaluation) and their work items, kept in ``plan.far``; built on first need; None where every
         segment is summed."""
         if not self._far_pays(plan, precision, max_steps):
             return None
+        key = precision if max_steps > 0 else (precision, 0)
         with self._far_lock:
             far = self._far.get(precision)
-            if far is not None and precision in plan.far:
-                return far
+            if far is not None and key in plan.far:
+                return far, plan.far[key]
             if torch.cuda.is_current_stream_capturing():
                 return None  # a capture cannot build them
             try:
@@ -337,10 +366,10 @@ class DeviceModel:
                     far = FarField(self, precision)
             except torch.OutOfMemoryError:
                 return None  # the clusters need as much again as the segments
-            plan.far[precision] = self._far_plan(far, plan, precision)
+            plan.far[key] = self._far_plan(far, plan, precision, max_steps == 0)
             torch.cuda.current_stream().synchronize()  # ready for every stream that tracks this model
             self._far[precision] = far
-            return far
+            return far, plan.far[key]
 
     def _far_pays(self, plan: Plan, precision: int, max_steps: int) -> bool:
         """Whether tracking ``plan`` for ``max_steps`` steps (0: one evaluation) is faster with the far
@@ -356,23 +385,14 @@ class DeviceModel:
         rate = rule["rate"][0 if plan.ppl > 0 else 1]
         return max(4 * max_steps, 1) * rule["saved"] * plan.pairs / rate > 0.35e-3 + precision * 2e-11 * self.nseg_padded
 
-    def _far_plan(self, far: FarField, plan: Plan, precision: int) -> FarPlan:
+    def _far_plan(self, far: FarField, plan: Plan, precision: int, single: bool) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
         npt = numpy.asarray(plan.design_npt, numpy.int64)
         pt_off = numpy.concatenate([[0], numpy.cumsum(npt)]).astype(numpy.int64)
-        # Work items.  Designs alike: one or two per CU, as all their items take the same time and between
-        # the two some CUs have twice the work of others (512 protons in the AG-CCT section, FP32: 256 items 35.7
-        # us per stage, 320 42.4, 480 35.3, 512 33.9, 640 42.4, 1,024 44.3; 128 protons: 21.5, 25.1, 24.4, 24.4,
-        # 33.2; FP64 8 gantries x 80: 256 items 23.4, 448 26.6, 512 26.4, 640 33.2).  Designs that differ in what
-        # their blocks need balance over smaller items (24 designs x 32, FP32: 498 items 70, 754 59, 1,012 64).
-        tiles = -(-npt // points_per_block(plan.ppl)) * nt
-        clusters = int((-(-npt // points_per_block(plan.ppl)) * -(-nt // 16)).sum())
-        cus = cu_count()
-        if tiles.max() <= 1.05 * tiles.min():
-            target = cus if clusters <= _FAR[precision]["share"] * cus else 2 * cus
-        else:
-            target = min(max(clusters // 5, cus), 6 * cus)
-        target = min(plan.nwork, target)
+        blocks = -(-npt // points_per_block(plan.ppl))
+        tiles = blocks * nt
+        target = far_items(int((blocks * -(-nt // 16)).sum()), bool(tiles.max() <= 1.05 * tiles.min()), single,
+                           precision, plan.ppl, cu_count(), plan.nwork)
         while True:  # the caller's partial sums hold plan.nwork items (every point block has one)
             args = (self.ndesign, _np(nt), _np(npt), _np(far.cluster_off), _np(pt_off), plan.ppl)
             n = int(N.lib.cctamd_far_plan(*args, target, None, None, None))
@@ -397,12 +417,13 @@ class DeviceModel:
                    precision, far, _p(state), plan.npt, _p(kq), _p(dt), _p(nsteps), int(max_steps), _p(scratch),
                    _p(partial), _p(record), int(record_every))
 
-    def _call(self, function, name: str, plan: Plan, precision: int, far: Optional[FarField], *args) -> None:
-        """A library call on this segment set and plan, with its clusters where ``far`` gives them."""
+    def _call(self, function, name: str, plan: Plan, precision: int, far_field: Optional[Tuple[FarField, FarPlan]],
+              *args) -> None:
+        """A library call on this segment set and plan, with its clusters where ``far_field`` gives them."""
         seg, org, near = self._seg(precision)
         w, head = plan, ()
-        if far is not None:
-            w = plan.far[precision]
+        if far_field is not None:
+            far, w = far_field
             head = (_p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.tiles))
             seg = seg if far.rows is None else far.rows
         N.check(function(*head, precision, plan.ppl, _p(seg), _p(org), _p(near), _p(w.work), w.nwork, _p(w.wbase),

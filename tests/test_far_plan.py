@@ -50,3 +50,23 @@ def test_items_cover_every_block_once(ppl, target):
                                                   ([4], [4], 1, 0)])
 def test_bad_arguments_are_refused(ntile, npt, ppl, target):
     assert _far_plan(ntile, npt, ppl, target) == -22
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, -2, -4])
+@pytest.mark.parametrize("precision", [33, 64])
+def test_items_fill_whole_rounds(precision, ppl):
+    """Designs that differ: no items past a full round of what the CUs have under way (two 8-wave items per CU,
+    one 4-wave item), unless the next round is nearly full too; never more than the caller's."""
+    from cctpy_amd.engine import far_items
+
+    cus = 256
+    each = 2 * cus if ppl > 0 else cus
+    for clusters in (1, 900, 1275, 2000, 2650, 3030, 4260, 5200, 9600, 100000):
+        for most in (7, 255, 300, 530, 986, 1025, 1536, 4096):
+            n = far_items(clusters, False, False, precision, ppl, cus, most)
+            assert 0 < n <= most and n <= 6 * cus
+            over = n % each
+            assert n == most and (most < each or over >= 0.7 * each) or over == 0, (clusters, most, n)
+    # maps: four per CU, whatever the designs
+    assert far_items(28800, True, True, precision, ppl, cus, 5000) == 4 * cus
+    assert far_items(28800, False, True, precision, ppl, cus, 900) == 900
