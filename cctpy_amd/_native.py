@@ -64,6 +64,10 @@ def _load() -> ctypes.CDLL:
     lib.cctamd_far_plan.restype = I64
     lib.cctamd_bs_field_far.argtypes = [P, P, P, P, P] + lib.cctamd_bs_field.argtypes
     lib.cctamd_bs_field_far.restype = INT
+    lib.cctamd_point_spread.argtypes = [INT, P, P, I64, P, I64, P, P]
+    lib.cctamd_point_spread.restype = INT
+    lib.cctamd_bs_field_routed.argtypes = [P, P, P, P, P, P, P, I64, P, P] + lib.cctamd_bs_field.argtypes
+    lib.cctamd_bs_field_routed.restype = INT
     lib.cctamd_track_rk4_far.argtypes = [P, P, P, P, P] + lib.cctamd_track_rk4.argtypes
     lib.cctamd_track_rk4_far.restype = INT
     lib.cctamd_winding_tangents.argtypes = [P, P, P, I64, I64, P, P]
@@ -101,5 +105,6 @@ EXPORTED = (
     "cctamd_pack_fp32", "cctamd_plan", "cctamd_bs_partial", "cctamd_bs_field", "cctamd_track_rk4",
     "cctamd_winding_tangents", "cctamd_track_rk4_taped", "cctamd_track_rk4_adjoint", "cctamd_phase_space",
     "cctamd_beam_objective_seed", "cctamd_bs_field_noalloc", "cctamd_far_coef_doubles", "cctamd_far_keys",
-    "cctamd_far_build", "cctamd_far_plan", "cctamd_bs_field_far", "cctamd_track_rk4_far",
+    "cctamd_far_build", "cctamd_far_plan", "cctamd_bs_field_far", "cctamd_track_rk4_far", "cctamd_point_spread",
+    "cctamd_bs_field_routed",
 )

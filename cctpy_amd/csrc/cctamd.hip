@@ -1050,6 +1050,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
                                                          const double* __restrict__ pts, int64_t ptot,
                                                          double* __restrict__ partial, StageArgs sa, FarSet fs) {
     constexpr int PB = kWave * PPL;
+    if (S < 0 && fs.route && spread_out(fs.route) == FAR) return;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1149,6 +1150,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1
     // LDS rows drop seg64's two pad doubles: (kl.x, kl.y), (kl.z, m.x), (m.y, m.z)
     __shared__ float4 lds[NS][3 * SEGS + 1];
     __shared__ double red[kWavesPerWG][3][PB];
+    if (fs.route && spread_out(fs.route) == FAR) return;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
@@ -1280,9 +1282,15 @@ __global__ __launch_bounds__(kWG) void k_field_reduce(int ppl, const double* __r
                                                       const int64_t* __restrict__ design_qs_off,
                                                       const double* __restrict__ bconst,
                                                       const double* __restrict__ pts, int64_t ptot,
-                                                      double* __restrict__ B) {
+                                                      double* __restrict__ B, const int64_t* __restrict__ route,
+                                                      const int64_t* __restrict__ far_wbase,
+                                                      const int32_t* __restrict__ far_nchunk) {
     const int64_t g = (int64_t)blockIdx.x * kWavesPerWG + (threadIdx.x >> 6);
     if (g >= ptot) return;
+    if (route && !spread_out(route)) {  // the partial sums are the far field's
+        design_wbase = far_wbase;
+        design_nchunk = far_nchunk;
+    }
     const double p[3] = {pts[g], pts[ptot + g], pts[2 * ptot + g]};
     const PointSlot sl = point_slot(g, ppl, partial, design_wbase, design_nchunk, design_pt_off, nd);
     double b[3];
@@ -1406,9 +1414,8 @@ hipError_t launch_bs_shape(int precision, int ppl, const void* seg, const double
 
 hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                          const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
-                         hipStream_t st) {
-    return launch_bs_shape<false>(precision, ppl, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st,
-                                  FarSet{});
+                         hipStream_t st, const FarSet& fs) {
+    return launch_bs_shape<false>(precision, ppl, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st, fs);
 }
 
 // The Biot-Savart pass of a segment set, with its clusters if it has any.
@@ -1416,11 +1423,11 @@ hipError_t launch_bs_set(const DeviceSet& ds, const double* pts, int64_t ptot, d
     return ds.far.geo ? launch_bs_shape<true>(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork,
                                               pts, ptot, partial, st, ds.far)
                       : launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
-                                      ptot, partial, st);
+                                      ptot, partial, st, ds.far);
 }
 
 int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, double* partial, double* B,
-                  hipStream_t st) {
+                  hipStream_t st, const DeviceSet* far) {
     if (!valid_common(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.nwork, ds.ndesign))
         return CCTAMD_EINVAL;
     if (npoints < 0) return CCTAMD_EINVAL;
@@ -1432,10 +1439,12 @@ int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, do
     const int64_t blocks = ceil_div(npoints, kWavesPerWG);
     if (blocks > 0x7fffffff) return CCTAMD_ERANGE;
     hipError_t e = launch_bs_set(ds, points, npoints, partial, st);
+    if (e == hipSuccess && far) e = launch_bs_set(*far, points, npoints, partial, st);
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(k_field_reduce, dim3((unsigned)blocks), dim3(kWG), 0, st, ds.ppl, partial, ds.design_wbase,
                        ds.design_nchunk, ds.design_pt_off, ds.ndesign, ds.qs, ds.design_qs_off, ds.bconst, points,
-                       npoints, B);
+                       npoints, B, far ? ds.far.route : nullptr, far ? far->design_wbase : nullptr,
+                       far ? far->design_nchunk : nullptr);
     return hip_status(hipGetLastError());
 }
 
@@ -1668,11 +1677,30 @@ int cctamd_bs_field_far(const double* geo, const double* geo_large, const double
                         const int32_t* design_nchunk, const int64_t* design_pt_off, int64_t ndesign, const double* qs,
                         const int64_t* design_qs_off, const double* bconst, const double* points, int64_t npoints,
                         double* partial, double* B, void* stream) {
-    const FarSet far{geo, geo_large, coef, coef_large, tiles};
+    const FarSet far{geo, geo_large, coef, coef_large, tiles, nullptr};
     if (!valid_far(far, precision, ppl) || (nwork > 0 && !partial)) return CCTAMD_EINVAL;
     const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
                        design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst, far};
     return field_checked(ds, points, npoints, partial, B, (hipStream_t)stream);
+}
+
+int cctamd_bs_field_routed(const int64_t* spread, const double* geo, const double* geo_large, const double* coef,
+                           const double* coef_large, const double* rows, const int32_t* far_work, int64_t far_nwork,
+                           const int64_t* far_wbase, const int32_t* far_nchunk, int precision, int ppl, const void* seg,
+                           const double* tile_org, const double* seg_near, const int32_t* work, int64_t nwork,
+                           const int64_t* design_wbase, const int32_t* design_nchunk, const int64_t* design_pt_off,
+                           int64_t ndesign, const double* qs, const int64_t* design_qs_off, const double* bconst,
+                           const double* points, int64_t npoints, double* partial, double* B, void* stream) {
+    const FarSet clusters{geo, geo_large, coef, coef_large, nullptr, spread};
+    if (precision != 64 || !valid_far(clusters, precision, ppl) || !spread || !rows || !far_work || !far_wbase ||
+        !far_nchunk || far_nwork <= 0 || far_nwork > nwork || !partial)
+        return CCTAMD_EINVAL;
+    const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase, design_nchunk,
+                       design_pt_off, ndesign, qs, design_qs_off, bconst,
+                       FarSet{nullptr, nullptr, nullptr, nullptr, nullptr, spread}};
+    const DeviceSet far{precision, ppl, rows, tile_org, seg_near, (const Work*)far_work, far_nwork, far_wbase,
+                        far_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst, clusters};
+    return field_checked(ds, points, npoints, partial, B, (hipStream_t)stream, &far);
 }
 
 int cctamd_track_rk4_far(const double* geo, const double* geo_large, const double* coef, const double* coef_large,
@@ -1682,7 +1710,7 @@ int cctamd_track_rk4_far(const double* geo, const double* geo_large, const doubl
                          const int64_t* design_qs_off, const double* bconst, double* state, int64_t nparticles,
                          const double* kq, const double* dt, const int64_t* nsteps, int64_t max_steps, double* scratch,
                          double* partial, double* record, int64_t record_every, void* stream) {
-    const FarSet far{geo, geo_large, coef, coef_large, tiles};
+    const FarSet far{geo, geo_large, coef, coef_large, tiles, nullptr};
     if (!valid_far(far, precision, ppl)) return CCTAMD_EINVAL;
     const DeviceSet ds{precision, ppl, seg, tile_org, seg_near, (const Work*)work, nwork, design_wbase,
                        design_nchunk, design_pt_off, ndesign, qs, design_qs_off, bconst, far};

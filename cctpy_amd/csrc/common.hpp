@@ -362,7 +362,12 @@ struct FarSet {
     const double *coef, *coef_large;  // [C][far_records(Q)][kFarRec], [C / 4][far_records(Q)][kFarRec]
     const int32_t* tiles;             // [C][kSmallTiles] tile of each place, -1 for none (FP32 path); NULL:
                                       // places are tiles of the packed rows passed beside this set (FP64 path)
+    const int64_t* route;             // [2] (FP64 fields) what k_point_spread found, NULL: no choice
 };
+
+// Whether the points' blocks reach across the segments (k_point_spread, where 2/3 comes from): then the far
+// field's kernels leave them to those that sum every segment, and these to them otherwise.
+__device__ __forceinline__ bool spread_out(const int64_t* __restrict__ route) { return 3 * route[0] > 2 * route[1]; }
 
 // ---------------------------------------------------- shared host helpers
 struct DeviceSet {  // one segment set + analytic magnets of D designs
@@ -379,18 +384,19 @@ struct DeviceSet {  // one segment set + analytic magnets of D designs
     const double* qs;
     const int64_t* design_qs_off;
     const double* bconst;
-    FarSet far = {nullptr, nullptr, nullptr, nullptr, nullptr};  // geo NULL: every segment summed one by one
+    FarSet far = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // geo NULL: every segment summed one by one
 };
 
 bool valid_common(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                   int64_t nwork, int64_t ndesign);
 hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                          const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
-                         hipStream_t st);
+                         hipStream_t st, const FarSet& fs = FarSet{});
 // Checked field evaluation (cctamd_bs_field): Biot-Savart pass into `partial` (nwork * 3 * PB
 // doubles), then the fixed-order reduction + QS + uniform fields into B. Returns a CCTAMD code.
+// far: the same set with its clusters, where the points choose between the two on the device (ds.far.route).
 int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, double* partial, double* B,
-                  hipStream_t st);
+                  hipStream_t st, const DeviceSet* far = nullptr);
 // RK4 steps [step0, step1) of every particle (forward), optional record of the
 // state every `record_every` steps (row (step+1)/record_every) and optional
 // tape of the stage points, velocities and fields relative to step0

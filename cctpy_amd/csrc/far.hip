@@ -603,6 +603,51 @@ __global__ void k_far_coef(int q, int64_t nsmall, int64_t nrec, const double* __
     o[5] = s * (dxs[1] - dys[0]);
 }
 
+// How far the blocks of a point set reach across the segments: route[0] / route[1] is the share of a block's
+// segments inside the block's ball, by 256 of them, in the mean over the blocks (weighed by their tiles).  With
+// points in no order along the magnet, or in rows across it, most segments are, and hardly any cluster is far
+// from a block.  FP64 maps of 3,000 to 20,000 points in the AG-CCT section, a single CCT, a population's design
+// and the gantry, time through the clusters over that of the full sum by the share: below 0.06 0.15-0.73, 0.3
+// 0.61-0.87, 0.56 0.78-0.95, 0.7 0.92-1.13, 1.0 (shuffled) 1.00-1.11: the full sum from 2/3 on (spread_out).
+// One wave per block; 5 us with the launch that clears the counts.
+__global__ __launch_bounds__(kWave) void k_point_spread(const double* __restrict__ seg64, const Work* __restrict__ work,
+                                                        const double* __restrict__ pts, int64_t ptot,
+                                                        unsigned long long* __restrict__ route) {
+    constexpr int kMost = 4, kSamples = 256;  // points per lane, segments looked at
+    const Work w = work[blockIdx.x];
+    if (w.chunk != 0) return;  // a block's first item
+    const Work last = work[blockIdx.x + w.nchunk - 1];
+    const int64_t row0 = (int64_t)w.tile_start * kTile;
+    const int64_t nrow = (int64_t)(last.tile_start + last.tile_count) * kTile - row0;
+    if (nrow <= 0) return;
+    const int lane = threadIdx.x;
+    double px[kMost], py[kMost], pz[kMost];
+#pragma unroll
+    for (int j = 0; j < kMost; ++j) {
+        const int at = lane + j * kWave;
+        const int64_t g = w.pt_start + (at < w.pt_count ? at : w.pt_count - 1);
+        px[j] = pts[g];
+        py[j] = pts[ptot + g];
+        pz[j] = pts[2 * ptot + g];
+    }
+    const Ball b = block_ball<kMost>(px, py, pz);
+    const double reach = b.r * b.r;
+    int live = 0, near = 0;
+    for (int j = 0; j < kSamples / kWave; ++j) {
+        const double* r = seg64 + (row0 + (lane + j * kWave) * nrow / kSamples) * 8;
+        const double dx = r[4] - b.x, dy = r[5] - b.y, dz = r[6] - b.z;
+        const bool is = carries(r);
+        live += __popcll(__ballot(is));
+        near += __popcll(__ballot(is && !(dx * dx + dy * dy + dz * dz >= reach)));
+    }
+    if (lane != 0) return;
+    const unsigned long long tiles = (unsigned long long)(nrow / kTile);
+    atomicAdd(route, near * tiles);
+    atomicAdd(route + 1, live * tiles);
+}
+
+__global__ void k_clear_counts(unsigned long long* __restrict__ route) { route[threadIdx.x] = 0; }
+
 }  // namespace
 }  // namespace cctamd_detail
 
@@ -664,6 +709,20 @@ int cctamd_far_build(int precision, const double* seg64, int unit, const float* 
                        ncluster, geo, geo_large, mom);
     hipLaunchKernelGGL(k_far_coef, dim3((unsigned)ceil_div(nr, 256)), dim3(256), 0, st, q, ncluster, nr, geo, geo_large,
                        mom, coef, coef_large);
+    return hip_status(hipGetLastError());
+}
+
+int cctamd_point_spread(int ppl, const double* seg64, const int32_t* work, int64_t nwork, const double* points,
+                        int64_t npoints, int64_t* spread, void* stream) {
+    if (!valid_ppl(ppl) || nwork < 0 || npoints < 0 || !spread) return CCTAMD_EINVAL;
+    if (nwork > 0 && (!seg64 || !work || !points || npoints == 0)) return CCTAMD_EINVAL;
+    if (nwork > 0x7fffffff) return CCTAMD_ERANGE;
+    hipStream_t st = (hipStream_t)stream;
+    unsigned long long* route = (unsigned long long*)spread;
+    hipLaunchKernelGGL(k_clear_counts, dim3(1), dim3(2), 0, st, route);
+    if (nwork > 0)
+        hipLaunchKernelGGL(k_point_spread, dim3((unsigned)nwork), dim3(kWave), 0, st, seg64, (const Work*)work, points,
+                           npoints, route);
     return hip_status(hipGetLastError());
 }
 

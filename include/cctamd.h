@@ -204,7 +204,22 @@ int cctamd_track_rk4(int precision, int ppl, const void *seg, const double *tile
  *                             item takes its share of what its block needs of them.
  * cctamd_bs_field_far and cctamd_track_rk4_far are cctamd_bs_field and cctamd_track_rk4 with
  * these clusters (precision 33: ppl 1, 2, 4, -2; precision 64: any ppl).
+ * cctamd_point_spread looks, for the items of cctamd_plan, how far point blocks reach across the
+ * segments: spread[0] / spread[1] (int64[2], device) is the share of the segments inside the blocks'
+ * balls, and where it is large the clusters are of no use.  cctamd_bs_field_routed (precision 64) is
+ * cctamd_bs_field where 3 spread[0] > 2 spread[1] and cctamd_bs_field_far otherwise, the choice made on the device; rows,
+ * far_work, far_wbase and far_nchunk are the clusters' (far_nwork <= nwork items).
  */
+int cctamd_point_spread(int ppl, const double *seg64, const int32_t *work, int64_t nwork, const double *points,
+                        int64_t npoints, int64_t *spread, void *stream);
+int cctamd_bs_field_routed(const int64_t *spread, const double *geo, const double *geo_large, const double *coef,
+                           const double *coef_large, const double *rows, const int32_t *far_work, int64_t far_nwork,
+                           const int64_t *far_wbase, const int32_t *far_nchunk, int precision, int ppl,
+                           const void *seg, const double *tile_org, const double *seg_near, const int32_t *work,
+                           int64_t nwork, const int64_t *design_wbase, const int32_t *design_nchunk,
+                           const int64_t *design_pt_off, int64_t ndesign, const double *qs,
+                           const int64_t *design_qs_off, const double *bconst, const double *points, int64_t npoints,
+                           double *partial, double *B, void *stream);
 int64_t cctamd_far_coef_doubles(int precision);
 int cctamd_far_keys(const double *seg64, int unit, const int64_t *unit_off, int64_t ndesign, int64_t nunit,
                     int64_t *key, float *centre, void *stream);

@@ -70,3 +70,16 @@ def test_items_fill_whole_rounds(precision, ppl):
     # maps: four per CU, whatever the designs
     assert far_items(28800, True, True, precision, ppl, cus, 5000) == 4 * cus
     assert far_items(28800, False, True, precision, ppl, cus, 900) == 900
+
+def test_bad_arguments_of_a_routed_field_are_refused():
+    """On the host, before any launch."""
+    some = ctypes.c_void_p(64)
+    assert N.lib.cctamd_point_spread(3, some, some, 1, some, 1, some, None) == -22
+    assert N.lib.cctamd_point_spread(2, some, some, 1, some, 1, None, None) == -22
+    assert N.lib.cctamd_point_spread(2, some, None, 1, some, 1, some, None) == -22
+    args = dict(spread=some, geo=some, geo_large=some, coef=some, coef_large=some, rows=some, far_work=some, far_nwork=1,
+                far_wbase=some, far_nchunk=some, precision=64, ppl=2)
+    rest = [some, None, None, some, 1, some, some, some, 1, some, some, some, some, 1, some, some, None]
+    for name, value in (("spread", None), ("geo", None), ("coef_large", None), ("rows", None), ("far_work", None),
+                        ("far_nwork", 0), ("far_nwork", 2), ("far_nchunk", None), ("precision", 33), ("ppl", 3)):
+        assert N.lib.cctamd_bs_field_routed(*{**args, name: value}.values(), *rest) == -22, name

@@ -1,0 +1,125 @@
+"""Field maps through the segment clusters, and those whose points have no use for them.
+
+An FP64 map of many points lets far clusters act through series (within 1e-13 of the sum of every segment: up to 10^5
+terms in another order), unless its blocks reach across the magnet, where every segment is summed (the same bits).
+What a call gives depends on its points alone, not on the calls before it."""
+import numpy as np
+import pytest
+import torch
+
+from tests._helpers import ensure_built, gpu_available
+
+pytestmark = pytest.mark.gpu
+
+ensure_built()
+
+from cctpy_amd import _native as N, engine, workloads as W  # noqa: E402
+from cctpy_amd.magnets import device_parts  # noqa: E402
+
+if not gpu_available():
+    pytest.skip("no GPU visible", allow_module_level=True)
+
+POINTS = [700, 0, 3, 450]  # the third design without windings
+
+
+@pytest.fixture(autouse=True)
+def maps_of_any_size(monkeypatch):
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    monkeypatch.setattr(engine, "_FAR_MAP_PAIRS", 0.0)
+
+
+def _beamlines():
+    designs = W.population(n_designs=3, n_particles=1, seed=5).designs
+    return [W.build_beamline(d) for d in designs]
+
+
+def _model(bls):
+    specs = [device_parts(bl).spec() for bl in bls]
+    specs.insert(2, engine.DesignSpec(qs=np.zeros((0, 16)), bconst=np.array([0.0, 0.0, 0.5])))
+    return engine.DeviceModel(specs, fp32=False)
+
+
+def _points(bls, order):
+    """Along each design's orbit, 20 mm around it, in order or shuffled within the design."""
+    rng = np.random.default_rng(4)
+    rows = []
+    for bl, n in zip(bls[:2] + [bls[0]] + bls[2:], POINTS):
+        q = [bl.trajectory.point_at(float(s)) for s in np.linspace(0, bl.get_length(), n + 2)[1:-1]]
+        p = np.array([[p.x, p.y, 0.0] for p in q]).reshape(n, 3) + rng.uniform(-0.02, 0.02, (n, 3))
+        rows.append(p if order == "ordered" else rng.permutation(p))
+    return torch.from_numpy(np.ascontiguousarray(np.concatenate(rows).T)).to(engine.device())
+
+
+def _field(model, pts, ppl, far=True):
+    plan = model.plan(POINTS, ppl)
+    _, partial = model.workspace(plan)
+    out = torch.full_like(pts, float("nan"))
+    if far:
+        model.field_tensors(plan, 64, pts, partial, out)
+    else:
+        soa = [engine._p(t) for t in (pts, partial, out)]
+        model._call(N.lib.cctamd_bs_field, "cctamd_bs_field", plan, 64, None, soa[0], plan.npt, soa[1], soa[2])
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, -2, -4])
+def test_ordered_maps_take_the_clusters(ppl):
+    bls = _beamlines()
+    model, pts = _model(bls), _points(bls, "ordered")
+    got = _field(model, pts, ppl)
+    want = _field(model, pts, ppl, far=False)
+    assert 64 in model._far and not np.array_equal(got, want)
+    assert np.max(np.abs(got - want)) <= 1e-13 * np.max(np.abs(want))
+    assert np.array_equal(_field(model, pts, ppl), got)
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, -2, -4])
+def test_shuffled_maps_sum_every_segment(ppl):
+    bls = _beamlines()
+    model, pts = _model(bls), _points(bls, "shuffled")
+    want = _field(model, pts, ppl, far=False)
+    assert np.array_equal(_field(model, pts, ppl), want)
+    assert not model._far  # nothing built for them
+    # nor do clusters that are there change it
+    ordered = _points(bls, "ordered")
+    first = _field(model, ordered, ppl)
+    assert 64 in model._far
+    assert np.array_equal(_field(model, pts, ppl), want)
+    assert np.array_equal(_field(model, ordered, ppl), first)
+    assert np.array_equal(_field(_model(bls), ordered, ppl), first)
+
+
+def test_points_that_are_not_finite():
+    """They reach everywhere: a map of them sums every segment; one of them leaves the other points as they are."""
+    bls = _beamlines()
+    model, pts = _model(bls), _points(bls, "ordered")
+    want = _field(model, pts, 2, far=False)
+    one = pts.clone()
+    one[0, 5] = float("nan")
+    got = _field(model, one, 2)
+    others = np.delete(np.arange(pts.shape[1]), 5)
+    assert np.isnan(got[:, 5]).all()
+    assert np.max(np.abs(got[:, others] - want[:, others])) <= 1e-13 * np.max(np.abs(want))
+    every = torch.full_like(pts, float("inf"))
+    assert np.array_equal(_field(model, every, 2), _field(model, every, 2, far=False), equal_nan=True)
+
+
+def test_a_captured_map_follows_its_points():
+    """The choice is the device's: replays with other points in the buffer are the eager calls on them."""
+    bls = _beamlines()
+    model = _model(bls)
+    sets = [_points(bls, "ordered"), _points(bls, "shuffled")]
+    want = [_field(model, p, 2) for p in sets]
+    plan = model.plan(POINTS, 2)
+    _, partial = model.workspace(plan)
+    pts, out = sets[0].clone(), torch.empty_like(sets[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        model.field_tensors(plan, 64, pts, partial, out)
+    for rep in range(4):
+        pts.copy_(sets[rep % 2])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want[rep % 2]), rep
+        assert np.array_equal(_field(model, sets[rep % 2], 2), want[rep % 2]), rep
