@@ -34,21 +34,27 @@ _TARGET_WG_PER_CU = 4
 _MIN_TILES_PER_ITEM = 4
 _LARGE_TILES = 64   # tiles of a large segment cluster (kParts * kSmallTiles in csrc/far.hpp)
 _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
-# Where tracking takes the far field: lanes x segments of a launch and large clusters per design from
-# which it does, or the lanes x segments from which it does whatever the clusters; the pair terms per
-# second of the full sum (64-point blocks and larger, smaller blocks), the share of their time that it
-# saves at the least, and the work items per cluster and block of a single design.
-# Measured per RK4 stage in us, full sum / far field.  FP64: 200 protons in one CCT of 720 tiles (5.9e6 pairs,
-# 11 clusters) 15.3 / 15.4, 300 (8.8e6) 20.0 / 17.0, 64 in the AG-CCT section at 60 segments per winding (2.0e6,
-# 15) 10.2 / 12.6, 16 at 120 (9.8e5, 30) 12.7 / 13.7, one in the gantry at 60 (1.3e6, 39) 11.5 / 10.8, 16 at 120
-# (2.6e6, 78) 15.9 / 12.3, 512 in the section at 720 (1.9e8, 180) 158 / 44.  FP32: 128 in the gantry at 60 (1.0e7,
-# 39) 18.0 / 17.3, 32 in the section at 720 (1.2e7, 180) 19.9 / 20.4, 32 in the gantry at 360 (1.5e7, 234) 19.6 /
-# 18.9, two designs x 32 (2.1e7, 158) 26.5 / 23.3, 4,096 in the gantry at 720 (3.9e9, 468) 1,620 / 230; single CCTs
-# stay with the full sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3, and nearer to the bound of
-# what the far field may move a track by).
-_FAR = {64: dict(pairs=1.25e6, large=36, any_pairs=8.5e6, rate=(1.25e12, 0.9e12), saved=0.6, share=24),
-        33: dict(pairs=1.3e7, large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25, share=6)}
-_FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters (0.35 ms at the rates above)
+# Where tracking takes the far field: lanes x segments of a launch (64-point blocks and larger, smaller blocks) and
+# large clusters per design from which it does, or the lanes x segments from which it does whatever the clusters; the
+# pair terms per second of the full sum (the same two block sizes) and the share of their time that a bunch saves at the
+# least; the set-up in s and s per segment; and the work items per cluster and block of a single design.
+# Measured per RK4 stage in us, full sum / far field, for a bunch and for particles all along the orbit.  FP64: one
+# in the gantry at 60 segments per winding (1.3e6 pairs, 39 clusters) 12.9 / 12.1 and 13.0 / 11.9, 64 in the AG-CCT section at
+# 60 (2.0e6, 15) 11.5 / 13.7, 32 at 120 (2.0e6, 30) 13.6 / 15.6, 16 at 360 (2.9e6, 90) 17.2 / 15.5 and 17.6 / 15.7, 32 in the
+# gantry at 120 (5.1e6, 78) 17.0 / 13.4 and 17.6 / 18.2, 200 in one CCT of 720 tiles (5.9e6, 11) 16.2 / 16.7, 300 (8.8e6)
+# 20.4 / 18.4, 64 in the gantry at 720 (6.1e7, 468) 68 / 19 and 72 / 89, 512 in the section at 720 (1.9e8, 180) 152 / 52
+# and 155 / 157.  FP32: 64 in the section at 360 (1.2e7, 90) 16.6 / 16.8, at 720 (2.4e7, 180) 23.4 / 18.2 and 23.6 / 29.8, 128 in
+# the gantry at 120 (2.0e7, 78) 24.5 / 18.2 and 38.2 / 31.6; 32-point blocks: 32 in the gantry at 360 (1.5e7, 234) 19.5 / 20.0
+# and 24.9 / 29.8, at 720 (3.1e7, 468) 27.1 / 25.7 and 31.2 / 42.7, four designs x 32 (4.4e7, 166) 33.9 / 28.2 and
+# 35.7 / 41.0; 4,096 in the gantry at 720 (3.9e9) 1,500 / 221 and 1,500 / 1,790; single CCTs stay with the full
+# sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3, and nearer to the bound of what the far field may move a
+# track by).  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640, 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
+_FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, rate=(1.25e12, 0.9e12), saved=0.6,
+                 setup=(0.47e-3, 1.45e-9), share=24),
+        33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25,
+                 setup=(0.40e-3, 0.66e-9), share=6)}
+_FAR_MAP_SAVED = (0.3, 0.7)  # of a map: single CCTs, of few clusters, and the section, a population's design, the gantry
+_FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters
 
 
 def device() -> torch.device:
@@ -376,14 +382,14 @@ class DeviceModel:
         field, its set-up (once per model) included: a function of the sizes alone, so that equal
         calls give equal bits."""
         rule = _FAR.get(precision)
-        if rule is None or plan.pairs < rule["pairs"] or (plan.large < rule["large"]
-                                                          and plan.pairs < rule["any_pairs"]):
-            return False
-        if self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
+        if rule is None or self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
             return False  # keys hold 15 bits of design; 16-point blocks of the FP32 path have no far-field kernel
-        # the set-up, 0.35 ms + 1.3 (FP32 0.7) ns per segment, against what the evaluations save
-        rate = rule["rate"][0 if plan.ppl > 0 else 1]
-        return max(4 * max_steps, 1) * rule["saved"] * plan.pairs / rate > 0.35e-3 + precision * 2e-11 * self.nseg_padded
+        size = 0 if plan.ppl > 0 else 1
+        if plan.pairs < rule["pairs"][size] or (plan.large < rule["large"] and plan.pairs < rule["any_pairs"]):
+            return False
+        saved = rule["saved"] if max_steps > 0 else _FAR_MAP_SAVED[plan.large >= 40]
+        base, each = rule["setup"]
+        return max(4 * max_steps, 1) * saved * plan.pairs / rule["rate"][size] > base + each * self.nseg_padded
 
     def _far_plan(self, far: FarField, plan: Plan, precision: int, single: bool) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)
@@ -437,14 +443,15 @@ class DeviceModel:
         if far_field is None:
             return ()
         far, w = far_field
-        return (spread, far.geo, far.geo_large, far.coef, far.coef_large, far.rows, w.work, w.nwork, w.wbase, w.nchunk)
+        return (_p(spread), _p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.rows), _p(w.work),
+                w.nwork, _p(w.wbase), _p(w.nchunk))
 
     def _call(self, function, name: str, plan: Plan, precision: int, far_field: Optional[Tuple[FarField, FarPlan]],
               *args, head: tuple = ()) -> None:
         """A library call on this segment set and plan, with its clusters where ``far_field`` gives them;
         ``head`` goes before."""
         seg, org, near = self._seg(precision)
-        w, head = plan, tuple(_p(a) if isinstance(a, torch.Tensor) else a for a in head)
+        w = plan
         if far_field is not None:
             far, w = far_field
             head = (_p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.tiles))

@@ -83,3 +83,42 @@ def test_bad_arguments_of_a_routed_field_are_refused():
     for name, value in (("spread", None), ("geo", None), ("coef_large", None), ("rows", None), ("far_work", None),
                         ("far_nwork", 0), ("far_nwork", 2), ("far_nchunk", None), ("precision", 33), ("ppl", 3)):
         assert N.lib.cctamd_bs_field_routed(*{**args, name: value}.values(), *rest) == -22, name
+
+
+def _pays(precision, ppl, segments, points, steps, designs=1):
+    """DeviceModel._far_pays of designs of so many segments and points each."""
+    from cctpy_amd import engine
+
+    model = object.__new__(engine.DeviceModel)
+    model.ndesign, model.nseg_padded = designs, designs * segments
+    pb = engine.points_per_block(ppl)
+    plan = engine.Plan(ppl=ppl, nwork=0, work=None, wbase=None, nchunk=None, design_pt_off=None, npt=designs * points,
+                       pairs=float(designs * -(-points // pb) * pb * segments), large=segments / 2048)
+    return model._far_pays(plan, precision, steps)
+
+
+def test_small_blocks_of_the_fp32_path_keep_the_full_sum():
+    """Where a bunch gains nothing and particles all along the orbit lose (gantry of 479,520 segments, 32 of them)."""
+    assert not _pays(33, -2, 479520, 32, 1000)
+    assert not _pays(33, -2, 959040, 32, 1000)
+    assert _pays(33, 1, 368640, 64, 1000)
+    assert _pays(33, -2, 204800, 32, 1000, designs=64)
+
+
+@pytest.mark.parametrize("precision,ppl,points", [(64, 2, 512), (64, 1, 64), (64, -2, 32), (33, 2, 512), (33, 1, 64)])
+def test_short_tracks_do_not_pay_for_clusters(precision, ppl, points):
+    """What a bunch saves of the full sum's time (0.6 on the FP64 path, 0.25 on the FP32 path) pays for the set-up as it
+    is measured (0.96 and 0.64 ms for the section) in one track."""
+    segments = 368640
+    rate = {(64, True): 1.25e12, (64, False): 0.9e12, (33, True): 2.5e12}[precision, ppl > 0]
+    saved, setup = {64: (0.6, 0.96e-3), 33: (0.25, 0.64e-3)}[precision]
+    from cctpy_amd.engine import points_per_block
+
+    lanes = -(-points // points_per_block(ppl)) * points_per_block(ppl)
+    taken = [n for n in range(1, 400) if _pays(precision, ppl, segments, points, n)]
+    assert taken and 4 * taken[0] * lanes * segments / rate * saved >= setup
+
+
+def test_maps_pay_for_their_clusters_in_one_call():
+    assert _pays(64, 2, 368640, 5003, 0) and not _pays(64, 2, 368640, 2000, 0)
+    assert not _pays(64, 2, 46080, 20000, 0)  # a single CCT: few clusters, 0.3 of the time saved
