@@ -1043,14 +1043,15 @@ __device__ __forceinline__ SegPair seg_pair(ConstDoubles s) {
     return p;
 }
 
-// Plain FP64 terms on global-frame segments.
-template <int PPL, int NW, bool FAR = false, int S = -1>
+// Plain FP64 terms on global-frame segments.  ROUTED: one of the two launches of a field whose points choose
+// between them (a kernel of its own: the look at fs.route cost the others 0.15-0.3 us per launch).
+template <int PPL, int NW, bool FAR = false, int S = -1, bool ROUTED = false>
 __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fused_waves(kKindF64, PPL, S, FAR)))) void k_bs_partial_f64(const double* __restrict__ seg64,
                                                          const Work* __restrict__ work,
                                                          const double* __restrict__ pts, int64_t ptot,
                                                          double* __restrict__ partial, StageArgs sa, FarSet fs) {
     constexpr int PB = kWave * PPL;
-    if (S < 0 && fs.route && spread_out(fs.route) == FAR) return;
+    if (ROUTED && spread_out(fs.route) == FAR) return;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1137,7 +1138,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(fuse
 // LDS per workgroup small enough for several workgroups per CU (<4, 2, 2>:
 // 7 waves per SIMD, 2.5 % faster than whole tiles at 4; 8 groups of 4 points
 // per lane were slower).
-template <int G, int PL, int PARTS, bool FAR>
+template <int G, int PL, int PARTS, bool FAR, bool ROUTED>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1))) void k_bs_partial_f64_grp(const double* __restrict__ seg64,
                                                              const Work* __restrict__ work,
                                                              const double* __restrict__ pts, int64_t ptot,
@@ -1150,7 +1151,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(FAR ? 3 : 1
     // LDS rows drop seg64's two pad doubles: (kl.x, kl.y), (kl.z, m.x), (m.y, m.z)
     __shared__ float4 lds[NS][3 * SEGS + 1];
     __shared__ double red[kWavesPerWG][3][PB];
-    if (fs.route && spread_out(fs.route) == FAR) return;
+    if (ROUTED && spread_out(fs.route) == FAR) return;
     const Work w = work[blockIdx.x];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
@@ -1387,10 +1388,10 @@ hipError_t launch_bs_shape(int precision, int ppl, const void* seg, const double
     if (ppl < 0) {
         if (precision == 64) {
             if (ppl == -2)
-                hipLaunchKernelGGL((k_bs_partial_f64_grp<4, 2, 2, FAR>), dim3((unsigned)nwork), dim3(kWG), 0, st,
+                hipLaunchKernelGGL((k_bs_partial_f64_grp<4, 2, 2, FAR, false>), dim3((unsigned)nwork), dim3(kWG), 0, st,
                                    (const double*)seg, work, pts, ptot, partial, fs);
             else
-                hipLaunchKernelGGL((k_bs_partial_f64_grp<8, 2, 4, FAR>), dim3((unsigned)nwork), dim3(kWG), 0, st,
+                hipLaunchKernelGGL((k_bs_partial_f64_grp<8, 2, 4, FAR, false>), dim3((unsigned)nwork), dim3(kWG), 0, st,
                                    (const double*)seg, work, pts, ptot, partial, fs);
             return hipGetLastError();
         }
@@ -1414,8 +1415,9 @@ hipError_t launch_bs_shape(int precision, int ppl, const void* seg, const double
 
 hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                          const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
-                         hipStream_t st, const FarSet& fs) {
-    return launch_bs_shape<false>(precision, ppl, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st, fs);
+                         hipStream_t st) {
+    return launch_bs_shape<false>(precision, ppl, seg, tile_org, seg_near, work, nwork, pts, ptot, partial, st,
+                                  FarSet{});
 }
 
 // The Biot-Savart pass of a segment set, with its clusters if it has any.
@@ -1423,7 +1425,38 @@ hipError_t launch_bs_set(const DeviceSet& ds, const double* pts, int64_t ptot, d
     return ds.far.geo ? launch_bs_shape<true>(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork,
                                               pts, ptot, partial, st, ds.far)
                       : launch_bs_any(ds.precision, ds.ppl, ds.seg, ds.tile_org, ds.seg_near, ds.work, ds.nwork, pts,
-                                      ptot, partial, st, ds.far);
+                                      ptot, partial, st);
+}
+
+// One of the two passes of an FP64 field whose points choose between them (ds.far.route).
+template <bool FAR>
+hipError_t launch_bs_routed(const DeviceSet& ds, const double* pts, int64_t ptot, double* partial, hipStream_t st) {
+    if (ds.nwork == 0) return hipSuccess;
+    const dim3 grid((unsigned)ds.nwork), wide(kWave * kBsWaves);
+    const double* seg = (const double*)ds.seg;
+    const StageArgs none{};
+    switch (ds.ppl) {
+        case 1:
+            hipLaunchKernelGGL((k_bs_partial_f64<1, kBsWaves, FAR, -1, true>), grid, wide, 0, st, seg, ds.work, pts, ptot,
+                               partial, none, ds.far);
+            break;
+        case 2:
+            hipLaunchKernelGGL((k_bs_partial_f64<2, kBsWaves, FAR, -1, true>), grid, wide, 0, st, seg, ds.work, pts, ptot,
+                               partial, none, ds.far);
+            break;
+        case 4:
+            hipLaunchKernelGGL((k_bs_partial_f64<4, kBsWaves, FAR, -1, true>), grid, wide, 0, st, seg, ds.work, pts, ptot,
+                               partial, none, ds.far);
+            break;
+        case -2:
+            hipLaunchKernelGGL((k_bs_partial_f64_grp<4, 2, 2, FAR, true>), grid, dim3(kWG), 0, st, seg, ds.work, pts, ptot,
+                               partial, ds.far);
+            break;
+        default:
+            hipLaunchKernelGGL((k_bs_partial_f64_grp<8, 2, 4, FAR, true>), grid, dim3(kWG), 0, st, seg, ds.work, pts, ptot,
+                               partial, ds.far);
+    }
+    return hipGetLastError();
 }
 
 int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, double* partial, double* B,
@@ -1438,8 +1471,9 @@ int field_checked(const DeviceSet& ds, const double* points, int64_t npoints, do
     if (ds.nwork > 0 && (!ds.work || !partial)) return CCTAMD_EINVAL;
     const int64_t blocks = ceil_div(npoints, kWavesPerWG);
     if (blocks > 0x7fffffff) return CCTAMD_ERANGE;
-    hipError_t e = launch_bs_set(ds, points, npoints, partial, st);
-    if (e == hipSuccess && far) e = launch_bs_set(*far, points, npoints, partial, st);
+    hipError_t e = far ? launch_bs_routed<false>(ds, points, npoints, partial, st)
+                       : launch_bs_set(ds, points, npoints, partial, st);
+    if (e == hipSuccess && far) e = launch_bs_routed<true>(*far, points, npoints, partial, st);
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(k_field_reduce, dim3((unsigned)blocks), dim3(kWG), 0, st, ds.ppl, partial, ds.design_wbase,
                        ds.design_nchunk, ds.design_pt_off, ds.ndesign, ds.qs, ds.design_qs_off, ds.bconst, points,

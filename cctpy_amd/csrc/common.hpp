@@ -391,7 +391,7 @@ bool valid_common(int precision, int ppl, const void* seg, const double* tile_or
                   int64_t nwork, int64_t ndesign);
 hipError_t launch_bs_any(int precision, int ppl, const void* seg, const double* tile_org, const double* seg_near,
                          const Work* work, int64_t nwork, const double* pts, int64_t ptot, double* partial,
-                         hipStream_t st, const FarSet& fs = FarSet{});
+                         hipStream_t st);
 // Checked field evaluation (cctamd_bs_field): Biot-Savart pass into `partial` (nwork * 3 * PB
 // doubles), then the fixed-order reduction + QS + uniform fields into B. Returns a CCTAMD code.
 // far: the same set with its clusters, where the points choose between the two on the device (ds.far.route).
