@@ -34,8 +34,8 @@ _TARGET_WG_PER_CU = 4
 _MIN_TILES_PER_ITEM = 4
 _LARGE_TILES = 64   # tiles of a large segment cluster (kParts * kSmallTiles in csrc/far.hpp)
 _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
-# Where tracking takes the far field: lanes x segments of a launch (64-point blocks and larger, smaller blocks) and
-# large clusters per design from which it does, or the lanes x segments from which it does whatever the clusters; the
+# Where tracking takes the far field (64-point blocks and larger, smaller blocks): lanes x segments of a launch and
+# large clusters per design from which it does, or fewer clusters but more lanes x segments (any_*); the
 # pair terms per second of the full sum (the same two block sizes) and the share of their time that a bunch saves at the
 # least; the set-up in s and s per segment; and the work items per cluster and block of a single design.
 # Measured per RK4 stage in us, full sum / far field, for a bunch and for particles all along the orbit.  FP64: one
@@ -48,12 +48,15 @@ _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # and 24.9 / 29.8, at 720 (3.1e7, 468) 27.1 / 25.7 and 31.2 / 42.7, four designs x 32 (4.4e7, 166) 33.9 / 28.2 and
 # 35.7 / 41.0; 4,096 in the gantry at 720 (3.9e9) 1,500 / 221 and 1,500 / 1,790; single CCTs stay with the full
 # sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3, and nearer to the bound of what the far field may move a
-# track by).  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640, 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
-_FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, rate=(1.25e12, 0.9e12), saved=0.6,
-                 setup=(0.47e-3, 1.45e-9), share=24),
-        33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, rate=(2.5e12, 1.75e12), saved=0.25,
+# track by).  Many designs of few clusters, FP64: 2,000 of 200 segments x 64 198 / 242 and 44 ms of set-up, 200 of 3,000
+# x 64 63 / 87, 64 of 8,000 x 64 46 / 49, 24 of 16,000 x 64 36 / 38, 24 of 23,040 x 100 86 / 65, 8 of 30,000 x 100 40 / 31; 100 of
+# 23,040 x 32 91 / 105.  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640, 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
+_FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, any_large=(10, 36), rate=(1.25e12, 0.9e12),
+                 saved=0.6, setup=(0.47e-3, 1.45e-9), share=24),
+        33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, any_large=(30, 30), rate=(2.5e12, 1.75e12), saved=0.25,
                  setup=(0.40e-3, 0.66e-9), share=6)}
 _FAR_MAP_SAVED = (0.3, 0.7)  # of a map: single CCTs, of few clusters, and the section, a population's design, the gantry
+_FAR_MOST_ROWS = 1 << 28  # rows of the clusters (FP64 160 B each, and 145 B while they are built): 43 GB
 _FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters
 
 
@@ -234,6 +237,7 @@ class DeviceModel:
         self.design_nseg = nseg
         S = int(self.design_tile_off[-1]) * N.TILE
         self.nseg_padded = S
+        self.cluster_rows = int((-(-self.design_ntile // _LARGE_TILES)).sum()) * _LARGE_TILES * N.TILE
         self.nseg = int(nseg.sum())
         # pad segments: kl = 0 and a midpoint far from every field point
         seg64 = torch.zeros((max(S, 1), 8), dtype=torch.float64, device=dev)
@@ -385,11 +389,12 @@ class DeviceModel:
         if rule is None or self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
             return False  # keys hold 15 bits of design; 16-point blocks of the FP32 path have no far-field kernel
         size = 0 if plan.ppl > 0 else 1
-        if plan.pairs < rule["pairs"][size] or (plan.large < rule["large"] and plan.pairs < rule["any_pairs"]):
+        large = rule["large"] if plan.pairs < rule["any_pairs"] else rule["any_large"][size]
+        if plan.pairs < rule["pairs"][size] or plan.large < large or self.cluster_rows > _FAR_MOST_ROWS:
             return False
         saved = rule["saved"] if max_steps > 0 else _FAR_MAP_SAVED[plan.large >= 40]
         base, each = rule["setup"]
-        return max(4 * max_steps, 1) * saved * plan.pairs / rule["rate"][size] > base + each * self.nseg_padded
+        return max(4 * max_steps, 1) * saved * plan.pairs / rule["rate"][size] > base + each * self.cluster_rows
 
     def _far_plan(self, far: FarField, plan: Plan, precision: int, single: bool) -> FarPlan:
         nt = numpy.ascontiguousarray(self.design_ntile, numpy.int64)

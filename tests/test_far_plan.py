@@ -91,6 +91,7 @@ def _pays(precision, ppl, segments, points, steps, designs=1):
 
     model = object.__new__(engine.DeviceModel)
     model.ndesign, model.nseg_padded = designs, designs * segments
+    model.cluster_rows = designs * -(-segments // 2048) * 2048
     pb = engine.points_per_block(ppl)
     plan = engine.Plan(ppl=ppl, nwork=0, work=None, wbase=None, nchunk=None, design_pt_off=None, npt=designs * points,
                        pairs=float(designs * -(-points // pb) * pb * segments), large=segments / 2048)
@@ -117,6 +118,19 @@ def test_short_tracks_do_not_pay_for_clusters(precision, ppl, points):
     lanes = -(-points // points_per_block(ppl)) * points_per_block(ppl)
     taken = [n for n in range(1, 400) if _pays(precision, ppl, segments, points, n)]
     assert taken and 4 * taken[0] * lanes * segments / rate * saved >= setup
+
+
+@pytest.mark.parametrize("ppl,segments,points,designs", [(1, 200, 64, 2000), (1, 1000, 64, 500), (1, 3000, 64, 200),
+                                                         (1, 8000, 64, 64), (1, 16000, 64, 24), (-2, 23040, 32, 100)])
+def test_many_small_designs_keep_the_full_sum(ppl, segments, points, designs):
+    """A design takes at least one large cluster of 2,048 rows, whatever it holds, and a few clusters are close to all of
+    its points."""
+    assert not _pays(64, ppl, segments, points, 1000, designs)
+
+
+def test_the_clusters_of_a_model_are_bounded():
+    assert _pays(64, 1, 400000, 64, 1000, designs=640)
+    assert not _pays(64, 1, 400000, 64, 1000, designs=1000)
 
 
 def test_maps_pay_for_their_clusters_in_one_call():
