@@ -298,6 +298,13 @@ class DeviceModel:
         self._far: Dict[int, FarField] = {}
         self._far_lock = threading.Lock()
 
+    def __getstate__(self) -> dict:  # copies and pickles: everything but the lock
+        return {k: v for k, v in self.__dict__.items() if k != "_far_lock"}
+
+    def __setstate__(self, state: dict) -> None:
+        self.__dict__.update(state)
+        self._far_lock = threading.Lock()
+
     # --------------------------------------------------------- adjoint data
     def adjoint_data(self):
         """(seg_tan [T][33][8] f32, tile_cct [T] i32, cct_coef [ncct] f64) for cctamd_track_rk4_adjoint."""
