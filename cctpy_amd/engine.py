@@ -296,13 +296,15 @@ class DeviceModel:
         self.bconst = torch.from_numpy(b).to(dev)
         self._plans: Dict[tuple, Plan] = {}
         self._far: Dict[int, FarField] = {}
+        self._stream = torch.cuda.current_stream()  # that of the tensors above
         self._far_lock = threading.Lock()
 
-    def __getstate__(self) -> dict:  # copies and pickles: everything but the lock
-        return {k: v for k, v in self.__dict__.items() if k != "_far_lock"}
+    def __getstate__(self) -> dict:  # copies and pickles: everything but the stream and the lock
+        return {k: v for k, v in self.__dict__.items() if k not in ("_stream", "_far_lock")}
 
     def __setstate__(self, state: dict) -> None:
         self.__dict__.update(state)
+        self._stream = torch.cuda.current_stream()
         self._far_lock = threading.Lock()
 
     # --------------------------------------------------------- adjoint data
@@ -372,21 +374,26 @@ class DeviceModel:
         if not self._far_pays(plan, precision, max_steps):
             return None
         key = precision if max_steps > 0 else (precision, 0)
+        far, items = self._far.get(precision), plan.far.get(key)
+        if far is not None and items is not None:
+            return far, items
+        if torch.cuda.is_current_stream_capturing():
+            return None  # a capture cannot build them
         with self._far_lock:
-            far = self._far.get(precision)
-            if far is not None and key in plan.far:
-                return far, plan.far[key]
-            if torch.cuda.is_current_stream_capturing():
-                return None  # a capture cannot build them
-            try:
-                if far is None:
-                    far = FarField(self, precision)
-            except torch.OutOfMemoryError:
-                return None  # the clusters need as much again as the segments
-            plan.far[key] = self._far_plan(far, plan, precision, max_steps == 0)
-            torch.cuda.current_stream().synchronize()  # ready for every stream that tracks this model
-            self._far[precision] = far
-            return far, plan.far[key]
+            far, items = self._far.get(precision), plan.far.get(key)
+            # On the model's own stream: they live as long as its segments, whichever stream tracks first (memory goes
+            # back to the stream that it was taken on, which knows nothing of the others' launches).
+            with torch.cuda.stream(self._stream):
+                try:
+                    if far is None:
+                        far = FarField(self, precision)
+                except torch.OutOfMemoryError:
+                    return None  # the clusters need as much again as the segments
+                if items is None:
+                    items = self._far_plan(far, plan, precision, max_steps == 0)
+                self._stream.synchronize()  # ready for every stream that tracks this model
+            self._far[precision], plan.far[key] = far, items
+            return far, items
 
     def _far_pays(self, plan: Plan, precision: int, max_steps: int) -> bool:
         """Whether tracking ``plan`` for ``max_steps`` steps (0: one evaluation) is faster with the far
@@ -580,6 +587,7 @@ class TrackGraph:
                  dt: torch.Tensor, nsteps: torch.Tensor, max_steps: int, scratch: torch.Tensor,
                  partial: torch.Tensor):
         self.buffers = (state, kq, dt, nsteps, scratch, partial)  # kept alive with the graph
+        self.model, self.plan = model, plan  # and the segments, clusters and work items that it reads
         model.far_field(plan, precision, max_steps)  # built before the capture, which cannot
         self.graph = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream()  # default priority

@@ -1,6 +1,9 @@
 """A model and its segment clusters copied, pickled, and used from several streams and threads."""
 import copy
+import gc
 import pickle
+import threading
+import weakref
 
 import numpy as np
 import pytest
@@ -57,3 +60,80 @@ def test_copies_of_a_model_track_alike(how, tracked, precision, monkeypatch):
     want = _track(model, precision, *rest)
     assert precision in model._far
     assert np.all(np.isfinite(want)) and np.array_equal(_track(other, precision, *rest), want)
+
+
+def _stream_of(tensor):
+    """The stream whose pool a tensor's memory is from."""
+    for seg in torch.cuda.memory_snapshot():
+        if seg["address"] <= tensor.data_ptr() < seg["address"] + seg["total_size"]:
+            return seg["stream"]
+    raise AssertionError("not an allocation of torch")
+
+
+@pytest.mark.parametrize("precision", [64, 33])
+def test_clusters_live_as_long_as_the_segments(precision, monkeypatch):
+    """Built by the first call on another stream, used by a third: the memory belongs to the model's stream, like its
+    segments', not to the stream that happened to come first."""
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    model, *rest = _case(precision)
+    torch.cuda.synchronize()
+    want = None
+    for _ in range(2):
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            got = _track(model, precision, *rest)
+        side.synchronize()
+        want = got if want is None else want
+        assert np.array_equal(got, want)
+    assert np.array_equal(_track(model, precision, *rest), want)
+    far, items = model._far[precision], model.plan(rest[-1], 1).far[precision]
+    own = _stream_of(model.seg64)
+    for t in (far.geo, far.geo_large, far.coef, far.coef_large, far.rows, far.tiles, items.work, items.wbase, items.nchunk):
+        assert t is None or _stream_of(t) == own
+
+
+@pytest.mark.parametrize("precision", [64, 33])
+def test_threads_share_the_first_build(precision, monkeypatch):
+    """Several threads, a stream each, track a model that has no clusters yet."""
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    model, *rest = _case(precision)
+    want = _track(model, precision, *rest)
+    model, *rest = _case(precision)
+    torch.cuda.synchronize()
+    start, got, failed = threading.Barrier(4), [None] * 4, []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait(30)
+                got[i] = _track(model, precision, *rest)
+        except BaseException as e:  # noqa: BLE001 - shown below
+            failed.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not failed and list(model._far) == [precision]
+    for g in got:
+        assert np.array_equal(g, want)
+
+
+@pytest.mark.parametrize("precision", [64, 33])
+def test_a_graph_keeps_what_it_reads(precision, monkeypatch):
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    model, state, kq, dt, ns, npt = _case(precision)
+    want = _track(model, precision, state, kq, dt, ns, npt)
+    plan = model.plan(npt, 1)
+    st = state.clone()
+    graph = engine.TrackGraph(model, plan, precision, st, kq, dt, ns, STEPS, *model.workspace(plan))
+    alive, items = weakref.ref(model), weakref.ref(plan.far[precision].work)
+    del model, plan
+    gc.collect()
+    assert alive() is not None and items() is not None
+    for _ in range(2):
+        st.copy_(state)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(st.cpu().numpy(), want)
