@@ -22,6 +22,7 @@ import ctypes
 import hashlib
 import math
 import threading
+import warnings
 from dataclasses import dataclass, field as dc_field
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -56,7 +57,7 @@ _FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, any_large=(1
         33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, any_large=(30, 30), rate=(2.5e12, 1.75e12), saved=0.25,
                  setup=(0.40e-3, 0.66e-9), share=6)}
 _FAR_MAP_SAVED = (0.3, 0.7)  # of a map: single CCTs, of few clusters, and the section, a population's design, the gantry
-_FAR_MOST_ROWS = 1 << 28  # rows of the clusters (FP64 160 B each, and 145 B while they are built): 43 GB
+_FAR_MOST_ROWS = 1 << 28  # rows of the clusters (FP64 161 B each, and 140 B while they are built): 43 GB
 _FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters
 
 
@@ -296,6 +297,7 @@ class DeviceModel:
         self.bconst = torch.from_numpy(b).to(dev)
         self._plans: Dict[tuple, Plan] = {}
         self._far: Dict[int, FarField] = {}
+        self._far_no_room: set = set()  # precisions whose clusters did not fit
         self._stream = torch.cuda.current_stream()  # that of the tensors above
         self._far_lock = threading.Lock()
 
@@ -380,6 +382,8 @@ class DeviceModel:
         if torch.cuda.is_current_stream_capturing():
             return None  # a capture cannot build them
         with self._far_lock:
+            if precision in self._far_no_room:
+                return None
             far, items = self._far.get(precision), plan.far.get(key)
             # On the model's own stream: they live as long as its segments, whichever stream tracks first (memory goes
             # back to the stream that it was taken on, which knows nothing of the others' launches).
@@ -387,10 +391,15 @@ class DeviceModel:
                 try:
                     if far is None:
                         far = FarField(self, precision)
+                    if items is None:
+                        items = self._far_plan(far, plan, precision, max_steps == 0)
                 except torch.OutOfMemoryError:
-                    return None  # the clusters need as much again as the segments
-                if items is None:
-                    items = self._far_plan(far, plan, precision, max_steps == 0)
+                    # FP64 161 bytes per row of the clusters for good and 140 while they are built, FP32 38 and 46, beside
+                    # 64 (FP32 144) of the segments.  Not tried again: equal calls give equal bits.
+                    self._far_no_room.add(precision)
+                    warnings.warn("not enough GPU memory for the segment clusters: this model sums every segment",
+                                  RuntimeWarning, stacklevel=4)
+                    return None
                 self._stream.synchronize()  # ready for every stream that tracks this model
             self._far[precision], plan.far[key] = far, items
             return far, items
@@ -400,7 +409,7 @@ class DeviceModel:
         field, its set-up (once per model) included: a function of the sizes alone, so that equal
         calls give equal bits."""
         rule = _FAR.get(precision)
-        if rule is None or self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
+        if rule is None or precision in self._far_no_room or self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
             return False  # keys hold 15 bits of design; 16-point blocks of the FP32 path have no far-field kernel
         size = 0 if plan.ppl > 0 else 1
         large = rule["large"] if plan.pairs < rule["any_pairs"] else rule["any_large"][size]

@@ -91,6 +91,7 @@ def _pays(precision, ppl, segments, points, steps, designs=1):
 
     model = object.__new__(engine.DeviceModel)
     model.ndesign, model.nseg_padded = designs, designs * segments
+    model._far_no_room = set()
     model.cluster_rows = designs * -(-segments // 2048) * 2048
     pb = engine.points_per_block(ppl)
     plan = engine.Plan(ppl=ppl, nwork=0, work=None, wbase=None, nchunk=None, design_pt_off=None, npt=designs * points,

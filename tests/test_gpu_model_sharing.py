@@ -137,3 +137,30 @@ def test_a_graph_keeps_what_it_reads(precision, monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(st.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("precision", [64, 33])
+@pytest.mark.parametrize("where", ["FarField", "_far_plan"])
+def test_clusters_that_do_not_fit(where, precision, monkeypatch):
+    """The model says so once and sums every segment from then on, also when there is room again: equal calls give
+    equal bits."""
+    rule = engine.DeviceModel._far_pays
+    model, *rest = _case(precision)
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: False)
+    full = _track(model, precision, *rest)
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    tries = []
+
+    def no_room(*a, **k):
+        tries.append(1)
+        raise torch.OutOfMemoryError("no room")
+
+    with monkeypatch.context() as m:
+        m.setattr(engine if where == "FarField" else engine.DeviceModel, where, no_room)
+        with pytest.warns(RuntimeWarning, match="segment clusters"):
+            assert np.array_equal(_track(model, precision, *rest), full)
+        assert np.array_equal(_track(model, precision, *rest), full)
+    assert np.array_equal(_track(model, precision, *rest), full)
+    assert len(tries) == 1 and not model._far
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", rule)
+    assert not model._far_pays(model.plan(rest[-1], 1), precision, 10 ** 6)
