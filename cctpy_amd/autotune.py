@@ -1,9 +1,9 @@
-"""Tile-shape autotuner for the split-K Biot-Savart kernel.
+"""Tile-shape autotuner for tracking.
 
 Candidates are (points per lane, work items per CU).  Each is timed with HIP
-events over a few field evaluations (split-K Biot-Savart pass + fixed-order
-reduction, the per-stage cost of tracking) on the real segment set and
-points; the fastest wins.  Results are cached per (device, precision, design
+events over a few RK4 steps on the real segment set and points, with particles
+that stay where they are: the launches of a long track through them, with the
+sum that it takes (segment clusters or every segment); the fastest wins.  Results are cached per (device, precision, design
 sizes) in memory and in a JSON file (``$CCTAMD_TUNE_CACHE`` or
 ``~/.cache/cctamd/tune.json``).
 """
@@ -49,8 +49,9 @@ def _store(key: str, val: dict) -> None:
 
 # Bumped whenever the kernels or the candidate set change, so that cached choices of an
 # older library are not reused.
-KERNEL_SET = 11
+KERNEL_SET = 12
 TIE = 0.015
+LONG = 1_000_000  # steps of a track that pays for its set-up
 
 
 def _key(model: "engine.DeviceModel", npt: Sequence[int], precision: int) -> str:
@@ -72,8 +73,11 @@ def tune(model: "engine.DeviceModel", npt: Sequence[int], precision: int, points
     """Best {"ppl", "target_items"} for this model, point layout and precision.
 
     ``points`` is one device tensor (3, P) or a list of them (e.g. states sampled along a
-    track: the FP32 kernel's cost depends on how close points come to the windings); a
-    candidate's cost is its time summed over the point sets, best of ``rounds``."""
+    track: the cost depends on how close points come to the windings); a candidate's cost is
+    the time of an RK4 stage in the mean over the point sets, ``launches`` steps at each, best of
+    ``rounds``.  Field evaluations, which it timed before, are not what a track launches (no clusters on the
+    FP32 path, and the host's part of a call hid what small beams take: 64 protons in a single CCT got 2
+    points per lane, 23.1 ms a pass instead of 16.9)."""
     key = _key(model, npt, precision)
     if use_cache:
         if key in _MEM:
@@ -86,21 +90,27 @@ def tune(model: "engine.DeviceModel", npt: Sequence[int], precision: int, points
     cus = engine.cu_count()
     ppls = PPL + ((-2, -4) if precision != 32 else ())
     cost: Dict[tuple, float] = {}
+    still = torch.zeros_like(sets[0])  # velocities, and steps of no length
+    states = [torch.cat([pts, still]) for pts in sets]
+    steps = torch.full((sets[0].shape[1],), launches, dtype=torch.int64, device=sets[0].device)
+    seen: Dict[tuple, int] = {}
     for _ in range(max(1, rounds)):
         for ppl in ppls:
             for per_cu in ITEMS_PER_CU:
                 plan = model.plan(npt, ppl, per_cu * cus)
-                _, partial = model.workspace(plan)
-                out = torch.empty_like(sets[0])
-                model.field_tensors(plan, precision, sets[0], partial, out)
+                far = model.far_field(plan, precision, LONG)
+                if far is not None and seen.setdefault((ppl, far[1].nwork), per_cu) != per_cu:
+                    continue  # the launches of a candidate with fewer items
+                scratch, partial = model.workspace(plan)
                 e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                e0.record()
-                for pts in sets:
-                    for _ in range(launches):
-                        model.field_tensors(plan, precision, pts, partial, out)
+                for i, state in enumerate([states[0]] + states):
+                    if i == 1:
+                        e0.record()
+                    model._track(plan, precision, state, still[0], still[0], steps, launches, scratch, partial, None, 1,
+                                 of_steps=LONG)
                 e1.record()
                 torch.cuda.synchronize()
-                ms = e0.elapsed_time(e1) / (launches * len(sets))
+                ms = e0.elapsed_time(e1) / (4 * launches * len(sets))
                 k = (ppl, per_cu)
                 cost[k] = min(cost.get(k, ms), ms)
     (ppl, per_cu), ms = pick(cost)

@@ -445,8 +445,9 @@ class DeviceModel:
         return FarPlan(n, on[2 * D:-D], on[:2 * D].view(torch.int64), on[-D:])
 
     def _track(self, plan: Plan, precision: int, state, kq, dt, nsteps, max_steps: int, scratch, partial, record,
-               record_every: int, far_field: bool = True) -> None:
-        far = self.far_field(plan, precision, max_steps) if far_field and max_steps > 0 else None
+               record_every: int, far_field: bool = True, of_steps: int = 0) -> None:
+        """``of_steps``: the length of the track that these steps are the beginning of, for the choice of the sum."""
+        far = self.far_field(plan, precision, max(max_steps, of_steps)) if far_field and max_steps > 0 else None
         self._call(N.lib.cctamd_track_rk4 if far is None else N.lib.cctamd_track_rk4_far, "cctamd_track_rk4", plan,
                    precision, far, _p(state), plan.npt, _p(kq), _p(dt), _p(nsteps), int(max_steps), _p(scratch),
                    _p(partial), _p(record), int(record_every))
