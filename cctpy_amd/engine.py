@@ -452,6 +452,14 @@ class DeviceModel:
                    precision, far, _p(state), plan.npt, _p(kq), _p(dt), _p(nsteps), int(max_steps), _p(scratch),
                    _p(partial), _p(record), int(record_every))
 
+    def tracked_field_tensors(self, plan: "Plan", precision: int, points: torch.Tensor, partial: torch.Tensor,
+                              out: torch.Tensor, steps: int) -> None:
+        """B (3, P) at device points (3, P) as the RK4 stages of a track of ``steps`` steps sum it: by the same
+        launches, clusters included (``field_tensors`` chooses for one evaluation)."""
+        far = self.far_field(plan, precision, steps) if steps > 0 else None
+        self._call(N.lib.cctamd_bs_field if far is None else N.lib.cctamd_bs_field_far, "cctamd_bs_field", plan,
+                   precision, far, _p(points), plan.npt, _p(partial), _p(out))
+
     def _map_far(self, plan: Plan, points: torch.Tensor) -> tuple:
         """Arguments of cctamd_bs_field_routed before those of cctamd_bs_field; () where every segment is
         summed.  Points in no order (a shuffled map, a raster across the magnet) have blocks that are close to
