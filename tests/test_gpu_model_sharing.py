@@ -164,3 +164,39 @@ def test_clusters_that_do_not_fit(where, precision, monkeypatch):
     assert len(tries) == 1 and not model._far
     monkeypatch.setattr(engine.DeviceModel, "_far_pays", rule)
     assert not model._far_pays(model.plan(rest[-1], 1), precision, 10 ** 6)
+
+
+@pytest.mark.parametrize("precision", [64, 33])
+def test_a_capture_builds_no_clusters(precision, monkeypatch):
+    """Captured before anything was tracked, a track sums every segment (the eager call of a model without them); with the
+    clusters there, it takes them."""
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: False)
+    model, state, kq, dt, ns, npt = _case(precision)
+    full = _track(model, precision, state, kq, dt, ns, npt)
+    monkeypatch.setattr(engine.DeviceModel, "_far_pays", lambda *a: True)
+    plan = model.plan(npt, 1)
+    scratch, partial = model.workspace(plan)
+    st = state.clone()
+
+    def captured():
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            model.track_tensors(plan, precision, st, kq, dt, ns, STEPS, scratch, partial)
+        return graph
+
+    def replayed(graph):
+        st.copy_(state)
+        graph.replay()
+        torch.cuda.synchronize()
+        return st.cpu().numpy()
+
+    before = captured()
+    assert not model._far and np.array_equal(replayed(before), full)
+    far = _track(model, precision, state, kq, dt, ns, npt)
+    assert not np.array_equal(far, full)
+    after = captured()
+    for _ in range(3):
+        assert np.array_equal(replayed(after), far)
+        assert np.array_equal(replayed(before), full)
+        assert np.array_equal(_track(model, precision, state, kq, dt, ns, npt), far)
