@@ -688,6 +688,8 @@ int cctamd_far_build(int precision, const double* seg64, int unit, const float* 
     const int q = precision == 64 ? kFarQ64 : kFarQ32;
     const int ntile = kSmallTiles;
     const int64_t places = ncluster * ntile, nrec = 2 * ncluster * far_records(q);
+    // k_bs_partial_f64 counts the packed rows in 31 bits
+    if (precision == 64 && places * kTile > 0x7fffffff) return CCTAMD_ERANGE;
     if (places > 0x7fffffff || ceil_div(places * kTile * 2, 256) > 0x7fffffff || ceil_div(nrec, 256) > 0x7fffffff ||
         nchunk > 0x7fffffff)
         return CCTAMD_ERANGE;

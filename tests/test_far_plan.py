@@ -137,3 +137,15 @@ def test_the_clusters_of_a_model_are_bounded():
 def test_maps_pay_for_their_clusters_in_one_call():
     assert _pays(64, 2, 368640, 5003, 0) and not _pays(64, 2, 368640, 2000, 0)
     assert not _pays(64, 2, 46080, 20000, 0)  # a single CCT: few clusters, 0.3 of the time saved
+
+
+def test_rows_past_31_bits_are_refused():
+    """Before any launch: the FP64 kernels count packed rows in 31 bits, 512 per cluster.  The FP32 path counts tiles."""
+    some = ctypes.c_void_p(64)
+
+    def build(precision, clusters):
+        return N.lib.cctamd_far_build(precision, some, 32 if precision == 33 else 8, some, some, some, 1, some, 1, clusters,
+                                      some, some, some, some, some, some, some, some, None)
+
+    assert build(64, 1 << 22) == -34
+    assert build(64, 1 << 27) == build(33, 1 << 27) == -34
