@@ -5,15 +5,16 @@ A *step* is one full tracking pass of the whole synthetic beam through the
 workload's beamline (all RK4 steps; default workload ``agcct_section``:
 368,640 winding segments + 2 quads, 512 protons, 2,510 RK4 steps of 1 mm).
 The timed passes use the FP32 Biot-Savart tracking path (per-tile
-re-centred FP32 terms summed as K x q - C per tile, FP64 accumulation across
-tiles, FP64 particle state); one pass of the plain FP64 path is timed beside
-it and is the reference for the final-position error.
+re-centred FP32 terms summed as K x q - C per tile, FP64 series for distant
+clusters of segments, FP64 accumulation across tiles, FP64 particle state); one
+pass of the FP64 path is timed beside it and is the reference for the
+final-position error, and one of the plain FP64 sum over every segment.
 Inputs are resident in HBM before timing starts; every pass restarts from the
 same initial state with a device-to-device copy.
 
 Besides the main line, ``extras`` (skip with ``--no-extras``) reports
   * the batched design population (64 designs of uneven segment counts, 32
-    protons each): FP32 forward, plain FP64 forward, and FP32 forward+adjoint
+    protons each): FP32 forward, FP64 forward, and FP32 forward+adjoint
     (beam-spot objective per design, checkpoints every 50 steps);
   * the differentiation workload (AG-CCT section + 1.1 m drift, 256 protons):
     FP32 forward+adjoint.
@@ -271,7 +272,7 @@ class Setup:
 
 def tracking_leg(name: str, max_steps: int = 0, passes: int = 3, ppl: int = 0, items_per_cu: int = 0,
                  adjoint_steps: int = 0) -> dict:
-    """FP32 and plain FP64 tracking passes of one workload (HIP-graph replay, inputs resident),
+    """FP32 and FP64 tracking passes of one workload (HIP-graph replay, inputs resident),
     their final-position difference, and optionally FP32 forward + adjoint over a step prefix.
     ppl = 0 lets the autotuner pick the block shape (it tracks a sample pass first)."""
     import numpy as np
@@ -473,23 +474,33 @@ def main() -> int:
     rate32 = S.particle_steps / (ms32 / 1e3)
     log(f"[bench] fp32: {ms32:.1f} ms/pass, {rate32:.4g} particle-steps/s")
 
-    fp64 = None
+    fp64 = plain = None
     err = None
     if not args.no_fp64:
         tuned[64] = S.shape(64, args.ppl, args.items_per_cu)
-        ms64, out64, _, _ = S.forward(64, tuned[64], 1, 1 if args.warmup > 0 else 0, args.graph)
+        ms64, out64, plan64t, _ = S.forward(64, tuned[64], 1, 1 if args.warmup > 0 else 0, args.graph)
         rate64 = S.particle_steps / (ms64 / 1e3)
         d = np.linalg.norm(out32[:, :3] - out64[:, :3], axis=1)
         err = {"max": float(d.max() * 1e6), "rms": float(np.sqrt(np.mean(d ** 2)) * 1e6),
                "p99": float(np.percentile(d, 99) * 1e6), "median": float(np.median(d) * 1e6),
                "within_1um": float(np.mean(d <= 1e-6))}
         fp64 = {"particle_steps_per_s": rate64, "pair_evals_per_s": S.pairs_per_pass / (ms64 / 1e3),
-                "ms_per_step": ms64, "ppl": tuned[64]["ppl"]}
+                "ms_per_step": ms64, "ppl": tuned[64]["ppl"],
+                "clusters": model.far_field(plan64t, 64, S.max_steps) is not None}
+        # the plain sum of every segment in FP64
+        plan = model.plan(S.npt, engine.block_shape_for(S.npt, 64))
+        scratch, partial = model.workspace(plan)
+        ms_plain = S.timed(lambda: model._track(plan, 64, S.st, S.kq, S.dt, S.ns_t, S.max_steps, scratch, partial, None, 1,
+                                                far_field=False), 1, 0)
+        plain = {"particle_steps_per_s": S.particle_steps / (ms_plain / 1e3),
+                 "pair_evals_per_s": S.pairs_per_pass / (ms_plain / 1e3), "ms_per_step": ms_plain, "ppl": plan.ppl}
         log(f"[bench] fp64: {ms64:.1f} ms/pass, {rate64:.4g} particle-steps/s; fp32 position error "
             f"max {err['max']:.3g} um, rms {err['rms']:.3g} um")
 
-    # live timing of the dominant kernel (split-K Biot-Savart, FP32) on the stream it runs on, at
-    # states recorded along the FP32 track (its cost depends on how close particles get to windings)
+    # live timing of the FP32 Biot-Savart kernel that sums every segment (fields, the adjoint, small tracks), on the
+    # stream it runs on, at states recorded along the FP32 track (its cost depends on how close particles get to
+    # windings), with the planner's default items; and of the evaluations that tracking launches, which let distant
+    # clusters of segments act through series where that is faster (pairs they stand for have no roofline)
     every = max(1, S.max_steps // 10)
     rec = torch.empty((S.max_steps // every + 1, 6, S.P), dtype=torch.float64, device=engine.device())
     S.st.copy_(S.s0)
@@ -497,22 +508,28 @@ def main() -> int:
     model.track_tensors(plan32, FP32, S.st, S.kq, S.dt, S.ns_t, S.max_steps, scratch32, partial32, record=rec,
                         record_every=every)
     per = max(5, args.roofline_launches // rec.shape[0])
-    avg_ms = float(np.mean([bs_launch_timing(plan32, rec[i, :3].contiguous(), partial32, per)
+    plan_full = model.plan(S.npt, plan32.ppl)
+    _, partial_full = model.workspace(plan_full)
+    avg_ms = float(np.mean([bs_launch_timing(plan_full, rec[i, :3].contiguous(), partial_full, per)
                             for i in range(rec.shape[0])]))
+    far = model.far_field(plan32, FP32, S.max_steps)
     flops = float(np.sum(np.asarray(S.npt) * model.design_nseg)) * FLOP_PER_PAIR
     achieved = flops / (avg_ms / 1e3) / 1e12
     kname = kernel_name(plan32.ppl)
     roofline = {"bound": "valu", "achieved": achieved, "peak": PEAK_TFLOPS[32], "unit": "TFLOP/s",
-                "frac": achieved / PEAK_TFLOPS[32], "traffic": measured_traffic(wl.name, kname, plan32.nwork),
+                "frac": achieved / PEAK_TFLOPS[32], "traffic": measured_traffic(wl.name, kname, plan_full.nwork),
                 "kernel": kname, "avg_launch_ms": avg_ms, "flop_per_launch": flops,
                 "algorithmic_bytes_per_launch": float(model.nseg_padded * 48 + plan32.npt * 24
-                                                      + plan32.nwork * 3 * engine.points_per_block(plan32.ppl) * 8)}
+                                                      + plan_full.nwork * 3 * engine.points_per_block(plan32.ppl) * 8),
+                "work_items": plan_full.nwork,
+                "launched_by_tracking": far is None,
+                "tracking_stage_ms": ms32 / (4 * S.max_steps)}
     if roofline["traffic"] is not None:  # HBM bytes per launch (counters) at this launch duration
         roofline["traffic_GB_per_s"] = roofline["traffic"] / (avg_ms / 1e3) / 1e9
     log(f"[bench] bs kernel: {avg_ms * 1e3:.1f} us/launch, {achieved:.2f} TFLOP/s "
         f"({100 * roofline['frac']:.1f}% of FP32 vector peak)")
 
-    # field of the FP32 path against FP64 at the same recorded states (relative error over points
+    # field of the FP32 path, by the sum that tracking launches, against FP64 at the same recorded states (relative error over points
     # whose field is at least 1 % of the largest, where a relative figure means something)
     plan64 = model.plan(S.npt, 2)
     _, partial64 = model.workspace(plan64)
@@ -520,7 +537,7 @@ def main() -> int:
     dns, bns = [], []
     for i in range(rec.shape[0]):
         pts = rec[i, :3].contiguous()
-        model.field_tensors(plan32, FP32, pts, partial32, b32)
+        model.tracked_field_tensors(plan32, FP32, pts, partial32, b32, S.max_steps)
         model.field_tensors(plan64, 64, pts, partial64, b64)
         dns.append((b32 - b64).norm(dim=0))
         bns.append(b64.norm(dim=0))
@@ -593,16 +610,20 @@ def main() -> int:
         "vs_baseline": None,
         "dtype": "f32",
         "dtype_detail": "f32 Biot-Savart pair terms and 32-segment tile sums; f64 terms for tiles a point lies "
-                        "among, f64 tile origins, sums across tiles and RK4 state",
+                        "among, f64 multipole series for distant clusters of segments, f64 tile origins, sums across "
+                        "tiles and RK4 state",
         "data": "synthetic",
         "config": {"workload": wl.name, "designs": len(S.bls), "segments": int(model.nseg), "protons": S.P,
                    "rk4_steps": S.max_steps, "steps_capped": args.max_steps > 0,
                    "footstep_mm": wl.footstep * 1e3, "length_m": wl.length,
-                   "parallelism": "single GPU", "ppl": plan32.ppl, "work_items": plan32.nwork, "hip_graph": args.graph,
+                   "parallelism": "single GPU", "ppl": plan32.ppl, "work_items": (far[1] if far else plan32).nwork,
+                   "clusters": far is not None, "hip_graph": args.graph,
                    "target_items": tuned[FP32]["target_items"]},
-        "pair_evals_per_s": S.pairs_per_pass / (ms32 / 1e3),
-        "fp64_plain": fp64,
+        "pair_evals_per_s": S.pairs_per_pass / (ms32 / 1e3),  # pairs that the results stand for, series included
+        "fp64": fp64,
+        "fp64_plain": plain,
         "speedup_vs_fp64": (rate32 / fp64["particle_steps_per_s"]) if fp64 else None,
+        "speedup_vs_fp64_plain": (rate32 / plain["particle_steps_per_s"]) if plain else None,
         "position_error_um_vs_fp64": err,
         "field_error_vs_fp64": field_err,
         "roofline": roofline,
