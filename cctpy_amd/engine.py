@@ -460,28 +460,24 @@ class DeviceModel:
         self._call(N.lib.cctamd_bs_field if far is None else N.lib.cctamd_bs_field_far, "cctamd_bs_field", plan,
                    precision, far, _p(points), plan.npt, _p(partial), _p(out))
 
-    def _map_far(self, plan: Plan, points: torch.Tensor) -> tuple:
-        """Arguments of cctamd_bs_field_routed before those of cctamd_bs_field; () where every segment is
-        summed.  Points in no order (a shuffled map, a raster across the magnet) have blocks that are close to
+    def _map_far(self, plan: Plan, points: torch.Tensor) -> Optional[Tuple[torch.Tensor, FarField, FarPlan]]:
+        """What the device found of the points (cctamd_point_spread) and the clusters with their work items for
+        cctamd_bs_field_routed; None where every segment is summed.  Points in no order (a shuffled map, a raster across the magnet) have blocks that are close to
         every cluster: they are summed segment by segment, which the device finds out for every call, so
         that equal calls give equal bits; the host asks before it builds clusters (one wait, with the
         build's)."""
         built = 64 in self._far
         if not self._far_pays(plan, 64, 0) or (not built and torch.cuda.is_current_stream_capturing()):
-            return ()
+            return None
         spread = torch.empty(2, dtype=torch.int64, device=points.device)
         N.check(N.lib.cctamd_point_spread(plan.ppl, _p(self.seg64), _p(plan.work), plan.nwork, _p(points), plan.npt,
                                           _p(spread), _stream()), "cctamd_point_spread")
         if not built:
             near, every = spread.tolist()
             if 3 * near > 2 * every:  # spread_out in csrc/common.hpp
-                return ()
+                return None
         far_field = self.far_field(plan, 64, 0)
-        if far_field is None:
-            return ()
-        far, w = far_field
-        return (_p(spread), _p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.rows), _p(w.work),
-                w.nwork, _p(w.wbase), _p(w.nchunk))
+        return None if far_field is None else (spread, *far_field)
 
     def _call(self, function, name: str, plan: Plan, precision: int, far_field: Optional[Tuple[FarField, FarPlan]],
               *args, head: tuple = ()) -> None:
@@ -577,8 +573,13 @@ class DeviceModel:
                       out: torch.Tensor) -> None:
         """B (3, P) at device points (3, P): Biot-Savart pass + fixed-order reduction + QS + uniform."""
         # a map pays for its clusters in one call; on the FP32 path a field keeps the terms of every segment
-        head = self._map_far(plan, points) if precision == 64 and plan.pairs > _FAR_MAP_PAIRS else ()
-        self._call(N.lib.cctamd_bs_field_routed if head else N.lib.cctamd_bs_field, "cctamd_bs_field", plan,
+        routed = self._map_far(plan, points) if precision == 64 and plan.pairs > _FAR_MAP_PAIRS else None
+        head: tuple = ()
+        if routed is not None:
+            spread, far, w = routed
+            head = (_p(spread), _p(far.geo), _p(far.geo_large), _p(far.coef), _p(far.coef_large), _p(far.rows),
+                    _p(w.work), w.nwork, _p(w.wbase), _p(w.nchunk))
+        self._call(N.lib.cctamd_bs_field if routed is None else N.lib.cctamd_bs_field_routed, "cctamd_bs_field", plan,
                    precision, None, _p(points), plan.npt, _p(partial), _p(out), head=head)
 
     def bs_partial_tensors(self, plan: "Plan", precision: int, points: torch.Tensor, partial: torch.Tensor) -> None:

@@ -3,6 +3,8 @@
 An FP64 map of many points lets far clusters act through series (within 1e-13 of the sum of every segment: up to 10^5
 terms in another order), unless its blocks reach across the magnet, where every segment is summed (the same bits).
 What a call gives depends on its points alone, not on the calls before it."""
+import weakref
+
 import numpy as np
 import pytest
 import torch
@@ -123,3 +125,28 @@ def test_a_captured_map_follows_its_points():
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), want[rep % 2]), rep
         assert np.array_equal(_field(model, sets[rep % 2], 2), want[rep % 2]), rep
+
+
+def test_what_the_device_found_outlives_the_launches(monkeypatch):
+    """The call holds the counts of the points until its kernels are on the stream: their memory cannot go to another
+    thread's tensors before."""
+    bls = _beamlines()
+    model, pts = _model(bls), _points(bls, "ordered")
+    want = _field(model, pts, 2)
+    found, alive = [], []
+    empty, call = torch.empty, model._call
+
+    def noted(*a, **k):
+        t = empty(*a, **k)
+        if k.get("dtype") == torch.int64:
+            found.append(weakref.ref(t))
+        return t
+
+    def launched(*a, **k):
+        alive.append(found[-1]() is not None)
+        call(*a, **k)
+
+    monkeypatch.setattr(torch, "empty", noted)
+    monkeypatch.setattr(model, "_call", launched)
+    assert np.array_equal(_field(model, pts, 2), want)
+    assert alive == [True] and found[-1]() is None
