@@ -469,15 +469,22 @@ class DeviceModel:
         built = 64 in self._far
         if not self._far_pays(plan, 64, 0) or (not built and torch.cuda.is_current_stream_capturing()):
             return None
+        spread = self._point_spread(plan, points)
+        if not built and self._spread_out(spread):
+            return None
+        far_field = self.far_field(plan, 64, 0)
+        return None if far_field is None else (spread, *far_field)
+
+    def _point_spread(self, plan: Plan, points: torch.Tensor) -> torch.Tensor:
         spread = torch.empty(2, dtype=torch.int64, device=points.device)
         N.check(N.lib.cctamd_point_spread(plan.ppl, _p(self.seg64), _p(plan.work), plan.nwork, _p(points), plan.npt,
                                           _p(spread), _stream()), "cctamd_point_spread")
-        if not built:
-            near, every = spread.tolist()
-            if 3 * near > 2 * every:  # spread_out in csrc/common.hpp
-                return None
-        far_field = self.far_field(plan, 64, 0)
-        return None if far_field is None else (spread, *far_field)
+        return spread
+
+    @staticmethod
+    def _spread_out(spread: torch.Tensor) -> bool:
+        near, every = spread.tolist()
+        return 3 * near > 2 * every  # spread_out in csrc/common.hpp
 
     def _call(self, function, name: str, plan: Plan, precision: int, far_field: Optional[Tuple[FarField, FarPlan]],
               *args, head: tuple = ()) -> None:
@@ -552,7 +559,9 @@ class DeviceModel:
         scratch = torch.empty((15, plan.npt), dtype=torch.float64, device=dev)
         partial = torch.empty(max(plan.nwork * 3 * points_per_block(ppl), 1), dtype=torch.float64, device=dev)
         rec = torch.empty((max_steps + 1, 6, plan.npt), dtype=torch.float64, device=dev) if record else None
-        self._track(plan, precision, soa, kq_t, dt_t, ns_t, max_steps, scratch, partial, rec, 1)
+        # particles all along the orbit have no use for the clusters; this call waits for the device anyway
+        far = self._far_pays(plan, precision, max_steps) and not self._spread_out(self._point_spread(plan, soa))
+        self._track(plan, precision, soa, kq_t, dt_t, ns_t, max_steps, scratch, partial, rec, 1, far_field=far)
         out = soa.cpu().numpy().T.copy()
         return out, (rec.cpu().numpy().transpose(0, 2, 1).copy() if rec is not None else None)
 

@@ -150,3 +150,34 @@ def test_what_the_device_found_outlives_the_launches(monkeypatch):
     monkeypatch.setattr(model, "_call", launched)
     assert np.array_equal(_field(model, pts, 2), want)
     assert alive == [True] and found[-1]() is None
+
+
+@pytest.mark.parametrize("precision,ppl", [(64, 1), (64, -2), (33, 1), (33, -2)])
+def test_host_particles_all_along_the_orbit_sum_every_segment(precision, ppl):
+    """A bunch takes the clusters, particles at all places of the orbit do not (and nothing is built for them)."""
+    bls = _beamlines()[:2]
+    model = engine.DeviceModel([device_parts(bl).spec() for bl in bls], fp32=precision != 64)
+    rng = np.random.default_rng(6)
+    n = 60
+    bunch, along = [], []
+    for bl in bls:
+        for rows, places in ((bunch, rng.normal(0.3, 2e-3, n)), (along, rng.uniform(0.05, 0.95, n) * bl.get_length())):
+            for s in places:
+                p, d = bl.trajectory.point_at(float(s)), bl.trajectory.direct_at(float(s))
+                rows.append([p.x, p.y, 0.0, 1.8e8 * d.x, 1.8e8 * d.y, 0.0])
+    args = (np.full(2 * n, 7.0e7), np.full(2 * n, 1e-3 / 1.8e8), np.full(2 * n, 3), [n, n])
+
+    def full(state):
+        plan = model.plan([n, n], ppl)
+        scratch, partial = model.workspace(plan)
+        st, kq, dt, ns = (torch.from_numpy(np.ascontiguousarray(a)).to(engine.device())
+                          for a in (np.array(state).T, *args[:3]))
+        model._track(plan, precision, st, kq, dt, ns, 3, scratch, partial, None, 1, far_field=False)
+        return st.cpu().numpy().T
+
+    assert np.array_equal(model.track(np.array(along), *args, precision=precision, ppl=ppl)[0], full(along))
+    assert not model._far
+    got, want = model.track(np.array(bunch), *args, precision=precision, ppl=ppl)[0], full(bunch)
+    assert precision in model._far and not np.array_equal(got, want)
+    np.testing.assert_allclose(got, want, rtol=1e-6 if precision == 33 else 1e-12, atol=1e-9)
+    assert np.array_equal(model.track(np.array(along), *args, precision=precision, ppl=ppl)[0], full(along))
