@@ -428,8 +428,8 @@ __global__ __launch_bounds__(kFarWG) void k_far_balls(const double* __restrict__
 // the sum of its parts' about its own centre (k_far_coef adds them).  A wave takes one m at a
 // time, eight rows per lane whose recurrences stay in registers, kFarChunk orders per round;
 // the lanes' sums are added in a fixed order through LDS.  10 FP64 instructions per row and
-// order: 0.37 ms for the AG-CCT section's 368,640 rows on the FP64 path, 0.17 ms on the FP32
-// path (both sizes of cluster), at 2 waves per SIMD and half of the issue slots.  Held to 168
+// order: 0.45 ms for the AG-CCT section's 368,640 rows on the FP64 path (orders up to 34 of the
+// potential), 0.16 ms on the FP32 path (both sizes of cluster), at 2 waves per SIMD and half of the issue slots.  Held to 168
 // VGPRs for a third wave it spills and takes 4 times as long; adding the wave's halves in
 // registers before LDS gained nothing.
 constexpr int kFarChunk = 4;

@@ -449,7 +449,7 @@ __device__ __forceinline__ void far_rows(ConstDoubles geo, const double* __restr
 // starts few series (those of its stretch).  Dealt out by series, or by eighths of one where there
 // were few, waves had two or three pieces of very different lengths, and each piece began with
 // powers of X + iY: 4,096 protons in the gantry spent 37 us of a stage here, now 18; a stage of 512
-// in the AG-CCT section (FP64) took 49.8 us, now 44.5.
+// in the AG-CCT section (FP64, orders up to 31) took 49.8 us, now 44.5.
 template <int Q, int LR, int NW, int PL>
 __device__ __forceinline__ void far_share(const FarLists<NW>& L, const FarCounts& n, const FarSet& fs, int me, int all, int lane,
                                           const double (&px)[PL], const double (&py)[PL], const double (&pz)[PL],

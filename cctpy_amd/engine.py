@@ -48,8 +48,8 @@ _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # the gantry at 120 (2.0e7, 78) 24.5 / 18.2 and 38.2 / 31.6; 32-point blocks: 32 in the gantry at 360 (1.5e7, 234) 19.5 / 20.0
 # and 24.9 / 29.8, at 720 (3.1e7, 468) 27.1 / 25.7 and 31.2 / 42.7, four designs x 32 (4.4e7, 166) 33.9 / 28.2 and
 # 35.7 / 41.0; 4,096 in the gantry at 720 (3.9e9) 1,500 / 221 and 1,500 / 1,790; single CCTs stay with the full
-# sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3, and nearer to the bound of what the far field may move a
-# track by).  Many designs of few clusters, FP64: 2,000 of 200 segments x 64 198 / 242 and 44 ms of set-up, 200 of 3,000
+# sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3: their clusters are few and close, and series in the place
+# of FP32 terms so near move a track by the FP32 sum's own error).  Many designs of few clusters, FP64: 2,000 of 200 segments x 64 198 / 242 and 44 ms of set-up, 200 of 3,000
 # x 64 63 / 87, 64 of 8,000 x 64 46 / 49, 24 of 16,000 x 64 36 / 38, 24 of 23,040 x 100 86 / 65, 8 of 30,000 x 100 40 / 31; 100 of
 # 23,040 x 32 91 / 105.  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640, 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
 _FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, any_large=(10, 36), rate=(1.25e12, 0.9e12),
