@@ -36,27 +36,30 @@ _MIN_TILES_PER_ITEM = 4
 _LARGE_TILES = 64   # tiles of a large segment cluster (kParts * kSmallTiles in csrc/far.hpp)
 _FAR_CHUNK = 16384  # units that are split together (kChunk in csrc/far.hip)
 # Where tracking takes the far field (64-point blocks and larger, smaller blocks): lanes x segments of a launch and
-# large clusters per design from which it does, or fewer clusters but more lanes x segments (any_*); the
-# pair terms per second of the full sum (the same two block sizes) and the share of their time that a bunch saves at the
-# least; the set-up in s and s per segment; and the work items per cluster and block of a single design.
+# large clusters per design from which it does, or fewer clusters but more lanes x segments (any_*); the pair terms
+# per second of the full sum (the same two block sizes) and the share of their time that a bunch saves at the least;
+# the set-up in s and s per segment; and the work items per cluster and block of a single design.
 # Measured per RK4 stage in us, full sum / far field, for a bunch and for particles all along the orbit.  FP64: one
-# in the gantry at 60 segments per winding (1.3e6 pairs, 39 clusters) 12.9 / 12.1 and 13.0 / 11.9, 64 in the AG-CCT section at
-# 60 (2.0e6, 15) 11.5 / 13.7, 32 at 120 (2.0e6, 30) 13.6 / 15.6, 16 at 360 (2.9e6, 90) 17.2 / 15.5 and 17.6 / 15.7, 32 in the
-# gantry at 120 (5.1e6, 78) 17.0 / 13.4 and 17.6 / 18.2, 200 in one CCT of 720 tiles (5.9e6, 11) 16.2 / 16.7, 300 (8.8e6)
-# 20.4 / 18.4, 64 in the gantry at 720 (6.1e7, 468) 68 / 19 and 72 / 89, 512 in the section at 720 (1.9e8, 180) 152 / 52
-# and 155 / 157.  FP32: 64 in the section at 360 (1.2e7, 90) 16.6 / 16.8, at 720 (2.4e7, 180) 23.4 / 18.2 and 23.6 / 29.8, 128 in
-# the gantry at 120 (2.0e7, 78) 24.5 / 18.2 and 38.2 / 31.6; 32-point blocks: 32 in the gantry at 360 (1.5e7, 234) 19.5 / 20.0
-# and 24.9 / 29.8, at 720 (3.1e7, 468) 27.1 / 25.7 and 31.2 / 42.7, four designs x 32 (4.4e7, 166) 33.9 / 28.2 and
-# 35.7 / 41.0; 4,096 in the gantry at 720 (3.9e9) 1,500 / 221 and 1,500 / 1,790; single CCTs stay with the full
-# sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7 / 17.3: their clusters are few and close, and series in the place
-# of FP32 terms so near move a track by the FP32 sum's own error).  Many designs of few clusters, FP64: 2,000 of 200 segments x 64 198 / 242 and 44 ms of set-up, 200 of 3,000
-# x 64 63 / 87, 64 of 8,000 x 64 46 / 49, 24 of 16,000 x 64 36 / 38, 24 of 23,040 x 100 86 / 65, 8 of 30,000 x 100 40 / 31; 100 of
-# 23,040 x 32 91 / 105.  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640, 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
+# in the gantry at 60 segments per winding (1.3e6 pairs, 39 clusters) 12.9 / 12.1 and 13.0 / 11.9, 64 in the AG-CCT
+# section at 60 (2.0e6, 15) 11.5 / 13.7, 32 at 120 (2.0e6, 30) 13.6 / 15.6, 16 at 360 (2.9e6, 90) 17.2 / 15.5 and
+# 17.6 / 15.7, 32 in the gantry at 120 (5.1e6, 78) 17.0 / 13.4 and 17.6 / 18.2, 200 in one CCT of 720 tiles (5.9e6,
+# 11) 16.2 / 16.7, 300 (8.8e6) 20.4 / 18.4, 64 in the gantry at 720 (6.1e7, 468) 68 / 19 and 72 / 89, 512 in the
+# section at 720 (1.9e8, 180) 152 / 52 and 155 / 157.  FP32: 64 in the section at 360 (1.2e7, 90) 16.6 / 16.8, at
+# 720 (2.4e7, 180) 23.4 / 18.2 and 23.6 / 29.8, 128 in the gantry at 120 (2.0e7, 78) 24.5 / 18.2 and 38.2 / 31.6;
+# 32-point blocks: 32 in the gantry at 360 (1.5e7, 234) 19.5 / 20.0 and 24.9 / 29.8, at 720 (3.1e7, 468) 27.1 / 25.7
+# and 31.2 / 42.7, four designs x 32 (4.4e7, 166) 33.9 / 28.2 and 35.7 / 41.0; 4,096 in the gantry at 720 (3.9e9)
+# 1,500 / 221 and 1,500 / 1,790; single CCTs stay with the full sum there (300 protons, 1,440 tiles: 1.8e7, 22, 19.7
+# / 17.3: their clusters are few and close, and series in the place of FP32 terms so near move a track by the FP32
+# sum's own error).  Many designs of few clusters, FP64: 2,000 of 200 segments x 64 198 / 242 and 44 ms of set-up,
+# 200 of 3,000 x 64 63 / 87, 64 of 8,000 x 64 46 / 49, 24 of 16,000 x 64 36 / 38, 24 of 23,040 x 100 86 / 65, 8 of
+# 30,000 x 100 40 / 31; 100 of 23,040 x 32 91 / 105.  Set-up: FP64 0.51 ms for 23,040 segments, 0.96 for 368,640,
+# 1.90 for 959,040; FP32 0.37, 0.64, 0.98.
 _FAR = {64: dict(pairs=(1.25e6, 1.25e6), large=36, any_pairs=8.5e6, any_large=(10, 36), rate=(1.25e12, 0.9e12),
                  saved=0.6, setup=(0.47e-3, 1.45e-9), share=24),
-        33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, any_large=(30, 30), rate=(2.5e12, 1.75e12), saved=0.25,
-                 setup=(0.40e-3, 0.66e-9), share=6)}
-_FAR_MAP_SAVED = (0.3, 0.7)  # of a map: single CCTs, of few clusters, and the section, a population's design, the gantry
+        33: dict(pairs=(2.0e7, 4.0e7), large=30, any_pairs=math.inf, any_large=(30, 30), rate=(2.5e12, 1.75e12),
+                 saved=0.25, setup=(0.40e-3, 0.66e-9), share=6)}
+# of a map's time: single CCTs, of few clusters; the section, a population's design and the gantry
+_FAR_MAP_SAVED = (0.3, 0.7)
 _FAR_MOST_ROWS = 1 << 28  # rows of the clusters (FP64 161 B each, and 140 B while they are built): 43 GB
 _FAR_MAP_PAIRS = 5.0e8  # no single evaluation below pays for its clusters
 
@@ -173,7 +176,8 @@ def far_items(clusters: int, alike: bool, single: bool, precision: int, ppl: int
     if alike:
         return min(cus if clusters <= _FAR[precision]["share"] * cus else 2 * cus, most)
     each = 2 * cus if ppl > 0 else cus
-    whole = int(min(max(clusters // 5, 2 * cus), 6 * cus, most) / each + 0.3) * each  # 0.3: a round that is nearly full
+    # 0.3: a round that is nearly full
+    whole = int(min(max(clusters // 5, 2 * cus), 6 * cus, most) / each + 0.3) * each
     return whole if 0 < whole <= most else most
 
 
@@ -394,8 +398,8 @@ class DeviceModel:
                     if items is None:
                         items = self._far_plan(far, plan, precision, max_steps == 0)
                 except torch.OutOfMemoryError:
-                    # FP64 161 bytes per row of the clusters for good and 140 while they are built, FP32 38 and 46, beside
-                    # 64 (FP32 144) of the segments.  Not tried again: equal calls give equal bits.
+                    # FP64 161 bytes per row of the clusters for good and 140 while they are built, FP32 38 and 46,
+                    # beside 64 (FP32 144) of the segments.  Not tried again: equal calls give equal bits.
                     self._far_no_room.add(precision)
                     warnings.warn("not enough GPU memory for the segment clusters: this model sums every segment",
                                   RuntimeWarning, stacklevel=4)
@@ -409,7 +413,9 @@ class DeviceModel:
         field, its set-up (once per model) included: a function of the sizes alone, so that equal
         calls give equal bits."""
         rule = _FAR.get(precision)
-        if rule is None or precision in self._far_no_room or self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
+        if rule is None or precision in self._far_no_room:
+            return False
+        if self.ndesign > 0x7fff or (precision == 33 and plan.ppl == -4):
             return False  # keys hold 15 bits of design; 16-point blocks of the FP32 path have no far-field kernel
         size = 0 if plan.ppl > 0 else 1
         large = rule["large"] if plan.pairs < rule["any_pairs"] else rule["any_large"][size]
@@ -462,10 +468,10 @@ class DeviceModel:
 
     def _map_far(self, plan: Plan, points: torch.Tensor) -> Optional[Tuple[torch.Tensor, FarField, FarPlan]]:
         """What the device found of the points (cctamd_point_spread) and the clusters with their work items for
-        cctamd_bs_field_routed; None where every segment is summed.  Points in no order (a shuffled map, a raster across the magnet) have blocks that are close to
-        every cluster: they are summed segment by segment, which the device finds out for every call, so
-        that equal calls give equal bits; the host asks before it builds clusters (one wait, with the
-        build's)."""
+        cctamd_bs_field_routed; None where every segment is summed.  Points in no order (a shuffled map, a raster
+        across the magnet) have blocks that are close to every cluster: they are summed segment by segment, which
+        the device finds out for every call, so that equal calls give equal bits; the host asks before it builds
+        clusters (one wait, with the build's)."""
         built = 64 in self._far
         if not self._far_pays(plan, 64, 0) or (not built and torch.cuda.is_current_stream_capturing()):
             return None
